@@ -94,4 +94,21 @@ __device__ __forceinline__ bool better_i32(int v, std::int64_t i, int best, std:
   return i < bi;
 }
 
+// float32 / int32 values ordered as 32-bit words.
+__device__ __forceinline__ bool word_nan(std::uint32_t a, bool fp) {
+  return fp && (a & 0x7fffffffU) > 0x7f800000U;
+}
+
+// Monotone key of the reference's float order (cpu_math.cpp:15-20): -0 maps
+// to +0, negative words are inverted, positive words get the top bit set.
+__device__ __forceinline__ std::uint32_t order_key(std::uint32_t a) {
+  if ((a & 0x7fffffffU) == 0) a = 0;
+  return (a & 0x80000000U) ? ~a : (a ^ 0x80000000U);
+}
+
+__device__ __forceinline__ bool word_less(std::uint32_t a, std::uint32_t b, bool fp) {
+  if (!fp) return static_cast<std::int32_t>(a) < static_cast<std::int32_t>(b);
+  return order_key(a) < order_key(b);
+}
+
 }  // namespace tcx

@@ -1,0 +1,91 @@
+"""topk on the device against the oracle at the sizes where its selection
+changes: rows that are all candidates, the threshold pass, the radix
+selection, and the three ways the chosen elements are put in order. Bit-exact
+values and indices."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+from conftest import require_gpu
+from hip_cases import assert_bits
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def cx():
+    require_gpu()
+    import tensorcx
+    return tensorcx
+
+
+def values_of(kind, shape, rng):
+    if kind == "int32":
+        return rng.integers(-2**31, 2**31, shape, dtype=np.int64).astype(np.int32)
+    if kind == "ties":  # more equal elements than the candidate buffer holds
+        return rng.integers(0, 3, shape).astype(np.float32)
+    if kind == "equal":
+        return np.full(shape, -0.0, np.float32)
+    x = rng.standard_normal(shape).astype(np.float32)
+    if kind == "special":
+        flat = x.reshape(-1)
+        at = rng.permutation(flat.size)[: max(8, flat.size // 8)]
+        flat[at] = rng.choice(np.array([np.nan, np.inf, -np.inf, 0.0, -0.0], np.float32), at.size)
+    return x
+
+
+def check(cx, x, axis, k, largest, sort):
+    values, indices = cx.topk(cx.tensor(x, device="hip"), k, axis, largest, sort)
+    expected_values, expected_indices = oracle.topk(x, k, axis, largest, sort)
+    what = f"{x.shape} axis={axis} k={k} largest={largest} sorted={sort}"
+    assert_bits(indices.numpy(), expected_indices, "indices " + what)
+    assert_bits(values.numpy(), expected_values, "values " + what)
+
+
+# (row length, ks): a wave takes rows up to 1024 and k up to 8 (with 1, 4 or 16
+# keys a lane), the direct rows end at 256 or 1024, the threshold pass at k = 64
+# or 256, the sort in LDS at k = 1024.
+EDGES = [(1, [1]), (63, [1, 8, 63]), (64, [2, 8, 9]), (65, [1, 8, 9]), (256, [1, 8, 64, 256]), (257, [1, 8, 64, 65, 257]),
+         (1024, [1, 8, 9, 64, 65, 1024]), (1025, [3, 8, 65, 256, 257, 1025]), (4097, [1, 64, 256, 1024, 1025, 4097]), (8192, [50, 64, 300]),
+         (8193, [50, 64, 256, 257]), (20001, [7, 256, 1500])]
+
+
+@pytest.mark.parametrize("kind", ["normal", "special", "ties", "equal", "int32"])
+@pytest.mark.parametrize("n,ks", EDGES, ids=[str(n) for n, _ in EDGES])
+def test_row_lengths_and_counts(cx, n, ks, kind):
+    rng = np.random.default_rng(n)
+    x = values_of(kind, (3, n), rng)
+    for k in ks:
+        for largest in (True, False):
+            for sort in (True, False):
+                check(cx, x, -1, k, largest, sort)
+
+
+@pytest.mark.parametrize("kind", ["special", "ties"])
+def test_other_axes(cx, kind):
+    rng = np.random.default_rng(5)
+    x = values_of(kind, (2, 1500, 3), rng)
+    for k in (1, 40, 70, 300, 1100, 1500):
+        check(cx, x, 1, k, True, True)
+        check(cx, x, 1, k, False, False)
+    short = values_of(kind, (3, 90, 7), rng)
+    for k in (1, 8, 9):
+        check(cx, short, 1, k, True, True)
+        check(cx, short, 1, k, False, False)
+
+
+def test_unaligned_rows(cx):
+    """Rows of an odd length start at every offset from a 16-byte boundary."""
+    rng = np.random.default_rng(6)
+    for n in (4099, 33001):
+        x = values_of("special", (9, n), rng)
+        check(cx, x, -1, 50, True, True)
+
+
+def test_more_rows_than_one_per_compute_unit(cx):
+    rng = np.random.default_rng(7)
+    check(cx, values_of("special", (3000, 70), rng), -1, 5, True, True)
+    check(cx, values_of("ties", (700, 1100), rng), -1, 20, True, False)
