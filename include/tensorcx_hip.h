@@ -441,6 +441,32 @@ int tcx_hip_flash_attention_f32(const float* q, const float* k, const float* v, 
                                 int64_t rows, int64_t cols, int64_t features, float scale, int causal,
                                 tcx_stream_t stream);
 
+typedef struct {
+  int64_t batch, rows, cols, features; /* as for tcx_hip_flash_attention_f32 */
+  float scale;
+  int32_t causal;
+  int32_t mask_kind; /* TCX_MASK_* */
+  /* The mask entry of (batch b, query i, key j), in elements: b counted
+   * row-major over mask_rank axes of mask_shape (their product is batch) with
+   * mask_strides, plus i * mask_row_stride + j * mask_col_stride. */
+  int32_t mask_rank;
+  int64_t mask_shape[TCX_HIP_MAX_RANK];
+  int64_t mask_strides[TCX_HIP_MAX_RANK];
+  int64_t mask_row_stride, mask_col_stride;
+} tcx_hip_flash_attention_desc_t;
+/* Workspace bytes that tcx_hip_flash_attention_f32_ws can use for desc: > 0
+ * when there are too few queries to fill the GPU, so that the keys are split
+ * over blocks whose states land in the workspace; 0 otherwise. */
+size_t tcx_hip_flash_attention_workspace_bytes(const tcx_hip_flash_attention_desc_t* desc);
+/* tcx_hip_flash_attention_f32 with a mask (kAttention's, core/inference.cpp:
+ * 123-161: false or -inf hides a key, other additive entries are added to the
+ * scaled score) and with that workspace (16-byte aligned; with NULL or fewer
+ * bytes than the query it runs unsplit). The workspace must stay allocated
+ * until the stream has run the call. */
+int tcx_hip_flash_attention_f32_ws(const float* q, const float* k, const float* v, float* out, const void* mask,
+                                   const tcx_hip_flash_attention_desc_t* desc, void* workspace,
+                                   size_t workspace_bytes, tcx_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

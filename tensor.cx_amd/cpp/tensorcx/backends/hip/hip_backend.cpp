@@ -934,19 +934,54 @@ Tensor attention(const OpDesc& op, std::span<const Tensor> inputs, Stream& s) {
   const AttentionSoftmaxPlan plan = attention_softmax_plan(softmax, preview);
   for (const Tensor& t : inputs) (void)device_ptr(t);
   if (numel(shape) == 0) return make_tensor(DType::kFloat32, shape);
-  // Unmasked attention over matching batches with 32/64/128 features: the
-  // fused kernel, scores never materialised.
+  // Attention over matching batches with 32/64/128 features: the fused
+  // kernels, scores never materialised.
   const Shape qb(q.shape.begin(), q.shape.end() - 2);
-  if (inputs.size() == 3 && qb == Shape(k.shape.begin(), k.shape.end() - 2) &&
-      qb == Shape(v.shape.begin(), v.shape.end() - 2) &&
-      tcx_hip_flash_attention_supported(features, v.shape.back()) &&
-      aligned16(device_ptr(q)) && aligned16(device_ptr(k)) && aligned16(device_ptr(v))) {
-    Tensor out = make_tensor(DType::kFloat32, shape);
-    ok_or_throw(tcx_hip_flash_attention_f32(f32(q), f32(k), f32(v), static_cast<float*>(out_ptr(out)), numel(qb),
-                                            rows, columns, features, *softmax.attention_scale, op.causal ? 1 : 0,
-                                            s),
-                "HIP attention");
-    return out;
+  if (qb == Shape(k.shape.begin(), k.shape.end() - 2) && qb == Shape(v.shape.begin(), v.shape.end() - 2) &&
+      tcx_hip_flash_attention_supported(features, v.shape.back()) && aligned16(device_ptr(q)) &&
+      aligned16(device_ptr(k)) && aligned16(device_ptr(v))) {
+    tcx_hip_flash_attention_desc_t d{};
+    d.batch = numel(qb);
+    d.rows = rows;
+    d.cols = columns;
+    d.features = features;
+    d.scale = static_cast<float>(*softmax.attention_scale);
+    d.causal = op.causal ? 1 : 0;
+    d.mask_kind = plan.mask_kind;
+    const Tensor* mask = inputs.size() == 4 ? &inputs[3] : nullptr;
+    bool fits = true;
+    if (mask != nullptr) {
+      const Shape strides = broadcast_strides(mask->shape, scores);
+      const Strided m = compress(qb, {Shape(strides.begin(), strides.end() - 2)}, 0, qb.size());
+      fits = m.shape.size() <= TCX_HIP_MAX_RANK;
+      if (fits) {
+        d.mask_rank = static_cast<int32_t>(m.shape.size());
+        for (std::size_t i = 0; i < m.shape.size(); ++i) {
+          d.mask_shape[i] = m.shape[i];
+          d.mask_strides[i] = m.strides[0][i];
+        }
+        d.mask_row_stride = strides[strides.size() - 2];
+        d.mask_col_stride = strides.back();
+      }
+    }
+    if (fits) {
+      Tensor out = make_tensor(DType::kFloat32, shape);
+      // With few queries the keys are split over blocks, their states in a
+      // workspace held until the stream has finished (without one, when that
+      // allocation fails, the keys stay together).
+      const std::size_t ws = tcx_hip_flash_attention_workspace_bytes(&d);
+      std::shared_ptr<HipBuffer> workspace;
+      if (ws) {
+        auto created = HipBuffer::create(ws);
+        if (created) workspace = created.move_value();
+      }
+      ok_or_throw(tcx_hip_flash_attention_f32_ws(f32(q), f32(k), f32(v), static_cast<float*>(out_ptr(out)),
+                                                 mask ? device_ptr(*mask) : nullptr, &d,
+                                                 workspace ? workspace->data() : nullptr, workspace ? ws : 0, s),
+                  "HIP attention");
+      if (workspace) ok_or_throw(tcx_hip_stream_synchronize(s), "HIP attention");
+      return out;
+    }
   }
   if (columns == 0) {  // no keys: every output row is an empty sum
     Tensor zeros;

@@ -2,12 +2,18 @@
 // materialising the scores, on v_mfma_f32_16x16x4_f32.
 //
 // Semantics are those of the reference composite (core/inference.cpp:123-161
-// over backends/cpu/cpu_inference.cpp:22-47) for unmasked and causal
-// attention: a score is dot(q, k) * scale (rounded), a key after the query is
-// -inf under causal, a row with any NaN score is NaN, a row whose maximum is
-// -inf is 0 * V, otherwise exp(s - max) / sum, times V. The sums run in a
-// different order (online softmax over key tiles), inside the reference
-// test's allclose(rtol=2e-4, atol=2e-5).
+// over backends/cpu/cpu_inference.cpp:22-47): a score is dot(q, k) * scale
+// (rounded) plus the additive mask (rounded); a key after the query under
+// causal, a false entry of a bool mask or a -inf entry of an additive one is
+// -inf; a row with any NaN score is NaN, a row whose maximum is -inf is 0 * V,
+// otherwise exp(s - max) / sum, times V. The sums run in a different order
+// (online softmax over key tiles), inside the reference test's
+// allclose(rtol=2e-4, atol=2e-5).
+//
+// Two kernels share the work: flash_attention_kernel, below, with matrix
+// instructions for 16 queries a wave, and flash_decode_kernel for up to four
+// queries, which only streams K and V. Where either has too few blocks for the
+// GPU, the keys are split over blocks and flash_combine_kernel joins the parts.
 //
 // Layout. A block owns 16 queries per wave of one batch matrix and walks the
 // keys in tiles of kKeys (64, or 32 where two blocks must share a CU). K and V
@@ -25,6 +31,9 @@
 // columns where its V rows hold a non-finite value (0 * inf or 0 * NaN is NaN
 // in every output row of the block). Blocks start with the longest query
 // tiles under causal masking.
+
+#include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 
@@ -44,7 +53,36 @@ struct FlashArgs {
   int causal;
   int xcd_blocks;   // group the blocks of one batch matrix on one XCD
   int heavy_first;  // causal: more blocks than fit at once, heaviest first
+  // Mask: element (batch b, query i, key j) at b's offset + i mask_row + j mask_col.
+  const void* mask;
+  int mask_kind;  // TCX_MASK_*
+  int mask_rank;
+  std::int64_t mask_shape[TCX_HIP_MAX_RANK], mask_stride[TCX_HIP_MAX_RANK];
+  std::int64_t mask_row, mask_col;
+  // Key split: split s of a work item takes split_keys keys from s split_keys
+  // (a multiple of the kernel's key tile); with splits > 1 its unnormalised
+  // outputs and its maxima and sums go to part and part_ml.
+  std::int64_t splits, split_keys;
+  float* part;     // [splits, batch, rows, D]
+  float* part_ml;  // [splits, batch, rows, 2]
 };
+
+// Offset of batch matrix b in the mask (its leading axes, row-major).
+__device__ __forceinline__ std::int64_t mask_offset(const FlashArgs& a, std::int64_t b) {
+  std::int64_t offset = 0;
+  for (int i = a.mask_rank - 1; i >= 0; --i) {
+    offset += b % a.mask_shape[i] * a.mask_stride[i];
+    b /= a.mask_shape[i];
+  }
+  return offset;
+}
+
+// The score under mask element `at`: + bias, or -inf where it is hidden.
+__device__ __forceinline__ float masked_score(float score, const FlashArgs& a, std::int64_t at) {
+  if (a.mask_kind == TCX_MASK_BOOL) return static_cast<const std::uint8_t*>(a.mask)[at] ? score : -__builtin_inff();
+  const float bias = static_cast<const float*>(a.mask)[at];
+  return bias == -__builtin_inff() ? bias : score + bias;
+}
 
 using float2_t = float __attribute__((ext_vector_type(2)));
 
@@ -114,16 +152,20 @@ __device__ __forceinline__ void flash_init(FlashState<kT>& st) {
 // folded into the state of the calling wave's 16 queries by the block's
 // kWaves waves (thread tid) on two K and two V stages. kKeys keys per tile
 // (64, or 32 to fit two blocks per CU), kB = kKeys / 16 MFMA blocks of keys.
-// With scan_tail, the V rows after the range (keys the causal mask hides from
-// every query of the tile) mark the feature columns holding an inf or NaN in
-// bad_column, cleared by the caller. The segment opens with a barrier, so a
-// segment may follow another on the same stages.
-
-template <int D, int kWaves, int kKeys, bool kCausal>
+// With scan_from >= 0, the V rows from key tile scan_from on (keys the causal
+// mask hides from every query of the tile) mark the feature columns holding an
+// inf or NaN in bad_column, cleared by the caller. The segment opens with a
+// barrier, so a segment may follow another on the same stages.
+//
+// kMask (TCX_MASK_*): lane (r, g) needs the mask entries of its query at keys
+// 16b + 4g + v, 4 kB words a tile. They are loaded a tile ahead, behind the
+// tile's DMA and ahead of the wait that ends the iteration: a load whose value
+// is used in its own iteration would wait for the DMA issued before it.
+template <int D, int kWaves, int kKeys, bool kCausal, int kMask>
 __device__ __forceinline__ void flash_segment(const FlashArgs& a, float (&ks)[2][kKeys * D],
                                               float (&vs)[2][kKeys * D], int* bad_column, int tid,
                                               std::int64_t batch, std::int64_t qtile, std::int64_t t_begin,
-                                              std::int64_t t_end, bool scan_tail, FlashState<D / 16>& st) {
+                                              std::int64_t t_end, std::int64_t scan_from, FlashState<D / 16>& st) {
   constexpr int kQTile = 16 * kWaves;
   constexpr int kT = D / 16;
   constexpr int kB = kKeys / 16;
@@ -253,6 +295,29 @@ __device__ __forceinline__ void flash_segment(const FlashArgs& a, float (&ks)[2]
   float tmax = neg_inf, m_new = neg_inf, m_sub = 0.F, alpha = 1.F, psum = 0.F;
   float av[4];
   int limit = kKeys;
+  using mask_word = std::conditional_t<kMask == TCX_MASK_BOOL, std::uint8_t, float>;
+  mask_word mk[kMask == TCX_MASK_NONE ? 1 : 4 * kB], mk_next[kMask == TCX_MASK_NONE ? 1 : 4 * kB];
+  const mask_word* __restrict__ mrow = nullptr;
+  if constexpr (kMask != TCX_MASK_NONE)
+    mrow = static_cast<const mask_word*>(a.mask) + mask_offset(a, batch) + min(query, a.rows - 1) * a.mask_row;
+  // Keys past the sequence read the last one's entry; the limit hides them.
+  auto load_mask = [&](std::int64_t tile, mask_word (&to)[kMask == TCX_MASK_NONE ? 1 : 4 * kB]) {
+    if constexpr (kMask != TCX_MASK_NONE) {
+      const std::int64_t j0 = tile * kKeys;
+      if (j0 + kKeys <= a.cols) {
+        const mask_word* __restrict__ p = mrow + (j0 + 4 * g) * a.mask_col;
+#pragma unroll
+        for (int b = 0; b < kB; ++b)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) to[4 * b + v] = p[(16 * b + v) * a.mask_col];
+      } else {
+#pragma unroll
+        for (int b = 0; b < kB; ++b)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) to[4 * b + v] = mrow[min(j0 + 16 * b + 4 * g + v, a.cols - 1) * a.mask_col];
+      }
+    }
+  };
   auto begin_tile = [&](std::int64_t tile) {
     const std::int64_t j0 = tile * kKeys;
     std::int64_t lim = a.cols - j0;
@@ -263,13 +328,18 @@ __device__ __forceinline__ void flash_segment(const FlashArgs& a, float (&ks)[2]
     tmax = neg_inf;
     psum = 0.F;
   };
-  // kMask: the tile may hold keys past the sequence or after the query.
-  auto step = [&]<int I, bool kMask>(mfma_acc (&s)[kB]) {
+  // kLimit: the tile may hold keys past the sequence or after the query.
+  auto step = [&]<int I, bool kLimit>(mfma_acc (&s)[kB]) {
     if constexpr (I < kB) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         float sc = s[I][v] * a.scale;
-        if constexpr (kMask) {
+        if constexpr (kMask == TCX_MASK_BOOL) {
+          sc = mk[4 * I + v] != 0 ? sc : neg_inf;
+        } else if constexpr (kMask == TCX_MASK_ADDITIVE) {
+          sc = mk[4 * I + v] == neg_inf ? neg_inf : sc + mk[4 * I + v];
+        }
+        if constexpr (kLimit) {
           if (16 * I + 4 * g + v >= limit) sc = neg_inf;
         }
         s[I][v] = sc;
@@ -325,10 +395,10 @@ __device__ __forceinline__ void flash_segment(const FlashArgs& a, float (&ks)[2]
   // and the K reads of group t + 1 in the first quad of group t; the last quad
   // also reads the first P V step's V operands.
   constexpr int kQuads = kT * kB;
-  auto scores_with_softmax = [&]<bool kMask, int... Q>(const float* __restrict__ kt_, const float* __restrict__ vt_,
+  auto scores_with_softmax = [&]<bool kLimit, int... Q>(const float* __restrict__ kt_, const float* __restrict__ vt_,
                                                        mfma_acc (&s_next)[kB], mfma_acc (&s)[kB],
                                                        float4_t (&kf)[2][kB], float (&vv)[2][kT],
-                                                       std::bool_constant<kMask>, std::integer_sequence<int, Q...>) {
+                                                       std::bool_constant<kLimit>, std::integer_sequence<int, Q...>) {
     auto quad = [&]<int J>() {
       constexpr int t = J / kB, e0 = (J % kB) * (4 / kB);
       if constexpr (J % kB == 0 && t + 1 < kT) read_k(kt_, t + 1, kf[(t + 1) & 1]);
@@ -340,7 +410,7 @@ __device__ __forceinline__ void flash_segment(const FlashArgs& a, float (&ks)[2]
           s_next[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t & 1][b][e], qf[t][e], s_next[b], 0, 0, 0);
       [&]<int... I>(std::integer_sequence<int, I...>) {
         ([&] {
-          if constexpr (I * kQuads / kSteps == J) step.template operator()<I, kMask>(s);
+          if constexpr (I * kQuads / kSteps == J) step.template operator()<I, kLimit>(s);
         }(), ...);
       }(std::make_integer_sequence<int, kSteps>{});
       __builtin_amdgcn_sched_barrier(0);
@@ -372,6 +442,7 @@ __device__ __forceinline__ void flash_segment(const FlashArgs& a, float (&ks)[2]
     issue(kb, ks[0], t_begin);
     issue(vb, vs[0], t_begin);
     if (t_begin + 1 < t_end) issue(kb, ks[1], t_begin + 1);
+    load_mask(t_begin, mk);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();  // K 0, V 0 and K 1 have landed
     scores(ks[0], s_cur);
@@ -388,6 +459,7 @@ __device__ __forceinline__ void flash_segment(const FlashArgs& a, float (&ks)[2]
     const int st = static_cast<int>((tile - t_begin) & 1);
     issue(vb, vs[st ^ 1], tile + 1);
     if (tile + 2 < t_end) issue(kb, ks[st], tile + 2);
+    load_mask(tile + 1, mk_next);
     begin_tile(tile);
 #pragma unroll
     for (int b = 0; b < kB; ++b) s_next[b] = mfma_acc{0.F, 0.F, 0.F, 0.F};
@@ -406,6 +478,10 @@ __device__ __forceinline__ void flash_segment(const FlashArgs& a, float (&ks)[2]
 #pragma unroll
     for (int b = 0; b < kB; ++b) s_cur[b] = s_next[b];
     __builtin_amdgcn_s_waitcnt(0);  // this wave's loads have landed
+    if constexpr (kMask != TCX_MASK_NONE) {
+#pragma unroll
+      for (int e = 0; e < 4 * kB; ++e) mk[e] = mk_next[e];
+    }
     __syncthreads();                // and every wave is done with this iteration's stages
   }
   if (tile < t_end) {
@@ -416,7 +492,7 @@ __device__ __forceinline__ void flash_segment(const FlashArgs& a, float (&ks)[2]
     accumulate(vs[st], s_cur, vv, std::make_integer_sequence<int, 4 * kB>{});
   }
 
-  if (scan_tail && t_end < tiles) {
+  if (scan_from >= 0 && scan_from < tiles) {
     // Columns of the V rows past the last run tile that hold an inf or NaN
     // (exponent all ones), eight independent loads in flight per thread and
     // no branch in the loop (a branch on each load's value serialised the
@@ -429,7 +505,7 @@ __device__ __forceinline__ void flash_segment(const FlashArgs& a, float (&ks)[2]
 #pragma unroll
       for (int e = 0; e < 4; ++e) flag[e] |= (__float_as_uint(w[e]) & kExp) == kExp ? 1U : 0U;
     };
-    std::int64_t row = t_end * kKeys + tid / (D / 4);
+    std::int64_t row = scan_from * kKeys + tid / (D / 4);
     for (; row + 7 * kPass < a.cols; row += 8 * kPass) {
       float4_t w[8];
 #pragma unroll
@@ -445,17 +521,20 @@ __device__ __forceinline__ void flash_segment(const FlashArgs& a, float (&ks)[2]
 }
 
 // Stores the calling wave's 16 output rows of query tile `qtile` from its
-// state (NaN in the columns bad_column marks, 0 * V for an all-masked row).
+// state (NaN in the columns bad_column marks, 0 * V for an all-masked row), or,
+// of one split of the keys, the state itself.
 template <int D, int kWaves>
 __device__ __forceinline__ void flash_store(const FlashArgs& a, const int* bad_column, int tid, std::int64_t batch,
-                                            std::int64_t qtile, const FlashState<D / 16>& st) {
+                                            std::int64_t qtile, std::int64_t split, const FlashState<D / 16>& st) {
   constexpr int kT = D / 16;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
   const std::int64_t q0 = qtile * (16 * kWaves) + wave * 16;
   const float neg_inf = -__builtin_inff();
-  float* __restrict__ ob = a.out + batch * a.rows * D;
+  const bool parts = a.splits > 1;
+  const std::int64_t first = (split * a.batch + batch) * a.rows;  // this split's row 0 of the batch matrix
+  float* __restrict__ ob = parts ? a.part + first * D : a.out + batch * a.rows * D;
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
     const int src = 4 * g + v;
@@ -467,9 +546,11 @@ __device__ __forceinline__ void flash_store(const FlashArgs& a, const int* bad_c
 #pragma unroll
     for (int t = 0; t < kT; ++t) {
       if (bad_column[output_feature<kT>(r, t)]) y[t] = __builtin_nanf("");
+      else if (parts) y[t] = st.o[t][v];
       else if (mv == neg_inf) y[t] = st.o[t][v] * 0.F;
       else y[t] = st.o[t][v] / lv;
     }
+    if (parts && r == 0) *reinterpret_cast<float2_t*>(a.part_ml + (first + qrow) * 2) = float2_t{mv, lv};
     float* const orow = ob + qrow * D;
     if constexpr (kT >= 4) {
 #pragma unroll
@@ -482,9 +563,9 @@ __device__ __forceinline__ void flash_store(const FlashArgs& a, const int* bad_c
   }
 }
 
-// One block per query tile.
-template <int D, int kWaves, int kKeys, bool kCausal>
-__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 8))) void flash_attention_kernel(
+// One block per query tile and split of the keys.
+template <int D, int kWaves, int kKeys, bool kCausal, int kMask>
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWaves == 1 ? 1 : 2, 8))) void flash_attention_kernel(
     FlashArgs a) {
   constexpr int kQTile = 16 * kWaves;
   __shared__ float ks[2][kKeys * D];
@@ -494,7 +575,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
   // One block per work item on a 1-D grid of n = qtiles x batch blocks; the
   // launch id maps to an item (batch-major by default).
   const std::int64_t n = a.qtiles * a.batch;
-  const std::int64_t id = blockIdx.x;
+  const std::int64_t split = blockIdx.x / n, id = blockIdx.x % n;
   std::int64_t batch = id / a.qtiles, qtile = id % a.qtiles;
   if (a.xcd_blocks) {
     // Launch id L runs on XCD L % 8: give XCD x the consecutive (batch-major)
@@ -522,23 +603,330 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
   const std::int64_t tiles = (a.cols + kKeys - 1) / kKeys;
   // Under causal masking tiles past the block's last query are not run.
   const std::int64_t run = kCausal ? min(tiles, q_last / kKeys + 1) : tiles;
+  const std::int64_t per = a.split_keys / kKeys;
+  const std::int64_t t_begin = min(split * per, run), t_end = min(t_begin + per, run);
   for (int d = tid; d < D; d += 64 * kWaves) bad_column[d] = 0;
   FlashState<D / 16> st;
   flash_init(st);
-  flash_segment<D, kWaves, kKeys, kCausal>(a, ks, vs, bad_column, tid, batch, qtile, 0, run, true, st);
+  flash_segment<D, kWaves, kKeys, kCausal, kMask>(a, ks, vs, bad_column, tid, batch, qtile, t_begin, t_end,
+                                                  split == a.splits - 1 ? run : -1, st);
   __syncthreads();
-  flash_store<D, kWaves>(a, bad_column, tid, batch, qtile, st);
+  flash_store<D, kWaves>(a, bad_column, tid, batch, qtile, split, st);
 }
 
-template <int D, int kWaves, int kKeys, bool kCausal>
-int launch_flash(FlashArgs a, std::int64_t batch, hipStream_t s) {
+// Sum over the kLanes lanes (8 or 16) of a group, in every lane of it.
+template <int kLanes>
+__device__ __forceinline__ float group_sum(float x) {
+  auto add = [&]<int kControl>() {
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), kControl, 0xf, 0xf, true));
+  };
+  add.template operator()<0xb1>();   // lane ^ 1
+  add.template operator()<0x4e>();   // lane ^ 2
+  add.template operator()<0x141>();  // mirror in eight lanes
+  if constexpr (kLanes == 16) add.template operator()<0x140>();  // mirror in sixteen
+  return x;
+}
+
+// Joins the online-softmax state (m, l and N outputs) of two disjoint sets of keys.
+template <int N>
+__device__ __forceinline__ void join_state(float& m, float& l, float (&o)[N], float m2, float l2, const float (&o2)[N]) {
+  const float top = fmaxf(m, m2);
+  const float at = top == -__builtin_inff() ? 0.F : top;
+  const float f = exp_attention(m - at), f2 = exp_attention(m2 - at);
+  m = top;
+  l = l * f + l2 * f2;
+#pragma unroll
+  for (int e = 0; e < N; ++e) o[e] = o[e] * f + o2[e] * f2;
+}
+
+// Attention of kRows queries (the last ones may repeat) over split_keys keys
+// of one batch matrix, not causal: decoding, where a K and a V row are used
+// once and the time is that of reading them. A group of lanes takes a key and
+// each lane kC 16-byte chunks of its rows; kEach keys a group and pass, so that
+// 16 loads a lane are in flight. Every group keeps an online softmax of its own
+// (no exchange between groups in the loop); the groups are joined at the end.
+// 32 heads of one query and 4096 keys, D = 128 (134 MB): 24.1 us with the
+// combine (5.6 TB/s), against 537 us for one block of flash_attention_kernel
+// per head.
+template <int D, int kRows>
+__global__ __launch_bounds__(256) void flash_decode_kernel(FlashArgs a) {
+  constexpr int kLanes = D >= 64 ? 16 : 8;
+  constexpr int kC = D / 4 / kLanes;
+  constexpr int kEach = 8 / kC;
+  constexpr int kPerWave = 64 / kLanes;
+  constexpr int kGroups = 4 * kPerWave;
+  constexpr int kPass = kGroups * kEach;
+  __shared__ float part_o[4][kRows][D];
+  __shared__ float part_m[4][kRows], part_l[4][kRows];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int li = lane % kLanes, group = wave * kPerWave + lane / kLanes;
+  const std::int64_t batch = blockIdx.x / a.splits, split = blockIdx.x % a.splits;
+  const std::int64_t k0 = split * a.split_keys, k1 = min(k0 + a.split_keys, a.cols);
+  const float neg_inf = -__builtin_inff();
+  const float* __restrict__ kb = a.k + batch * a.cols * D + 4 * li;
+  const float* __restrict__ vb = a.v + batch * a.cols * D + 4 * li;
+  const std::int64_t mask0 = a.mask_kind != TCX_MASK_NONE ? mask_offset(a, batch) : 0;
+  float4_t q[kRows][kC];
+  float o[kRows][4 * kC], m[kRows], l[kRows];
+#pragma unroll
+  for (int r = 0; r < kRows; ++r) {
+    const std::int64_t row = min(static_cast<std::int64_t>(r), a.rows - 1);
+#pragma unroll
+    for (int c = 0; c < kC; ++c)
+      q[r][c] = *reinterpret_cast<const float4_t*>(a.q + (batch * a.rows + row) * D + 4 * (c * kLanes + li));
+#pragma unroll
+    for (int e = 0; e < 4 * kC; ++e) o[r][e] = 0.F;
+    m[r] = neg_inf;
+    l[r] = 0.F;
+  }
+  auto pass = [&]<bool kTail>(std::int64_t j, std::bool_constant<kTail>) {
+    float4_t kf[kEach][kC], vf[kEach][kC];
+    std::int64_t key[kEach];
+#pragma unroll
+    for (int u = 0; u < kEach; ++u) {
+      key[u] = j + u * kGroups + group;
+      const std::int64_t at = kTail ? min(key[u], k1 - 1) : key[u];
+#pragma unroll
+      for (int c = 0; c < kC; ++c) kf[u][c] = stream_load(reinterpret_cast<const float4_t*>(kb + at * D + 4 * c * kLanes));
+    }
+#pragma unroll
+    for (int u = 0; u < kEach; ++u) {
+      const std::int64_t at = kTail ? min(key[u], k1 - 1) : key[u];
+#pragma unroll
+      for (int c = 0; c < kC; ++c) {
+        vf[u][c] = stream_load(reinterpret_cast<const float4_t*>(vb + at * D + 4 * c * kLanes));
+        if (kTail && key[u] >= k1) vf[u][c] = float4_t{0.F, 0.F, 0.F, 0.F};
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+      float s[kEach], top = m[r];
+#pragma unroll
+      for (int u = 0; u < kEach; ++u) {
+        float dot = 0.F;
+#pragma unroll
+        for (int c = 0; c < kC; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) dot = fmaf(q[r][c][e], kf[u][c][e], dot);
+        s[u] = group_sum<kLanes>(dot) * a.scale;
+        if (a.mask_kind != TCX_MASK_NONE)
+          s[u] = masked_score(s[u], a, mask0 + min(static_cast<std::int64_t>(r), a.rows - 1) * a.mask_row +
+                                           min(key[u], a.cols - 1) * a.mask_col);
+        if (kTail && key[u] >= k1) s[u] = neg_inf;
+        top = fmaxf(top, s[u]);
+      }
+      const float at = top == neg_inf ? 0.F : top;  // as in flash_segment: every key so far hidden
+      const float f = exp_attention(m[r] - at);
+      m[r] = top;
+      l[r] *= f;
+#pragma unroll
+      for (int e = 0; e < 4 * kC; ++e) o[r][e] *= f;
+#pragma unroll
+      for (int u = 0; u < kEach; ++u) {
+        const float p = exp_attention(s[u] - at);
+        l[r] += p;
+#pragma unroll
+        for (int c = 0; c < kC; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[r][4 * c + e] = fmaf(p, vf[u][c][e], o[r][4 * c + e]);
+      }
+    }
+  };
+  std::int64_t j = k0;
+  for (; j + kPass <= k1; j += kPass) pass(j, std::false_type{});
+  if (j < k1) pass(j, std::true_type{});
+#pragma unroll
+  for (int r = 0; r < kRows; ++r) {
+#pragma unroll
+    for (int offset = kLanes; offset < 64; offset <<= 1) {
+      float o2[4 * kC];
+      const float m2 = __shfl_xor(m[r], offset, kWave), l2 = __shfl_xor(l[r], offset, kWave);
+#pragma unroll
+      for (int e = 0; e < 4 * kC; ++e) o2[e] = __shfl_xor(o[r][e], offset, kWave);
+      join_state(m[r], l[r], o[r], m2, l2, o2);
+    }
+    if (lane < kLanes) {
+#pragma unroll
+      for (int c = 0; c < kC; ++c)
+        *reinterpret_cast<float4_t*>(&part_o[wave][r][4 * (c * kLanes + li)]) =
+            float4_t{o[r][4 * c], o[r][4 * c + 1], o[r][4 * c + 2], o[r][4 * c + 3]};
+      if (lane == 0) {
+        part_m[wave][r] = m[r];
+        part_l[wave][r] = l[r];
+      }
+    }
+  }
+  __syncthreads();
+  const std::int64_t first = (split * a.batch + batch) * a.rows;
+  for (int i = t; i < kRows * D; i += 256) {
+    const int r = i / D, d = i % D;
+    if (r >= a.rows) break;
+    float mv = part_m[0][r], lv = part_l[0][r], ov[1] = {part_o[0][r][d]};
+#pragma unroll
+    for (int w = 1; w < 4; ++w) {
+      const float o2[1] = {part_o[w][r][d]};
+      join_state(mv, lv, ov, part_m[w][r], part_l[w][r], o2);
+    }
+    if (a.splits > 1) {
+      a.part[(first + r) * D + d] = ov[0];
+      if (d == 0) *reinterpret_cast<float2_t*>(a.part_ml + (first + r) * 2) = float2_t{mv, lv};
+    } else {
+      a.out[(batch * a.rows + r) * D + d] = mv == neg_inf ? ov[0] * 0.F : ov[0] / lv;
+    }
+  }
+}
+
+// Joins the splits of every output row, one wave a row (splits <= 64: lane s
+// holds the maximum and the sum of split s), in the order of the splits.
+template <int D>
+__global__ __launch_bounds__(256) void flash_combine_kernel(FlashArgs a) {
+  constexpr int kE = D >= 64 ? D / 64 : 1;
+  const int lane = threadIdx.x & 63;
+  const std::int64_t rows = a.batch * a.rows;
+  const std::int64_t step = static_cast<std::int64_t>(gridDim.x) * 4;
+  const int splits = static_cast<int>(a.splits);
+  const float neg_inf = -__builtin_inff();
+  for (std::int64_t row = static_cast<std::int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6); row < rows; row += step) {
+    float2_t ml{neg_inf, 0.F};
+    if (lane < splits) ml = *reinterpret_cast<const float2_t*>(a.part_ml + (lane * rows + row) * 2);
+    float top = ml.x;
+#pragma unroll
+    for (int offset = 32; offset > 0; offset >>= 1) top = fmaxf(top, __shfl_xor(top, offset, kWave));
+    const float at = top == neg_inf ? 0.F : top;
+    const float weight = exp_attention(ml.x - at);
+    const float sum = wave_sum(ml.y * weight);
+    const int d = lane * kE;
+    float y[kE] = {};
+    if (d < D) {
+      const float* __restrict__ p = a.part + row * D + d;
+      auto add = [&]<int kN>(int s, std::integral_constant<int, kN>) {  // splits s .. s + kN - 1
+        float v[kN][kE];
+#pragma unroll
+        for (int u = 0; u < kN; ++u)
+#pragma unroll
+          for (int e = 0; e < kE; ++e) v[u][e] = p[(s + u) * rows * D + e];
+#pragma unroll
+        for (int u = 0; u < kN; ++u) {
+          const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), s + u));
+#pragma unroll
+          for (int e = 0; e < kE; ++e) y[e] += w * v[u][e];
+        }
+      };
+      int s = 0;
+      for (; s + 8 <= splits; s += 8) add(s, std::integral_constant<int, 8>{});
+      for (; s < splits; ++s) add(s, std::integral_constant<int, 1>{});
+#pragma unroll
+      for (int e = 0; e < kE; ++e) a.out[row * D + d + e] = top == neg_inf ? y[e] * 0.F : y[e] / sum;
+    }
+  }
+}
+
+// How one call runs: the kernel and its split of the keys.
+struct FlashPlan {
+  bool decode;      // flash_decode_kernel
+  int waves, keys;  // of flash_attention_kernel
+  std::int64_t splits, split_keys;
+  std::size_t bytes;  // of the workspace that holds the splits' states
+};
+
+std::int64_t ceil_div(std::int64_t a, std::int64_t b) { return (a + b - 1) / b; }
+
+constexpr std::int64_t kDecodeRows = 4;
+constexpr std::int64_t kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};  // flash_combine_kernel: a lane each
+
+// A form of flash_attention_kernel and what a key tile costs in it, in
+// microseconds of one CU: in a block that has the CU to itself, and for each
+// block where several share it.
+struct FlashForm {
+  int waves, keys;
+  double alone, shared;
+  int resident;  // blocks a CU holds
+};
+
+// The split of the keys that is expected to end first, with its time in
+// microseconds. A block's time is its tiles on the busiest of 256 CUs and 4 us
+// of start and end a round; a split call also runs the combine (4 us and the
+// states written and read at 4 TB/s). Under causal masking almost half of the
+// parts of a split are empty. Within 15 % of what MI355X took for 20 shapes of
+// 3 to 512 matrices, 5 to 2048 queries and 128 to 4096 keys; a split has to
+// promise 8 %.
+double best_split(const FlashForm& f, std::int64_t batch, std::int64_t rows, std::int64_t cols, std::int64_t features,
+                  bool causal, std::int64_t& splits) {
+  const std::int64_t items = ceil_div(rows, 16 * f.waves) * batch, tiles = std::max<std::int64_t>(ceil_div(cols, f.keys), 1);
+  double best = 0;
+  splits = 1;
+  for (const std::int64_t n : kSplits) {
+    if (n > 1 && (n > tiles || items * n > 2048)) break;
+    const std::int64_t per = ceil_div(tiles, n);
+    if (n > 1 && ceil_div(tiles, per) != n) continue;  // another count cuts the tiles the same way
+    const double blocks = static_cast<double>(causal && n > 1 ? items * (n + 1) : items * n) * (causal && n > 1 ? 0.6 : 1.0);
+    const std::int64_t on_cu = ceil_div(static_cast<std::int64_t>(blocks), 256);
+    double time = static_cast<double>(per) * (on_cu > 1 ? static_cast<double>(on_cu) * f.shared : f.alone);
+    if (causal && n == 1 && on_cu > 1)  // the light blocks fill in beside the heavy ones
+      time = std::max(static_cast<double>(per) * f.alone, 0.5 * time);
+    time += 4.0 * static_cast<double>(ceil_div(on_cu, f.resident));
+    if (n > 1) time += 4.0 + static_cast<double>(n * batch * rows * features) * 2e-6;
+    if (n == 1) best = time;
+    else if (time < 0.92 * best) best = time, splits = n;
+  }
+  return best;
+}
+
+FlashPlan flash_plan(std::int64_t batch, std::int64_t rows, std::int64_t cols, std::int64_t features, bool causal,
+                     int mask_kind) {
+  FlashPlan p{};
+  if (rows <= kDecodeRows && !causal && cols > 0) {
+    // Up to 256 blocks of at least 128 keys (8 splits of 32 x 4096 x 128 24.1
+    // us, 32 splits 25.2, one 91.4); short sequences whole, since the combine
+    // costs more than it brings (16 x 300 x 64 6.6 us, 8.2 in two).
+    p.decode = true;
+    std::int64_t splits = 1;
+    for (const std::int64_t n : kSplits)
+      if (n * batch <= 256 && n * 128 <= cols && cols >= 512) splits = n;
+    p.split_keys = ceil_div(ceil_div(cols, splits), 64) * 64;
+    p.splits = ceil_div(cols, p.split_keys);
+  } else {
+    // Tile shapes measured on MI355X. Four waves and 32-key tiles in general:
+    // at D = 128 64 KB of LDS, so that two blocks share a CU, under causal
+    // masking a heavy and a light one (89 TFLOP/s at 16 x 2048 x 128 against
+    // 86 for a register-staged 4-wave kernel, 92 against 71 at 32 x 2048 x 64).
+    // Unmasked at D = 64 and 128 also eight waves and 64-key tiles (one block
+    // per CU): 281 against 291 us at 16 x 2048 x 128, but 78 against 53 at 16 x
+    // 1024 x 64, where its blocks are too few; at D = 32 94 against 90 TFLOP/s
+    // for the small tiles. Up to 16 queries one wave holds them all: 60 us
+    // against 81 for 512 matrices of 16 queries and 512 keys at D = 128.
+    const int d = features == 128 ? 2 : features == 64 ? 1 : 0;
+    static constexpr FlashForm kFour[] = {{4, 32, 1.0, 0.8, 5}, {4, 32, 1.53, 1.27, 4}, {4, 32, 2.65, 2.27, 2}};
+    static constexpr FlashForm kEight[] = {{}, {8, 64, 4.6, 4.6, 1}, {8, 64, 8.7, 8.7, 1}};
+    static constexpr FlashForm kOne[] = {{1, 32, 1.0, 0.4, 8}, {1, 32, 1.7, 0.6, 5}, {1, 32, 2.85, 1.9, 2}};
+    const bool plain = !causal && mask_kind == TCX_MASK_NONE;
+    FlashForm form = plain && rows <= 16 ? kOne[d] : kFour[d];
+    double time = best_split(form, batch, rows, cols, features, causal, p.splits);
+    if (plain && rows > 64 && features >= 64) {
+      std::int64_t splits;
+      if (best_split(kEight[d], batch, rows, cols, features, false, splits) < time) {
+        form = kEight[d];
+        p.splits = splits;
+      }
+    }
+    p.waves = form.waves;
+    p.keys = form.keys;
+    p.split_keys = std::max<std::int64_t>(ceil_div(ceil_div(cols, p.keys), p.splits), 1) * p.keys;
+    p.splits = std::max<std::int64_t>(ceil_div(cols, p.split_keys), 1);
+  }
+  if (p.splits > 1) p.bytes = static_cast<std::size_t>(p.splits * batch * rows) * (features + 2) * sizeof(float);
+  return p;
+}
+
+template <int D, int kWaves, int kKeys, bool kCausal, int kMask>
+int launch_flash(FlashArgs a, hipStream_t s) {
   constexpr int kQTile = 16 * kWaves;
-  a.qtiles = (a.rows + kQTile - 1) / kQTile;
-  a.batch = batch;
-  if (a.qtiles > 0x7fffffff / batch) return fail(TCX_INVALID_ARGUMENT, "attention grid is too large");
-  const std::int64_t blocks = a.qtiles * batch;
+  a.qtiles = ceil_div(a.rows, kQTile);
+  if (a.qtiles > 0x7fffffff / a.batch / a.splits) return fail(TCX_INVALID_ARGUMENT, "attention grid is too large");
+  const std::int64_t items = a.qtiles * a.batch;
+  const std::int64_t blocks = items * a.splits;
   // Causal blocks keep their heavy/light order instead.
-  a.xcd_blocks = !kCausal && blocks % 8 == 0 ? 1 : 0;
+  a.xcd_blocks = !kCausal && items % 8 == 0 ? 1 : 0;
   if constexpr (kCausal) {
     thread_local int slots = 0;
     if (slots == 0) {
@@ -546,17 +934,47 @@ int launch_flash(FlashArgs a, std::int64_t batch, hipStream_t s) {
       (void)hipGetDevice(&device);
       if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus < 1)
         cus = 256;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, flash_attention_kernel<D, kWaves, kKeys, kCausal>,
-                                                        64 * kWaves, 0) != hipSuccess ||
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+              &per_cu, flash_attention_kernel<D, kWaves, kKeys, kCausal, kMask>, 64 * kWaves, 0) != hipSuccess ||
           per_cu < 1)
         per_cu = 2;
       slots = per_cu * cus;
     }
     a.heavy_first = blocks > slots ? 1 : 0;
   }
-  hipLaunchKernelGGL((flash_attention_kernel<D, kWaves, kKeys, kCausal>), dim3(static_cast<unsigned>(blocks)),
+  hipLaunchKernelGGL((flash_attention_kernel<D, kWaves, kKeys, kCausal, kMask>), dim3(static_cast<unsigned>(blocks)),
                      dim3(64 * kWaves), 0, s, a);
   return check(hipGetLastError(), "flash attention launch");
+}
+
+template <int D>
+int launch_decode(const FlashArgs& a, hipStream_t s) {
+  if (a.batch > 0x7fffffff / a.splits) return fail(TCX_INVALID_ARGUMENT, "attention grid is too large");
+  const dim3 grid(static_cast<unsigned>(a.batch * a.splits));
+  if (a.rows == 1) hipLaunchKernelGGL((flash_decode_kernel<D, 1>), grid, dim3(256), 0, s, a);
+  else if (a.rows == 2) hipLaunchKernelGGL((flash_decode_kernel<D, 2>), grid, dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((flash_decode_kernel<D, 4>), grid, dim3(256), 0, s, a);
+  return check(hipGetLastError(), "decode attention launch");
+}
+
+template <int D, bool kCausal>
+int launch_masked(const FlashArgs& a, hipStream_t s) {
+  if (a.mask_kind == TCX_MASK_BOOL) return launch_flash<D, 4, 32, kCausal, TCX_MASK_BOOL>(a, s);
+  return launch_flash<D, 4, 32, kCausal, TCX_MASK_ADDITIVE>(a, s);
+}
+
+template <int D>
+int launch_features(const FlashArgs& a, const FlashPlan& p, hipStream_t s) {
+  int rc;
+  if (p.decode) rc = launch_decode<D>(a, s);
+  else if (a.mask_kind != TCX_MASK_NONE) rc = a.causal ? launch_masked<D, true>(a, s) : launch_masked<D, false>(a, s);
+  else if (a.causal) rc = launch_flash<D, 4, 32, true, TCX_MASK_NONE>(a, s);
+  else if (p.waves == 1) rc = launch_flash<D, 1, 32, false, TCX_MASK_NONE>(a, s);
+  else if (D == 32 || p.waves == 4) rc = launch_flash<D, 4, 32, false, TCX_MASK_NONE>(a, s);
+  else rc = launch_flash<D >= 64 ? D : 64, 8, 64, false, TCX_MASK_NONE>(a, s);
+  if (rc != TCX_OK || a.splits == 1) return rc;
+  hipLaunchKernelGGL((flash_combine_kernel<D>), dim3(grid_for(a.batch * a.rows, 4, kStrideBlocks)), dim3(256), 0, s, a);
+  return check(hipGetLastError(), "attention combine launch");
 }
 
 }  // namespace
@@ -568,38 +986,91 @@ int tcx_hip_flash_attention_supported(int64_t features, int64_t value_features) 
   return features == value_features && (features == 32 || features == 64 || features == 128) ? 1 : 0;
 }
 
-int tcx_hip_flash_attention_f32(const float* q, const float* k, const float* v, float* out, int64_t batch,
-                                int64_t rows, int64_t cols, int64_t features, float scale, int causal,
-                                tcx_stream_t stream) {
+size_t tcx_hip_flash_attention_workspace_bytes(const tcx_hip_flash_attention_desc_t* desc) {
+  if (desc == nullptr || desc->batch <= 0 || desc->rows <= 0 || desc->cols < 0 ||
+      !tcx_hip_flash_attention_supported(desc->features, desc->features))
+    return 0;
+  return tcx::flash_plan(desc->batch, desc->rows, desc->cols, desc->features, desc->causal != 0, desc->mask_kind).bytes;
+}
+
+int tcx_hip_flash_attention_f32_ws(const float* q, const float* k, const float* v, float* out, const void* mask,
+                                   const tcx_hip_flash_attention_desc_t* desc, void* workspace,
+                                   size_t workspace_bytes, tcx_stream_t stream) {
   using namespace tcx;
-  if (batch < 0 || rows < 0 || cols < 0) return fail(TCX_INVALID_ARGUMENT, "attention extents must be non-negative");
-  if (!tcx_hip_flash_attention_supported(features, features))
+  if (desc == nullptr) return fail(TCX_INVALID_ARGUMENT, "attention descriptor is null");
+  const auto& d = *desc;
+  if (d.batch < 0 || d.rows < 0 || d.cols < 0) return fail(TCX_INVALID_ARGUMENT, "attention extents must be non-negative");
+  if (!tcx_hip_flash_attention_supported(d.features, d.features))
     return fail(TCX_INVALID_ARGUMENT, "fused attention supports 32, 64 or 128 features");
-  if (batch == 0 || rows == 0) return TCX_OK;
-  if (q == nullptr || out == nullptr || (cols > 0 && (k == nullptr || v == nullptr)))
+  if (d.mask_kind < TCX_MASK_NONE || d.mask_kind > TCX_MASK_ADDITIVE)
+    return fail(TCX_INVALID_ARGUMENT, "unknown attention mask kind");
+  if (d.batch == 0 || d.rows == 0) return TCX_OK;
+  const bool masked = d.mask_kind != TCX_MASK_NONE && d.cols > 0;
+  if (q == nullptr || out == nullptr || (d.cols > 0 && (k == nullptr || v == nullptr)) || (masked && mask == nullptr))
     return fail(TCX_INVALID_ARGUMENT, "attention buffers are null");
   for (const void* p : {static_cast<const void*>(q), static_cast<const void*>(k), static_cast<const void*>(v),
                         static_cast<const void*>(out)})
     if (p != nullptr && (reinterpret_cast<std::uintptr_t>(p) & 15U) != 0)
       return fail(TCX_INVALID_ARGUMENT, "fused attention buffers must be 16-byte aligned");
-  if (int rc = ready(); rc != TCX_OK) return rc;
-  const FlashArgs a{q, k, v, out, rows, cols, 0, 0, scale, causal != 0, 0, 0};
-  const auto s = static_cast<hipStream_t>(stream);
-  // Tile shapes measured on MI355X at 2048 x 2048. Unmasked: 8 waves and
-  // 64-key tiles for D = 128 and 64 (one block per CU at D = 128: 110 against
-  // 107 TFLOP/s with 4 waves and 32-key tiles), 4 waves and 32-key tiles for
-  // D = 32 (94 against 90). Causal: 4 waves and 32-key tiles (64 KB of LDS at
-  // D = 128), so that two blocks share each CU in the heavy/light order (89
-  // TFLOP/s at 16 x 2048 x 128 against 86 for a register-staged 4-wave kernel,
-  // 92 against 71 at 32 x 2048 x 64).
-  if (a.causal) {
-    if (features == 32) return launch_flash<32, 4, 32, true>(a, batch, s);
-    if (features == 64) return launch_flash<64, 4, 32, true>(a, batch, s);
-    return launch_flash<128, 4, 32, true>(a, batch, s);
+  FlashArgs a{};
+  if (masked) {
+    if (d.mask_rank < 0 || d.mask_rank > TCX_HIP_MAX_RANK)
+      return fail(TCX_INVALID_ARGUMENT, "attention mask rank must be in [0, 8]");
+    std::int64_t count = 1;
+    for (int i = 0; i < d.mask_rank; ++i) {
+      if (d.mask_shape[i] < 1) return fail(TCX_INVALID_ARGUMENT, "attention mask extents must be positive");
+      a.mask_shape[i] = d.mask_shape[i];
+      a.mask_stride[i] = d.mask_strides[i];
+      count *= d.mask_shape[i];
+    }
+    if (count != d.batch) return fail(TCX_INVALID_ARGUMENT, "attention mask axes must multiply to the batch");
+    a.mask = mask;
+    a.mask_kind = d.mask_kind;
+    a.mask_rank = d.mask_rank;
+    a.mask_row = d.mask_row_stride;
+    a.mask_col = d.mask_col_stride;
   }
-  if (features == 32) return launch_flash<32, 4, 32, false>(a, batch, s);
-  if (features == 64) return launch_flash<64, 8, 64, false>(a, batch, s);
-  return launch_flash<128, 8, 64, false>(a, batch, s);
+  if (int rc = ready(); rc != TCX_OK) return rc;
+  FlashPlan p = flash_plan(d.batch, d.rows, d.cols, d.features, d.causal != 0, a.mask_kind);
+  if (p.splits > 1 && (workspace == nullptr || workspace_bytes < p.bytes ||
+                       (reinterpret_cast<std::uintptr_t>(workspace) & 15U) != 0)) {
+    // No room for the splits' states: one block takes all keys.
+    p.split_keys *= p.splits;
+    p.splits = 1;
+  }
+  a.q = q;
+  a.k = k;
+  a.v = v;
+  a.out = out;
+  a.rows = d.rows;
+  a.cols = d.cols;
+  a.batch = d.batch;
+  a.scale = d.scale;
+  a.causal = d.causal != 0;
+  a.splits = p.splits;
+  a.split_keys = p.split_keys;
+  if (p.splits > 1) {
+    a.part = static_cast<float*>(workspace);
+    a.part_ml = a.part + p.splits * d.batch * d.rows * d.features;
+  }
+  const auto s = static_cast<hipStream_t>(stream);
+  if (d.features == 32) return launch_features<32>(a, p, s);
+  if (d.features == 64) return launch_features<64>(a, p, s);
+  return launch_features<128>(a, p, s);
+}
+
+int tcx_hip_flash_attention_f32(const float* q, const float* k, const float* v, float* out, int64_t batch,
+                                int64_t rows, int64_t cols, int64_t features, float scale, int causal,
+                                tcx_stream_t stream) {
+  tcx_hip_flash_attention_desc_t d{};
+  d.batch = batch;
+  d.rows = rows;
+  d.cols = cols;
+  d.features = features;
+  d.scale = scale;
+  d.causal = causal != 0;
+  d.mask_kind = TCX_MASK_NONE;
+  return tcx_hip_flash_attention_f32_ws(q, k, v, out, nullptr, &d, nullptr, 0, stream);
 }
 
 }  // extern "C"

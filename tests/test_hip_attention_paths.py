@@ -1,0 +1,202 @@
+"""The fused attention kernels against the oracle where their dispatch and
+their edges lie: few queries (split and unsplit keys), masks of every kind and
+broadcast, and special values under them. The bar is the reference test's,
+allclose(rtol=2e-4, atol=2e-5)."""
+
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle
+from conftest import require_gpu
+from hip_cases import assert_close
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def cx():
+    require_gpu()
+    import tensorcx
+    return tensorcx
+
+
+def f32(shape, seed):
+    return np.random.default_rng(seed).normal(size=shape).astype(np.float32)
+
+
+def check(cx, q, k, v, mask=None, causal=False):
+    args = [cx.tensor(t, device="hip") for t in (q, k, v)]
+    held = None if mask is None else cx.tensor(mask, device="hip")
+    got = cx.attention(*args, held, is_causal=causal).numpy()
+    with np.errstate(all="ignore"):
+        expected = oracle.attention(q, k, v, mask, causal)
+    assert_close(got, expected, 2e-4, 2e-5, f"{q.shape} x {k.shape} causal={causal}")
+
+
+def masks(kind, shape, rng):
+    """A mask of `shape` that hides about a third of the keys."""
+    if kind == "bool":
+        return rng.random(shape) > 0.3
+    mask = rng.normal(size=shape).astype(np.float32)
+    mask[rng.random(shape) < 0.2] = -np.inf
+    return mask
+
+
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("rows", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("cols", [1, 63, 64, 65, 127, 128, 255, 256, 257, 1000, 4099])
+def test_few_queries(cx, d, rows, cols):
+    """One to four queries stream the keys, over one block or (256 keys and
+    more for few batch matrices) several; five take the matrix kernel."""
+    check(cx, f32((2, 3, rows, d), 1), f32((2, 3, cols, d), 2), f32((2, 3, cols, d), 3))
+
+
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("kind", ["bool", "additive"])
+def test_few_queries_special_values(cx, d, kind):
+    rng = np.random.default_rng(d)
+    q, k, v = f32((3, 2, 2, d), 4), f32((3, 2, 700, d), 5), f32((3, 2, 700, d), 6)
+    mask = masks(kind, (3, 1, 2, 700), rng)
+    mask[1, 0, 0] = False if kind == "bool" else -np.inf   # a row with every key hidden
+    mask[2, 0, 1, :400] = False if kind == "bool" else -np.inf  # whole splits hidden
+    check(cx, q, k, v, mask)
+    q[0, 0, 1, 3] = np.nan
+    k[0, 1, 600] = np.inf
+    k[2, 0, 5] = -np.inf
+    v[1, 1, 650, 7] = np.inf     # shows as inf, or as NaN where its key is hidden
+    v[2, 1, 3, 0] = np.nan
+    check(cx, q, k, v, mask)
+    check(cx, q, k, v)
+
+
+def test_few_queries_many_batch_matrices(cx):
+    q, k, v = f32((1500, 4, 64), 7), f32((1500, 300, 64), 8), f32((1500, 300, 64), 9)
+    check(cx, q, k, v)
+
+
+# (batch matrices, rows, cols): one wave for up to 16 queries; four or eight
+# waves, whole or split, with splits that end in the middle of a key tile and
+# causal parts that are empty.
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("batch,rows,cols", [(3, 5, 4097), (4, 16, 1000), (4, 17, 1000), (2, 64, 2050), (3, 130, 1500),
+                                             (4, 512, 515), (70, 16, 200), (20, 129, 700), (256, 16, 33)])
+def test_split_keys(cx, d, causal, batch, rows, cols):
+    q, k, v = f32((batch, rows, d), 26), f32((batch, cols, d), 27), f32((batch, cols, d), 28)
+    check(cx, q, k, v, None, causal)
+
+
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+def test_split_keys_special_values(cx, d, causal):
+    q, k, v = f32((2, 90, d), 29), f32((2, 1300, d), 30), f32((2, 1300, d), 31)
+    q[0, 3, 7] = np.nan
+    k[0, 1200] = np.inf
+    k[0, 60] = -np.inf
+    v[1, 1250, 5] = np.nan   # in the last split, behind the causal mask of every query
+    v[1, 40, 6] = np.inf
+    check(cx, q, k, v, None, causal)
+    mask = masks("additive", (2, 90, 1300), np.random.default_rng(6))
+    mask[1, 5] = -np.inf
+    mask[0, 9, 100:] = -np.inf
+    check(cx, q, k, v, mask, causal)
+
+
+# Mask shapes against scores of (2, 3, rows, cols): shared, for each batch,
+# for each head, for each key, for each query, full.
+SHAPES = [lambda r, c: (r, c), lambda r, c: (2, 1, 1, c), lambda r, c: (1, 3, r, c), lambda r, c: (c,),
+          lambda r, c: (2, 3, r, 1), lambda r, c: (2, 3, r, c)]
+
+
+@pytest.mark.parametrize("kind", ["bool", "additive"])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d,rows,cols", [(32, 70, 31), (64, 64, 64), (64, 65, 33), (128, 130, 257), (128, 1, 300),
+                                         (64, 4, 129), (32, 17, 1)])
+def test_masks(cx, d, rows, cols, causal, kind):
+    rng = np.random.default_rng(rows * cols)
+    q, k, v = f32((2, 3, rows, d), 11), f32((2, 3, cols, d), 12), f32((2, 3, cols, d), 13)
+    for shape in SHAPES:
+        check(cx, q, k, v, masks(kind, shape(rows, cols), rng), causal)
+
+
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("kind", ["bool", "additive"])
+def test_mask_special_values(cx, d, kind):
+    rng = np.random.default_rng(3)
+    q, k, v = f32((2, 90, d), 14), f32((2, 110, d), 15), f32((2, 110, d), 16)
+    mask = masks(kind, (2, 90, 110), rng)
+    mask[0, 5] = False if kind == "bool" else -np.inf
+    if kind == "additive":
+        mask[1, 7, 3], mask[1, 8, 4] = np.nan, np.inf
+    q[0, 3, 7] = np.nan
+    k[0, 11] = np.inf
+    k[0, 12] = -np.inf
+    v[1, 80, 5] = np.nan
+    v[1, 109, 6] = np.inf
+    for causal in (False, True):
+        check(cx, q, k, v, mask, causal)
+
+
+def test_mask_over_nine_batch_axes(cx):
+    """Alternating broadcast axes fold to at most eight; nine take the
+    unfused route, whose own limit refuses them."""
+    lead = (2, 1, 2, 1, 2, 1, 2, 2)
+    q, k, v = f32(lead + (3, 32), 17), f32(lead + (5, 32), 18), f32(lead + (5, 32), 19)
+    rng = np.random.default_rng(4)
+    check(cx, q, k, v, masks("bool", (2, 1, 1, 1, 2, 1, 1, 2, 3, 5), rng))
+
+
+class Desc(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int64) for n in ("batch", "rows", "cols", "features")] + [
+        ("scale", ctypes.c_float), ("causal", ctypes.c_int32), ("mask_kind", ctypes.c_int32),
+        ("mask_rank", ctypes.c_int32), ("mask_shape", ctypes.c_int64 * 8), ("mask_strides", ctypes.c_int64 * 8),
+        ("mask_row_stride", ctypes.c_int64), ("mask_col_stride", ctypes.c_int64)]
+
+
+def fused(capi, q, k, v, mask, desc):
+    """The C entry on device copies, without a workspace; the mask starts one
+    element past a 16-byte boundary."""
+    held = [capi.DeviceArray.from_numpy(t) for t in (q, k, v)]
+    store = capi.DeviceArray.from_numpy(np.concatenate([np.zeros(1, mask.dtype), mask.reshape(-1)]))
+    out = capi.DeviceArray(q.shape)
+    capi.check(capi.lib().tcx_hip_flash_attention_f32_ws(
+        *(ctypes.c_void_p(t.ptr) for t in held), ctypes.c_void_p(out.ptr),
+        ctypes.c_void_p(store.ptr + mask.itemsize), ctypes.byref(desc), None, ctypes.c_size_t(0),
+        ctypes.c_void_p(capi.stream())), "attention")
+    capi.synchronize()
+    return out.numpy()
+
+
+@pytest.mark.parametrize("kind", ["bool", "additive"])
+@pytest.mark.parametrize("rows", [2, 40])
+def test_mask_at_an_odd_address(cx, rows, kind):
+    import tensorcx_hip_capi as capi
+    q, k, v = f32((2, rows, 64), 20), f32((2, 300, 64), 21), f32((2, 300, 64), 22)
+    mask = masks(kind, (2, rows, 300), np.random.default_rng(5))
+    desc = Desc(batch=2, rows=rows, cols=300, features=64, scale=0.125, mask_kind=1 if kind == "bool" else 2,
+                mask_rank=1, mask_row_stride=300, mask_col_stride=1)
+    desc.mask_shape[0], desc.mask_strides[0] = 2, rows * 300
+    assert_close(fused(capi, q, k, v, mask, desc), oracle.attention(q, k, v, mask), 2e-4, 2e-5, "odd address")
+    desc.mask_shape[0] = 3
+    with pytest.raises(capi.HipError):
+        fused(capi, q, k, v, mask, desc)
+
+
+@pytest.mark.parametrize("rows", [1, 3])
+def test_without_a_workspace(cx, rows):
+    """The C entry without a workspace, or with one too small, keeps the keys
+    of a matrix in one block."""
+    import tensorcx_hip_capi as capi
+    lib = capi.lib()
+    q, k, v = f32((2, rows, 64), 23), f32((2, 900, 64), 24), f32((2, 900, 64), 25)
+    dq, dk, dv = (capi.DeviceArray.from_numpy(t) for t in (q, k, v))
+    out = capi.DeviceArray(q.shape)
+    capi.flash_attention(dq.ptr, dk.ptr, dv.ptr, out.ptr, 2, rows, 900, 64, 0.125, False)
+    capi.synchronize()
+    assert_close(out.numpy(), oracle.attention(q, k, v), 2e-4, 2e-5, "no workspace")
+    assert lib.tcx_hip_flash_attention_f32_ws(None, None, None, None, None, None, None, ctypes.c_size_t(0),
+                                              None) == capi.TCX_INVALID_ARGUMENT
