@@ -396,6 +396,16 @@ int tcx_hip_clip(int dtype, const void* x, const void* lo, const void* hi, void*
  * index; sorted == 0 lists the chosen k in index order. */
 int tcx_hip_topk(int dtype, const void* x, void* values, int32_t* indices, int64_t outer, int64_t reduce,
                  int64_t inner, int64_t k, int largest, int sorted, tcx_stream_t stream);
+/* Workspace bytes that tcx_hip_topk_ws can use: > 0 for fewer rows than the
+ * GPU has CUs, of at least 16384 elements, and k <= 256, whose parts are then
+ * selected by several blocks a row; 0 otherwise. */
+size_t tcx_hip_topk_workspace_bytes(int64_t outer, int64_t reduce, int64_t inner, int64_t k);
+/* tcx_hip_topk with that workspace (8-byte aligned; NULL or fewer bytes than
+ * the query: one block a row). Same results, bit for bit; the workspace must
+ * stay allocated until the stream has run the call. */
+int tcx_hip_topk_ws(int dtype, const void* x, void* values, int32_t* indices, int64_t outer, int64_t reduce,
+                    int64_t inner, int64_t k, int largest, int sorted, void* workspace, size_t workspace_bytes,
+                    tcx_stream_t stream);
 
 /* ---- inference primitives (replace reference backends/cuda/kernels/
  * inference.cu; semantics of backends/cpu/cpu_inference.cpp) ---- */

@@ -754,9 +754,19 @@ std::pair<Tensor, Tensor> topk(const OpDesc& op, const Tensor& x, Stream& s) {
     if (a < axis) outer *= x.shape[static_cast<std::size_t>(a)];
     if (a > axis) inner *= x.shape[static_cast<std::size_t>(a)];
   }
-  ok_or_throw(tcx_hip_topk(tcx_dtype(x.dtype), xp, out_ptr(values), static_cast<int32_t*>(out_ptr(indices)), outer,
-                           reduce, inner, op.k, op.largest ? 1 : 0, op.sorted ? 1 : 0, s),
+  // Few long rows are selected in parts, whose choices go to a workspace held
+  // until the stream has finished (a block a row, when that allocation fails).
+  const std::size_t ws = tcx_hip_topk_workspace_bytes(outer, reduce, inner, op.k);
+  std::shared_ptr<HipBuffer> workspace;
+  if (ws) {
+    auto created = HipBuffer::create(ws);
+    if (created) workspace = created.move_value();
+  }
+  ok_or_throw(tcx_hip_topk_ws(tcx_dtype(x.dtype), xp, out_ptr(values), static_cast<int32_t*>(out_ptr(indices)), outer,
+                              reduce, inner, op.k, op.largest ? 1 : 0, op.sorted ? 1 : 0,
+                              workspace ? workspace->data() : nullptr, workspace ? ws : 0, s),
               "HIP topk");
+  if (workspace) ok_or_throw(tcx_hip_stream_synchronize(s), "HIP topk");
   return {std::move(values), std::move(indices)};
 }
 

@@ -24,9 +24,12 @@
 //
 // What bounds it: the row is read once from HBM and once more from L2 (the
 // selection reads nothing else), so a row costs two passes at the rate that
-// one CU draws, and rows fewer than the CUs leave the rest idle: 29.5 us for 32
-// rows of 128256 with k = 50, 100 us for 1024 of 50257 with k = 40. One pass
-// over the row for each of the k elements, as before, took 11.40 and 5.84 ms.
+// one CU draws: 100 us for 1024 rows of 50257 with k = 40. With a workspace,
+// fewer rows than CUs are cut into parts (launch_topk_parts): 21 us for 32 rows
+// of 128256 with k = 50. One pass over the row for each of the k elements, as
+// before, took 5.84 and 11.40 ms.
+
+#include <algorithm>
 
 #include "common.hpp"
 
@@ -41,6 +44,20 @@ struct TopkArgs {
   std::int32_t* indices;
   std::int64_t rows, reduce, inner, k;
   int largest, sorted;
+  // Rows in parts of part_len elements, where they are fewer than the CUs: the
+  // places of the k first of each part go to places [rows, parts, k].
+  std::int64_t parts, part_len;
+  std::uint64_t* places;
+};
+
+// The elements one block selects from: n of a row from element `first` on, and
+// where its choice goes (the row's outputs, or the places of a part).
+struct TopkSpan {
+  const std::uint32_t* x;
+  std::int64_t first, n, k;
+  std::uint32_t* values;
+  std::int32_t* indices;
+  std::uint64_t* places;
 };
 
 // Larger keys come first; equal keys are ties.
@@ -61,8 +78,9 @@ __device__ __forceinline__ std::int32_t index_of(std::uint64_t place) {
 
 // f(word, index) for this thread's share of a row. Contiguous rows of at least
 // 4 kThreads elements (so that every thread has some) are read 16 bytes at a
-// time, eight loads in flight, whatever the row's alignment: the elements in
-// front of the first 16-byte boundary and after the last are single words.
+// time, four or eight loads in flight, whatever the row's alignment: the
+// elements in front of the first 16-byte boundary and after the last are single
+// words.
 template <int kThreads, typename F>
 __device__ __forceinline__ void scan_row(const std::uint32_t* __restrict__ x, std::int64_t n, std::int64_t inner, F&& f) {
   using word4 = std::uint32_t __attribute__((ext_vector_type(4)));
@@ -86,7 +104,15 @@ __device__ __forceinline__ void scan_row(const std::uint32_t* __restrict__ x, st
 #pragma unroll
       for (int u = 0; u < 8; ++u) four(w[u], q + u * kThreads);
     }
-    for (; q < quads; q += kThreads) four(body[q], q);
+    // What is left, four at a time too: loads past the end repeat the last.
+    for (; q < quads; q += 4 * kThreads) {
+      word4 w[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) w[u] = body[min(q + u * kThreads, quads - 1)];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (q + u * kThreads < quads) four(w[u], q + u * kThreads);
+    }
     const std::int64_t tail = head + 4 * quads;
     if (t < head) f(x[t], t);
     if (tail + t < n) f(x[tail + t], tail + t);
@@ -129,65 +155,78 @@ __device__ __forceinline__ std::uint32_t wave_nth_largest(std::uint32_t v, int r
   return static_cast<std::uint32_t>(__shfl(static_cast<int>(v), rank, kWave));
 }
 
-// visit(c, before) in one lane for each c < count, with before the number of
-// c' < count for which precedes(c', c): lanes in groups of a power of two
-// share the counting of one c. Called by the whole block; no barriers.
-template <int kThreads, typename P, typename V>
-__device__ __forceinline__ void rank_each(int count, P&& precedes, V&& visit) {
+// visit(c, above) in one lane for each c < count, with above the number of
+// c' < count whose value(c') is larger: lanes in groups of a power of two share
+// the counting of one c, eight LDS reads in flight each (one at a time, the
+// reads' latency made 750 candidates cost 30 us). Called by the whole block; no
+// barriers.
+template <int kThreads, typename F, typename V>
+__device__ __forceinline__ void rank_each(int count, F&& value, V&& visit) {
   int group = kWave;
   while (group > 1 && count * group > kThreads) group >>= 1;
   const int g = threadIdx.x & (group - 1);
   const int step = kThreads / group;
   for (int base = 0; base < count; base += step) {
     const int c = base + threadIdx.x / group;
-    const int self = c < count ? c : count - 1;
-    int before = 0;
-    for (int j = g; j < count; j += group) before += precedes(j, self) ? 1 : 0;
-    for (int offset = group / 2; offset > 0; offset >>= 1) before += __shfl_xor(before, offset, kWave);
-    if (g == 0 && c < count) visit(c, before);
+    const auto mine = value(c < count ? c : count - 1);
+    int above = 0, j = g;
+    for (; j + 7 * group < count; j += 8 * group) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) above += value(j + u * group) > mine ? 1 : 0;
+    }
+    for (; j < count; j += group) above += value(j) > mine ? 1 : 0;
+    for (int offset = group / 2; offset > 0; offset >>= 1) above += __shfl_xor(above, offset, kWave);
+    if (g == 0 && c < count) visit(c, above);
   }
 }
 
-// The k first of the `count` candidates in LDS, written out.
+// The k candidates s.chosen, written out in index order.
 template <int kThreads>
-__device__ __forceinline__ void emit_candidates(TopkShared<kThreads>& s, const TopkArgs& a, int count,
-                                                std::uint32_t* values, std::int32_t* indices) {
-  const int k = static_cast<int>(a.k);  // <= count
-  const auto ahead = [&](int j, int c) { return s.place[j] > s.place[c]; };
-  if (a.sorted) {
-    rank_each<kThreads>(count, ahead, [&](int c, int before) {
-      if (before >= k) return;
-      values[before * a.inner] = s.word[c];
-      indices[before * a.inner] = index_of(s.place[c]);
-    });
-    return;
-  }
-  rank_each<kThreads>(count, ahead, [&](int c, int before) {
-    if (before < k) s.chosen[before] = c;
-  });
-  __syncthreads();
+__device__ __forceinline__ void emit_by_index(TopkShared<kThreads>& s, const TopkArgs& a, const TopkSpan& w) {
   rank_each<kThreads>(
-      k,
-      [&](int j, int c) { return index_of(s.place[s.chosen[j]]) < index_of(s.place[s.chosen[c]]); },
+      static_cast<int>(w.k),
+      [&](int c) { return ~index_of(s.place[s.chosen[c]]); },  // lower indices above
       [&](int c, int before) {
         const int at = s.chosen[c];
-        values[before * a.inner] = s.word[at];
-        indices[before * a.inner] = index_of(s.place[at]);
+        w.values[before * a.inner] = s.word[at];
+        w.indices[before * a.inner] = index_of(s.place[at]);
       });
+}
+
+// The k first of the `count` candidates in LDS, written out.
+template <int kThreads, bool kParts>
+__device__ __forceinline__ void emit_candidates(TopkShared<kThreads>& s, const TopkArgs& a, const TopkSpan& w, int count) {
+  const int k = static_cast<int>(w.k);  // <= count
+  rank_each<kThreads>(
+      count, [&](int c) { return s.place[c]; },
+      [&](int c, int before) {
+        if (before >= k) return;
+        if constexpr (kParts) {
+          w.places[before] = s.place[c];
+        } else if (a.sorted) {
+          w.values[before * a.inner] = s.word[c];
+          w.indices[before * a.inner] = index_of(s.place[c]);
+        } else {
+          s.chosen[before] = c;
+        }
+      });
+  if (kParts || a.sorted) return;
+  __syncthreads();
+  emit_by_index<kThreads>(s, a, w);
 }
 
 // The key of the k-th element and how many of the elements equal to it are
 // among the k (s.need): 8 bits a pass from the top.
 template <int kThreads, bool kFp>
-__device__ std::uint32_t radix_kth(TopkShared<kThreads>& s, const TopkArgs& a, const std::uint32_t* __restrict__ x) {
+__device__ std::uint32_t radix_kth(TopkShared<kThreads>& s, const TopkArgs& a, const TopkSpan& span) {
   const bool largest = a.largest != 0;
   const int t = threadIdx.x;
   std::uint32_t prefix = 0, mask = 0;
-  if (t == 0) s.need = static_cast<std::uint32_t>(a.k);
+  if (t == 0) s.need = static_cast<std::uint32_t>(span.k);
   for (int shift = 24; shift >= 0; shift -= 8) {
     for (int b = t; b < 256; b += kThreads) s.histogram[b] = 0;
     __syncthreads();
-    scan_row<kThreads>(x, a.reduce, a.inner, [&](std::uint32_t w, std::int64_t) {
+    scan_row<kThreads>(span.x, span.n, a.inner, [&](std::uint32_t w, std::int64_t) {
       const std::uint32_t key = topk_key<kFp>(w, largest);
       if ((key & mask) == prefix) atomicAdd(&s.histogram[(key >> shift) & 255U], 1U);
     });
@@ -266,22 +305,21 @@ __device__ void sort_output(const TopkArgs& a, std::uint32_t* values, std::int32
 
 // Radix selection, then the chosen elements in index order: to the output, or
 // to LDS where they are still to be put in order and fit.
-template <int kThreads, bool kFp>
-__device__ void select_row(TopkShared<kThreads>& s, const TopkArgs& a, const std::uint32_t* __restrict__ x,
-                           std::uint32_t* values, std::int32_t* indices) {
+template <int kThreads, bool kFp, bool kParts>
+__device__ void select_span(TopkShared<kThreads>& s, const TopkArgs& a, const TopkSpan& span) {
   constexpr int kWaves = kThreads / kWave;
   const bool largest = a.largest != 0;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const std::uint32_t kth = radix_kth<kThreads, kFp>(s, a, x);
-  const std::int64_t ties = s.need, n = a.reduce;
-  const bool in_lds = a.sorted && a.k <= kCandidates;
+  const std::uint32_t kth = radix_kth<kThreads, kFp>(s, a, span);
+  const std::int64_t ties = s.need, n = span.n;
+  const bool in_lds = kParts || (a.sorted && span.k <= kCandidates);
   std::int64_t greater_run = 0, equal_run = 0;
-  for (std::int64_t start = 0; start < n && greater_run + min(equal_run, ties) < a.k; start += kThreads) {
+  for (std::int64_t start = 0; start < n && greater_run + min(equal_run, ties) < span.k; start += kThreads) {
     const std::int64_t i = start + t;
     std::uint32_t w = 0;
     bool greater = false, equal = false;
     if (i < n) {
-      w = x[i * a.inner];
+      w = span.x[i * a.inner];
       const std::uint32_t key = topk_key<kFp>(w, largest);
       greater = key > kth;
       equal = key == kth;
@@ -307,51 +345,61 @@ __device__ void select_row(TopkShared<kThreads>& s, const TopkArgs& a, const std
     if (greater || (equal && equal_before < ties)) {
       const std::int64_t at = greater_before + min(equal_before, ties);
       if (in_lds) {
-        s.place[at] = place_of(topk_key<kFp>(w, largest), i);
+        s.place[at] = place_of(topk_key<kFp>(w, largest), span.first + i);
         s.word[at] = w;
       } else {
-        values[at * a.inner] = w;
-        indices[at * a.inner] = static_cast<std::int32_t>(i);
+        span.values[at * a.inner] = w;
+        span.indices[at * a.inner] = static_cast<std::int32_t>(i);
       }
     }
   }
-  if (!a.sorted) return;
+  if (!in_lds && !a.sorted) return;
   __syncthreads();
-  if (in_lds) emit_candidates<kThreads>(s, a, static_cast<int>(a.k), values, indices);
-  else sort_output<kThreads, kFp>(a, values, indices);
+  if (in_lds) emit_candidates<kThreads, kParts>(s, a, span, static_cast<int>(span.k));
+  else sort_output<kThreads, kFp>(a, span.values, span.indices);
 }
 
-template <int kThreads, bool kFp>
+template <int kThreads, bool kFp, bool kParts>
 __global__ __launch_bounds__(kThreads) void topk_kernel(TopkArgs a) {
   constexpr int kWaves = kThreads / kWave;
   __shared__ TopkShared<kThreads> s;
   const bool largest = a.largest != 0;
   const int t = threadIdx.x;
-  for (std::int64_t row = blockIdx.x; row < a.rows; row += gridDim.x) {
+  const std::int64_t parts = kParts ? a.parts : 1, items = a.rows * parts;
+  for (std::int64_t item = blockIdx.x; item < items; item += gridDim.x) {
+    const std::int64_t row = item / parts, part = item % parts;
     const std::int64_t outer = row / a.inner, column = row % a.inner;
-    const std::uint32_t* __restrict__ x = a.x + outer * a.reduce * a.inner + column;
-    std::uint32_t* const values = a.values + outer * a.k * a.inner + column;
-    std::int32_t* const indices = a.indices + outer * a.k * a.inner + column;
-    __syncthreads();  // the previous row is done with s
-    if (a.reduce <= kThreads) {
-      if (t < a.reduce) {
-        const std::uint32_t w = x[t * a.inner];
-        s.place[t] = place_of(topk_key<kFp>(w, largest), t);
+    TopkSpan span;
+    span.first = kParts ? part * a.part_len : 0;
+    span.n = kParts ? min(a.part_len, a.reduce - span.first) : a.reduce;
+    span.k = kParts ? min(a.k, span.n) : a.k;
+    span.x = a.x + (outer * a.reduce + span.first) * a.inner + column;
+    span.values = a.values + outer * a.k * a.inner + column;
+    span.indices = a.indices + outer * a.k * a.inner + column;
+    span.places = kParts ? a.places + item * a.k : nullptr;
+    __syncthreads();  // the previous item is done with s
+    if constexpr (kParts) {  // a short last part: places below every element's
+      for (std::int64_t j = span.k + t; j < a.k; j += kThreads) span.places[j] = 0;
+    }
+    if (span.n <= kThreads) {
+      if (t < span.n) {
+        const std::uint32_t w = span.x[t * a.inner];
+        s.place[t] = place_of(topk_key<kFp>(w, largest), span.first + t);
         s.word[t] = w;
       }
       __syncthreads();
-      emit_candidates<kThreads>(s, a, static_cast<int>(a.reduce), values, indices);
+      emit_candidates<kThreads, kParts>(s, a, span, static_cast<int>(span.n));
       continue;
     }
-    if (a.k > kThreads / 4) {
-      select_row<kThreads, kFp>(s, a, x, values, indices);
+    if (span.k > kThreads / 4) {
+      select_span<kThreads, kFp, kParts>(s, a, span);
       continue;
     }
     std::uint32_t best = 0;
-    scan_row<kThreads>(x, a.reduce, a.inner, [&](std::uint32_t w, std::int64_t) {
+    scan_row<kThreads>(span.x, span.n, a.inner, [&](std::uint32_t w, std::int64_t) {
       best = max(best, topk_key<kFp>(w, largest));
     });
-    const int per_wave = (static_cast<int>(a.k) + kWaves - 1) / kWaves;  // <= 16
+    const int per_wave = (static_cast<int>(span.k) + kWaves - 1) / kWaves;  // <= 16
     const std::uint32_t bound = wave_nth_largest(best, per_wave - 1);
     if ((t & 63) == 0) s.wave_a[t >> 6] = bound;
     if (t == 0) s.count = 0;
@@ -359,19 +407,67 @@ __global__ __launch_bounds__(kThreads) void topk_kernel(TopkArgs a) {
     std::uint32_t least = s.wave_a[0];
 #pragma unroll
     for (int v = 1; v < kWaves; ++v) least = min(least, s.wave_a[v]);
-    scan_row<kThreads>(x, a.reduce, a.inner, [&](std::uint32_t w, std::int64_t i) {
+    scan_row<kThreads>(span.x, span.n, a.inner, [&](std::uint32_t w, std::int64_t i) {
       const std::uint32_t key = topk_key<kFp>(w, largest);
       if (key < least) return;
       const std::uint32_t at = atomicAdd(&s.count, 1U);
       if (at < kCandidates) {
-        s.place[at] = place_of(key, i);
+        s.place[at] = place_of(key, span.first + i);
         s.word[at] = w;
       }
     });
     __syncthreads();
-    if (s.count <= kCandidates) emit_candidates<kThreads>(s, a, static_cast<int>(s.count), values, indices);
-    else select_row<kThreads, kFp>(s, a, x, values, indices);
+    if (s.count <= kCandidates) emit_candidates<kThreads, kParts>(s, a, span, static_cast<int>(s.count));
+    else select_span<kThreads, kFp, kParts>(s, a, span);
   }
+}
+
+// The k first of the parts' choices (parts * k <= kCandidates), a block a row.
+// Each part's places come in order, so the place of an element among all of
+// them is its rank in its own part and a binary search in each other one.
+__global__ __launch_bounds__(1024) void topk_join_kernel(TopkArgs a) {
+  __shared__ TopkShared<1024> s;
+  const int t = threadIdx.x, parts = static_cast<int>(a.parts), k = static_cast<int>(a.k), count = parts * k;
+  const std::int64_t row = blockIdx.x, outer = row / a.inner, column = row % a.inner;
+  TopkSpan span{};
+  span.x = a.x + outer * a.reduce * a.inner + column;
+  span.k = a.k;
+  span.values = a.values + outer * a.k * a.inner + column;
+  span.indices = a.indices + outer * a.k * a.inner + column;
+  std::uint64_t mine = 0;
+  if (t < count) {
+    mine = a.places[row * count + t];
+    s.place[t] = mine;
+    s.word[t] = mine != 0 ? span.x[index_of(mine) * a.inner] : 0U;
+  }
+  __syncthreads();
+  if (t < count && mine != 0) {
+    const int own = t / k;
+    int before = t % k;
+#pragma unroll 4
+    for (int part = 0; part < parts; ++part) {
+      const std::uint64_t* const other = s.place + part * k;
+      int above = 0;  // of other[0 .. k), those larger than mine
+      for (int length = k; length > 0;) {
+        const int half = length >> 1;
+        const bool larger = other[above + half] > mine;
+        above += larger ? half + 1 : 0;
+        length = larger ? length - half - 1 : half;
+      }
+      before += part != own ? above : 0;
+    }
+    if (before < k) {
+      if (a.sorted) {
+        span.values[before * a.inner] = s.word[t];
+        span.indices[before * a.inner] = index_of(mine);
+      } else {
+        s.chosen[before] = t;
+      }
+    }
+  }
+  if (a.sorted) return;
+  __syncthreads();
+  emit_by_index<1024>(s, a, span);
 }
 
 // Short rows and few of them asked for: one wave a row, the row in registers
@@ -433,8 +529,24 @@ void launch_topk_wave(const TopkArgs& a, hipStream_t s) {
 template <int kThreads, bool kFp>
 void launch_topk(const TopkArgs& a, hipStream_t s) {
   const std::int64_t cap = kMaxLaunchWorkItems / kThreads;
-  hipLaunchKernelGGL((topk_kernel<kThreads, kFp>), dim3(static_cast<unsigned>(a.rows < cap ? a.rows : cap)),
+  hipLaunchKernelGGL((topk_kernel<kThreads, kFp, false>), dim3(static_cast<unsigned>(a.rows < cap ? a.rows : cap)),
                      dim3(kThreads), 0, s, a);
+}
+
+// The number of parts to cut a row into (1: whole). Fewer rows than the 256 CUs
+// and at least two parts of 8192 elements; all parts' choices are joined in LDS.
+std::int64_t topk_parts(std::int64_t rows, std::int64_t reduce, std::int64_t k) {
+  const std::int64_t parts = std::min({256 / rows, reduce / 8192, kCandidates / std::max<std::int64_t>(k, 1)});
+  return k <= 256 && parts >= 2 ? parts : 1;
+}
+
+// The parts, each a block, and their join: 32 rows of 128256 with k = 50 in 15 +
+// 6 us against 29.5 us for a block a row, whose two passes are bound by what one
+// CU reads; one row of 128256 20 against 29 us.
+template <bool kFp>
+void launch_topk_parts(const TopkArgs& a, hipStream_t s) {
+  hipLaunchKernelGGL((topk_kernel<1024, kFp, true>), dim3(static_cast<unsigned>(a.rows * a.parts)), dim3(1024), 0, s, a);
+  hipLaunchKernelGGL(topk_join_kernel, dim3(static_cast<unsigned>(a.rows)), dim3(1024), 0, s, a);
 }
 
 // A wave a row up to kWaveRow elements and k = kWaveK: with k = 1, 14.7 us for
@@ -459,8 +571,17 @@ void launch_topk_rows(const TopkArgs& a, hipStream_t s) {
 
 extern "C" {
 
-int tcx_hip_topk(int dtype, const void* x, void* values, int32_t* indices, int64_t outer, int64_t reduce,
-                 int64_t inner, int64_t k, int largest, int sorted, tcx_stream_t stream) {
+size_t tcx_hip_topk_workspace_bytes(int64_t outer, int64_t reduce, int64_t inner, int64_t k) {
+  if (outer <= 0 || inner <= 0 || outer > 256 || inner > 256 || reduce > 0x7fffffff || k <= 0 || k > reduce) return 0;
+  const std::int64_t rows = outer * inner;
+  if (rows > 256) return 0;
+  const std::int64_t parts = tcx::topk_parts(rows, reduce, k);
+  return parts > 1 ? static_cast<size_t>(rows * parts * k) * sizeof(std::uint64_t) : 0;
+}
+
+int tcx_hip_topk_ws(int dtype, const void* x, void* values, int32_t* indices, int64_t outer, int64_t reduce,
+                    int64_t inner, int64_t k, int largest, int sorted, void* workspace, size_t workspace_bytes,
+                    tcx_stream_t stream) {
   using namespace tcx;
   if (dtype != TCX_FLOAT32 && dtype != TCX_INT32) return fail(TCX_INVALID_ARGUMENT, "math operations require float32 or int32");
   if (outer < 0 || reduce < 0 || inner < 0) return fail(TCX_INVALID_ARGUMENT, "topk extents must be non-negative");
@@ -472,11 +593,27 @@ int tcx_hip_topk(int dtype, const void* x, void* values, int32_t* indices, int64
   if (x == nullptr || values == nullptr || indices == nullptr) return fail(TCX_INVALID_ARGUMENT, "topk buffers are null");
   if (int rc = ready(); rc != TCX_OK) return rc;
   const auto s = static_cast<hipStream_t>(stream);
-  const TopkArgs a{static_cast<const std::uint32_t*>(x), static_cast<std::uint32_t*>(values), indices, rows, reduce,
-                   inner, k, largest, sorted};
+  TopkArgs a{static_cast<const std::uint32_t*>(x), static_cast<std::uint32_t*>(values), indices, rows, reduce,
+             inner, k, largest, sorted, 1, reduce, nullptr};
+  const size_t needed = tcx_hip_topk_workspace_bytes(outer, reduce, inner, k);
+  if (needed != 0 && workspace != nullptr && workspace_bytes >= needed &&
+      (reinterpret_cast<std::uintptr_t>(workspace) & 7U) == 0) {
+    const std::int64_t parts = topk_parts(rows, reduce, k);
+    a.part_len = ((reduce + parts - 1) / parts + 3) / 4 * 4;
+    a.parts = (reduce + a.part_len - 1) / a.part_len;
+    a.places = static_cast<std::uint64_t*>(workspace);
+    if (dtype == TCX_FLOAT32) launch_topk_parts<true>(a, s);
+    else launch_topk_parts<false>(a, s);
+    return check(hipGetLastError(), "topk launch");
+  }
   if (dtype == TCX_FLOAT32) launch_topk_rows<true>(a, s);
   else launch_topk_rows<false>(a, s);
   return check(hipGetLastError(), "topk launch");
+}
+
+int tcx_hip_topk(int dtype, const void* x, void* values, int32_t* indices, int64_t outer, int64_t reduce,
+                 int64_t inner, int64_t k, int largest, int sorted, tcx_stream_t stream) {
+  return tcx_hip_topk_ws(dtype, x, values, indices, outer, reduce, inner, k, largest, sorted, nullptr, 0, stream);
 }
 
 }  // extern "C"

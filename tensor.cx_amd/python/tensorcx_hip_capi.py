@@ -41,7 +41,7 @@ EXPORTS = [
     "tcx_hip_rownorm_workspace_bytes", "tcx_hip_softmax_f32_ws", "tcx_hip_rmsnorm_f32_ws",
     "tcx_hip_layernorm_f32_ws",
     "tcx_hip_bias_act_f32", "tcx_hip_unary_f32", "tcx_hip_binary", "tcx_hip_fill",
-    "tcx_hip_math_unary", "tcx_hip_clip", "tcx_hip_topk", "tcx_hip_embedding_f32",
+    "tcx_hip_math_unary", "tcx_hip_clip", "tcx_hip_topk", "tcx_hip_topk_workspace_bytes", "tcx_hip_topk_ws", "tcx_hip_embedding_f32",
     "tcx_hip_attention_softmax_f32", "tcx_hip_flash_attention_supported", "tcx_hip_flash_attention_f32",
     "tcx_hip_flash_attention_workspace_bytes", "tcx_hip_flash_attention_f32_ws",
     "tcx_hip_gather_strided", "tcx_hip_copy_blocks", "tcx_hip_cast", "tcx_hip_scalar_op", "tcx_hip_predicate",

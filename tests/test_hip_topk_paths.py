@@ -64,6 +64,18 @@ def test_row_lengths_and_counts(cx, n, ks, kind):
                 check(cx, x, -1, k, largest, sort)
 
 
+@pytest.mark.parametrize("kind", ["normal", "special", "ties", "equal", "int32"])
+@pytest.mark.parametrize("shape,axis", [((1, 16384), -1), ((3, 16389), -1), ((2, 65541), -1), ((128, 16385), -1),
+                                        ((129, 16385), -1), ((16400, 5), 0)])
+def test_rows_in_parts(cx, shape, axis, kind):
+    """Few long rows are cut into parts (of lengths that leave a short last
+    one); 129 rows and k = 257 are not."""
+    x = values_of(kind, shape, np.random.default_rng(shape[0]))
+    for k in (1, 50, 256, 257):
+        check(cx, x, axis, k, True, True)
+    check(cx, x, axis, 50, False, False)
+
+
 @pytest.mark.parametrize("kind", ["special", "ties"])
 def test_other_axes(cx, kind):
     rng = np.random.default_rng(5)
