@@ -84,11 +84,14 @@ int tcx_hip_allocate(size_t bytes, void** ptr, tcx_hip_pool_t** owner);
 /* Returns a block from tcx_hip_allocate: to its pool's cache when that pool
  * is still active and has room, else hipFree. Never fails the caller. */
 void tcx_hip_release(void* ptr, size_t bytes, tcx_hip_pool_t* owner);
-/* tcx_hip_release that never caches the block: storage that was exposed to
- * another framework (DLPack export, copies included) may still be read by
- * work on streams this library cannot see, so it goes straight back to
- * hipFree, which waits for the device (the reference's exported-buffer rule,
- * bindings/dlpack.cpp:204-206 and cuda_buffer.h:35). */
+/* tcx_hip_release that never returns the block to its pool's cache: storage
+ * that was exposed to another framework (DLPack export, copies included) may
+ * still be read by work on streams this library cannot see (the reference's
+ * exported-buffer rule, bindings/dlpack.cpp:204-206 and cuda_buffer.h:35). The
+ * block is freed, which waits for the device, or kept (at most 16 blocks and
+ * 512 MiB in all) for an allocation of the same size that waits for the device
+ * first; blocks kept are freed when device memory runs out and when any pool
+ * is trimmed or left. */
 void tcx_hip_release_uncached(void* ptr, size_t bytes, tcx_hip_pool_t* owner);
 
 /* Checks memory handed over by another framework before a tensor borrows it

@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <iterator>
 #include <mutex>
 #include <new>
 #include <string>
@@ -71,9 +72,123 @@ struct tcx_hip_pool {
 namespace {
 thread_local tcx_hip_pool* active_pool = nullptr;
 
+// Exported storage after its release. Another framework may still read it by
+// work that is queued on streams this library cannot see, so a block is handed
+// out again only after hipDeviceSynchronize, which hipFree would have made its
+// releaser wait for as well. Mapping and unmapping a result of 2 MiB and more
+// for each exchange cost 40 to 280 us of a call. Exact sizes, the newest first;
+// at most kRetiredBlocks blocks and kRetiredBytes bytes, the oldest freed for a
+// new one; all freed when device memory runs out and when a pool is trimmed or
+// left. One list for all threads: a block belongs to no stream once the device
+// has been waited for.
+struct Retired {
+  void* ptr;
+  size_t bytes;
+  int device;
+  std::uint64_t number;  // of its release
+  bool idle;             // the device has been waited for since
+};
+constexpr size_t kRetiredBlocks = 16, kRetiredBytes = size_t{512} << 20;
+std::mutex retired_mutex;
+std::uint64_t releases = 0;  // under retired_mutex
+
+// Never destroyed: at process end the runtime that would free the blocks may
+// be gone already.
+std::vector<Retired>& retired() {
+  static auto* blocks = new std::vector<Retired>;
+  return *blocks;
+}
+
+void free_retired() {
+  std::vector<Retired> blocks;
+  {
+    std::lock_guard lock(retired_mutex);
+    blocks.swap(retired());
+  }
+  for (const Retired& b : blocks) (void)hipFree(b.ptr);
+}
+
+// Takes a released block over; false where it has to be freed instead.
+bool retire(void* ptr, size_t bytes) noexcept {
+  int device = 0;
+  hipPointerAttribute_t attributes{};
+  if (bytes > kRetiredBytes / 2 || hipGetDevice(&device) != hipSuccess ||
+      hipPointerGetAttributes(&attributes, ptr) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  if (attributes.device != device) return false;  // another device's work is not waited for here
+  try {
+    std::vector<Retired> old;
+    {
+      std::lock_guard lock(retired_mutex);
+      auto& blocks = retired();
+      size_t held = bytes;
+      for (const Retired& b : blocks) held += b.bytes;
+      size_t drop = 0;
+      while (drop < blocks.size() && (blocks.size() - drop >= kRetiredBlocks || held > kRetiredBytes))
+        held -= blocks[drop++].bytes;
+      old.assign(blocks.begin(), blocks.begin() + static_cast<std::ptrdiff_t>(drop));
+      blocks.reserve(2 * kRetiredBlocks);
+      blocks.erase(blocks.begin(), blocks.begin() + static_cast<std::ptrdiff_t>(drop));
+      blocks.push_back({ptr, bytes, device, ++releases, false});
+    }
+    for (const Retired& b : old) (void)hipFree(b.ptr);
+  } catch (...) {
+    return false;
+  }
+  return true;
+}
+
+// A retired block of this size, once the device has finished all work queued
+// before now; null when there is none (or the device cannot be waited for, as
+// during a stream capture). The wait is outside the lock.
+void* reuse_retired(size_t bytes) {
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess) return nullptr;
+  Retired block{};
+  std::uint64_t until = 0;
+  {
+    std::lock_guard lock(retired_mutex);
+    auto& blocks = retired();
+    const auto found = std::find_if(blocks.rbegin(), blocks.rend(),
+                                    [&](const Retired& b) { return b.bytes == bytes && b.device == device; });
+    if (found == blocks.rend()) return nullptr;
+    block = *found;
+    until = releases;
+    blocks.erase(std::next(found).base());
+  }
+  if (block.idle) return block.ptr;
+  const bool waited = hipDeviceSynchronize() == hipSuccess;
+  if (!waited) (void)hipGetLastError();
+  std::lock_guard lock(retired_mutex);
+  if (!waited) {
+    retired().push_back(block);  // the room it left is reserved
+    return nullptr;
+  }
+  for (Retired& b : retired()) b.idle = b.idle || (b.device == device && b.number <= until);
+  return block.ptr;
+}
+
+hipError_t device_malloc(void** ptr, size_t bytes) {
+  if (void* const again = reuse_retired(bytes)) {
+    *ptr = again;
+    return hipSuccess;
+  }
+  hipError_t error = hipMalloc(ptr, bytes);
+  if (error != hipErrorOutOfMemory) return error;
+  {
+    std::lock_guard lock(retired_mutex);
+    if (retired().empty()) return error;
+  }
+  (void)hipGetLastError();
+  free_retired();
+  return hipMalloc(ptr, bytes);
+}
+
 int hip_allocate(void** ptr, size_t bytes) {
   if (tcx::forked()) return tcx::refuse_forked();
-  const hipError_t error = hipMalloc(ptr, bytes);
+  const hipError_t error = device_malloc(ptr, bytes);
   if (error == hipErrorOutOfMemory) {
     tcx::set_error("hipMalloc: out of memory");
     return TCX_POOL_OOM;
@@ -177,7 +292,8 @@ void pool_release(tcx_hip_pool* pool, void* ptr, size_t bytes, bool allow_cache)
     } else {
       ++pool->stats.uncached_returns;
       ++pool->stats.free_calls;
-      if (pool->runtime.free(ptr) != TCX_OK) {
+      const bool kept = !allow_cache && pool->default_runtime && retire(ptr, bytes);
+      if (!kept && pool->runtime.free(ptr) != TCX_OK) {
         ++pool->stats.free_failures;
         pool->stats.failed_free_bytes += bytes;
       }
@@ -274,7 +390,7 @@ int tcx_hip_allocate(size_t bytes, void** ptr, tcx_hip_pool_t** owner) {
   }
   const int status = tcx::ready();
   if (status != TCX_OK) return status;
-  return tcx::check(hipMalloc(ptr, bytes), "hipMalloc");
+  return tcx::check(device_malloc(ptr, bytes), "hipMalloc");
 }
 
 void tcx_hip_release(void* ptr, size_t bytes, tcx_hip_pool_t* owner) {
@@ -292,7 +408,7 @@ void tcx_hip_release_uncached(void* ptr, size_t bytes, tcx_hip_pool_t* owner) {
     pool_release(owner, ptr, bytes, false);
     return;
   }
-  (void)hipFree(ptr);
+  if (!retire(ptr, bytes)) (void)hipFree(ptr);
 }
 
 int tcx_hip_borrow_check(const void* ptr, size_t bytes) {
@@ -383,12 +499,14 @@ int tcx_hip_pool_exit(tcx_hip_pool_t* pool) {
   if (active_pool != pool)
     return tcx::fail(TCX_INVALID_ARGUMENT, "memory pool must exit on its owning thread");
   active_pool = nullptr;
+  if (pool->default_runtime) free_retired();
   std::lock_guard lock(pool->mutex);
   pool->stats.active = 0;
   return pool_trim_locked(pool);
 }
 
 int tcx_hip_pool_trim(tcx_hip_pool_t* pool) {
+  if (pool->default_runtime) free_retired();
   std::lock_guard lock(pool->mutex);
   return pool_trim_locked(pool);
 }
