@@ -108,17 +108,24 @@ std::int64_t gemm_splits(const tcx_hip_gemm_desc_t* d, std::int64_t batches) {
   return 1;
 }
 
-// Unbatched products whose K or N is not a multiple of 4 cannot use 16-byte
-// rows and run the scalar-load kernels (1025^3: 62 us against 23 us for
-// 1024^3). With a workspace, large ones run zero-padded copies instead: A [M][K4],
-// B [K4][N4] (or [N4][K4]) and the output [M][N4] in the workspace, the
-// aligned routes on those, then the output stripped back to [M][N] with the
-// bias and activation applied as the kernels' epilogue applies them. The
-// padded k terms are 0 x 0. Only products of at least kPadMinWork
-// multiply-adds pay for the copies and three extra launches: measured on
-// MI355X, padded against scalar loads, 4096 x 4095 x 4096 1058 against 1276
-// us, 2048 x 2049 x 2048 249 / 267, 3000 x 3001 x 1000 241 / 253; around
-// 10^9 multiply-adds it lost (1000 x 1001 x 999 transposed 40 / 32 us).
+// 128x128 tiles that fill the CUs: at least one round of 256, the last round at
+// least 90 % full.
+bool full_rounds_128(std::int64_t m, std::int64_t n, std::int64_t batches) {
+  const std::int64_t tiles = ((m + 127) / 128) * ((n + 127) / 128) * batches;
+  return tiles >= 256 && tiles * 10 >= (tiles + 255) / 256 * 256 * 9;
+}
+
+// Unbatched products whose K or N is not a multiple of 4 have no 16-byte rows.
+// The direct 64x64 kernel's ragged form takes most of them; where 128x128 tiles
+// would fill the CUs, large ones run zero-padded copies in a workspace instead:
+// A [M][K4], B [K4][N4] (or [N4][K4]) and the output [M][N4], the aligned routes
+// on those, then the output stripped back to [M][N] with the bias and activation
+// applied as the kernels' epilogue applies them. The padded k terms are 0 x 0.
+// Measured on MI355X, padded against ragged 64x64 tiles: 4096 x 4095 x 4096 1064
+// against 1253 us, 8191 x 2047 x 300 135 / 154, 4096 x 4096 x 525 200 / 225; but
+// without full rounds 2048 x 2049 x 2048 242 / 204, 3000 x 3001 x 1000 237 / 205,
+// 3441 x 4096 x 525 transposed 240 / 183. Around 10^9 multiply-adds the copies
+// and three extra launches cost more than they bring.
 constexpr std::int64_t kPadMinWork = std::int64_t{1} << 32;
 constexpr std::int64_t kPadAlign = 64;  // floats: 256-byte aligned regions
 
@@ -129,7 +136,9 @@ struct PadPlan {
 
 PadPlan pad_plan(const tcx_hip_gemm_desc_t* d) {
   PadPlan p{false, 0, 0, 0, 0, 0};
-  if (d->batch_rank != 0 || (d->k % 4 == 0 && d->n % 4 == 0) || d->m * d->n * d->k < kPadMinWork) return p;
+  if (d->batch_rank != 0 || (d->k % 4 == 0 && d->n % 4 == 0) || d->m * d->n * d->k < kPadMinWork ||
+      !full_rounds_128(d->m, d->n, 1))
+    return p;
   auto up = [](std::int64_t v, std::int64_t q) { return (v + q - 1) / q * q; };
   p.pad = true;
   p.k4 = up(d->k, 4);
@@ -295,7 +304,8 @@ extern "C" int tcx_hip_gemm_f32_ws(const float* lhs, const float* rhs, float* ou
   // One row of A against a transposed B, or one column of B: a
   // matrix-vector product, the long operand's rows streamed in whole cache
   // lines (one or no batch axis).
-  if (d->batch_rank <= 1 && strides_vec && d->k % 4 == 0 && aligned16(lhs) && aligned16(rhs)) {
+  // (Rows of 64 k at any address; shorter ones only where 16-byte.)
+  if (d->batch_rank <= 1 && (d->k >= 64 || (strides_vec && d->k % 4 == 0 && aligned16(lhs) && aligned16(rhs)))) {
     const std::int64_t lbs = d->batch_rank == 1 ? d->lhs_batch_strides[0] : 0;
     const std::int64_t rbs = d->batch_rank == 1 ? d->rhs_batch_strides[0] : 0;
     if (trans_b && d->m == 1)
@@ -340,12 +350,12 @@ extern "C" int tcx_hip_gemm_f32_ws(const float* lhs, const float* rhs, float* ou
   // 31.8 -> 20.4, 2048x1x2048 28.3 -> 13.3, 64 batches of 8x1024x1024
   // transposed 255.8 -> 57.6.
   constexpr std::int64_t kSkinny = gemm::kStreamMaxSkinny;
-  if (strides_vec && gemm::stream_fits(d->k) && aligned16(lhs)) {
-    if (trans_b && d->m <= kSkinny && d->n >= kStreamMinRows && aligned16(rhs))
-      return gemm::launch_stream<false, true>(args, s);
+  if (gemm::stream_fits(d->k)) {
+    const bool lhs_vec = strides_vec && d->k % 4 == 0 && aligned16(lhs), both_vec = lhs_vec && aligned16(rhs);
+    if (trans_b && d->m <= kSkinny && d->n >= kStreamMinRows) return gemm::launch_stream<false, true>(args, both_vec, s);
     if (d->n <= kSkinny && d->m >= kStreamMinRows) {
-      if (!trans_b) return gemm::launch_stream<true, false>(args, s);
-      if (aligned16(rhs)) return gemm::launch_stream<false, false>(args, s);
+      if (!trans_b) return gemm::launch_stream<true, false>(args, lhs_vec, s);
+      return gemm::launch_stream<false, false>(args, both_vec, s);
     }
   }
   // Many tiles of a short K (<= 64) and a narrow N (<= 64): the 64x64 tiles
@@ -355,7 +365,7 @@ extern "C" int tcx_hip_gemm_f32_ws(const float* lhs, const float* rhs, float* ou
   // 30 -> 61 us), so it stays narrow.
   if (vec && d->k <= 64 && d->n <= 64 && gemm::small_fits(d->m, d->n, d->k) &&
       ((d->m + 63) / 64) * ((d->n + 63) / 64) * batches > 768)
-    return gemm::launch_small(args, trans_b, s);
+    return gemm::launch_small(args, trans_b, vec, s);
   const std::int64_t tiles_256 = ((d->m + 255) / 256) * ((d->n + 255) / 256) * batches;
   // (Unaligned shapes take the scalar-load variant, which does not fit the
   // 256x256 tile's registers; they use the 128x128 tile.)
@@ -378,15 +388,13 @@ extern "C" int tcx_hip_gemm_f32_ws(const float* lhs, const float* rhs, float* ou
     return gemm::launch_direct<128, 128, 32, 32, 64, 2>(args, false, s);
   }
   if (vec && tiles_256 >= 256) return launch_config<256, 256, 32, 64, 128, 2, true>(args, trans_b, true, s);
-  // 128x128 tiles when there are >= 256 of them and the last round of 256
-  // blocks is >= 90 % full (3000x3000x1000: 576 tiles fill 75 % and ran 221 us
-  // against 203 us with 64x64 tiles).
-  const std::int64_t tiles_128 = ((d->m + 127) / 128) * ((d->n + 127) / 128) * batches;
-  if (tiles_128 >= 256 && tiles_128 * 10 >= (tiles_128 + 255) / 256 * 256 * 9)
+  // 128x128 tiles when they fill the CUs (3000x3000x1000: 576 tiles fill 75 %
+  // of their last round and ran 221 us against 203 us with 64x64 tiles).
+  if (full_rounds_128(d->m, d->n, batches))
     return launch_config<128, 128, 16, 32, 64, 2, false, 2>(args, trans_b, vec, s);
   const std::int64_t tiles_64 = ((d->m + 63) / 64) * ((d->n + 63) / 64) * batches;
   if (tiles_64 < 128) {
-    if (vec && gemm::small_fits(d->m, d->n, d->k)) return gemm::launch_small(args, trans_b, s);
+    if (gemm::small_fits(d->m, d->n, d->k)) return gemm::launch_small(args, trans_b, vec, s);
     return launch_config<32, 32, 32, 32, 32, 2, false, 8>(args, trans_b, vec, s);
   }
   // Up to three rounds of 64x64 tiles: the direct-to-LDS 64x64 kernel, edge
@@ -398,15 +406,19 @@ extern "C" int tcx_hip_gemm_f32_ws(const float* lhs, const float* rhs, float* ou
   // 1200^3 50.2 -> 40.8, 1600^3 92.4 -> 82.0, 4 x 500x600x700 34.2 -> 27.6 us;
   // with a fuller last round, or one round, 64x64 tiles stay ahead by 2-6 %
   // (1280^3, 1400^3, 1700^3; 1000^3 23.5 against 24.6 us).
-  if (vec && tiles_64 <= 768 && gemm::direct64_fits(d->m, d->n, d->k)) {
+  // Without 16-byte rows the direct kernel's ragged form stays ahead past three
+  // rounds too, from K = 128 on (10 x 2472x385xK, scalar loads against ragged:
+  // K = 33 52 / 62 us, 129 89 / 87, 257 123 / 109; 3000x3001x1000 253 / 205).
+  const bool direct64 = gemm::direct64_fits(d->m, d->n, d->k) && (vec || trans_b || d->n >= 4);
+  if (direct64 && (tiles_64 <= 768 || (!vec && d->k >= 128))) {
     // Skinny shapes whose 64x64 tiles are mostly padding run the small
     // kernel's 32x32 tiles when those waste at most two thirds as much
     // (8192x4x1000: 23.0 -> 13.1 us, 4x8192x1000: 22.5 -> 10.5 us; 1000^3
     // stays on 64x64 tiles, 24.2 against 33.8 us).
     const std::int64_t tiles_32 = ((d->m + 31) / 32) * ((d->n + 31) / 32) * batches;
-    if (8 * tiles_64 > 3 * tiles_32 && gemm::small_fits(d->m, d->n, d->k)) return gemm::launch_small(args, trans_b, s);
+    if (8 * tiles_64 > 3 * tiles_32 && gemm::small_fits(d->m, d->n, d->k)) return gemm::launch_small(args, trans_b, vec, s);
     const std::int64_t last = tiles_64 % 256;
-    return gemm::launch_direct64(args, trans_b, tiles_64 > 256 && last > 0 && last <= 128, s);
+    return gemm::launch_direct64(args, trans_b, tiles_64 > 256 && tiles_64 <= 768 && last > 0 && last <= 128, vec, s);
   }
   return launch_config<64, 64, 16, 32, 32, 4, false, 4>(args, trans_b, vec, s);
 }

@@ -732,6 +732,17 @@ int launch_direct(GemmArgs& args, bool trans_b, hipStream_t stream) {
   return check(hipGetLastError(), "gemm_f32 split reduce launch");
 }
 
+// A 16-byte load of the last k of a row of K floats, K not a multiple of 4,
+// is moved back to start at K - 4 so that it stays in the row. This puts the
+// K % 4 = rem values it was meant for in front and zeros behind them.
+__device__ __forceinline__ void ragged_tail(float4_t& v, int rem) {
+  const float4_t t = v;
+  v.x = rem == 1 ? t.w : rem == 2 ? t.z : t.y;
+  v.y = rem == 1 ? 0.F : rem == 2 ? t.w : t.z;
+  v.z = rem == 3 ? t.w : 0.F;
+  v.w = 0.F;
+}
+
 // Direct-to-LDS GEMM for BM x 64 output tiles of any shape (edge tiles
 // included), BM = 64 or 32: BM / 4 waves in four K groups of BM / 16 32x32
 // waves, each group taking 16 of every 64 staged k (its partial tile is added
@@ -760,7 +771,15 @@ int launch_direct(GemmArgs& args, bool trans_b, hipStream_t stream) {
 //   Output column of MFMA column r in block j: 32 wn + 2r + j for a [k, n] B
 //   (a lane's two columns are adjacent, one 8-byte read per k), 32 wn + 16j +
 //   r for a transposed B.
-template <bool kTransB, int BM>
+//   kRagged: K or N no multiple of 4, or an operand off a 16-byte boundary.
+//   The same 16-byte DMA from 4-byte aligned rows; a chunk of k that K cuts is
+//   loaded from K - 4 on and put right where the fragments are read
+//   (ragged_tail, last k-tile only), and the one chunk of a [k, n] B that would
+//   reach past the matrix, the last of its last row, is written by hand before
+//   the last tile is read. Against the scalar-load tiles of gemm_f32_kernel:
+//   1025^3 61.7 -> 39.1 us, 1001x1003x999 31.9 -> 24.0, 3898x320x753
+//   transposed 45.8 -> 27.0, 3328x1408x706 transposed 110 -> 82.
+template <bool kTransB, int BM, bool kRagged>
 __global__ __launch_bounds__(16 * BM) __attribute__((amdgpu_waves_per_eu(4, 8))) void gemm_f32_direct64_kernel(
     GemmArgs a) {
   static_assert(BM == 64 || BM == 32);
@@ -844,21 +863,26 @@ __global__ __launch_bounds__(16 * BM) __attribute__((amdgpu_waves_per_eu(4, 8)))
 #pragma clang diagnostic pop
   // An offset past every panel (voff + soff stays below 2^32): a zero read.
   constexpr int kOut = 0x7fffffff;
+  const int rem = static_cast<int>(K & 3);
   auto issue = [&](int stage, int k0) {
     const unsigned row_byte = static_cast<unsigned>(4 * wave * 64 * 4);
     const bool a_in = k0 + 4 * a_chunk < K;
-    dma16(a_rsrc, lds_of(&As[stage][0][0]) + row_byte, a_in ? a_voff : kOut, __builtin_amdgcn_readfirstlane(k0 * 4));
+    // Ragged: the k offset in the VGPR, less what moves a cut chunk back into its row.
+    const int over = k0 + 4 * a_chunk + 4 - static_cast<int>(K);
+    const int a_k = kRagged ? 4 * (k0 - max(over, 0)) : 0;
+    const int a_soff = kRagged ? 0 : __builtin_amdgcn_readfirstlane(k0 * 4);
+    dma16(a_rsrc, lds_of(&As[stage][0][0]) + row_byte, a_in ? a_voff + a_k : kOut, a_soff);
 #pragma unroll
     for (int h = 0; h < kBInst; ++h) {
       const unsigned b_byte = row_byte + static_cast<unsigned>(4 * kWaves * h * 64 * 4);
       if constexpr (kTransB) {
-        dma16(b_rsrc, lds_of(&Bs[stage][0][0]) + b_byte, a_in ? b_voff[h] : kOut,
-              __builtin_amdgcn_readfirstlane(k0 * 4));
+        dma16(b_rsrc, lds_of(&Bs[stage][0][0]) + b_byte, a_in ? b_voff[h] + a_k : kOut, a_soff);
       } else {
         // k rows past K and column chunks past N take the out-of-range
         // offset on the VGPR side alone, so the zero fill does not depend on
         // whether the range check counts the SGPR offset.
-        const bool b_in = k0 + 4 * kWaves * h + row < K && n0 + 4 * b_chunk < N;
+        const std::int64_t b_row = k0 + 4 * kWaves * h + row;
+        const bool b_in = b_row < K && n0 + 4 * b_chunk < N && !(kRagged && b_row == K - 1 && n0 + 4 * b_chunk + 4 > N);
         dma16(b_rsrc, lds_of(&Bs[stage][0][0]) + b_byte, b_in ? b_voff[h] : kOut,
               __builtin_amdgcn_readfirstlane(k0 * static_cast<int>(N) * 4));
       }
@@ -914,13 +938,45 @@ __global__ __launch_bounds__(16 * BM) __attribute__((amdgpu_waves_per_eu(4, 8)))
         for (int j = 0; j < 2; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.a[i][q], f.b[j][q], acc[i][j], 0, 0, 0);
   };
-  auto compute = [&](int stage) {
+  const int k_tiles = static_cast<int>((K + BKT - 1) / BKT);
+  // The cut chunk of k tile kt, where this lane's fragment holds it.
+  auto fix = [&](int kt, Frag& f) {
+    if constexpr (kRagged) {
+      if (rem == 0 || kt != k_tiles - 1) return;
+      if (kt * BKT + 4 * (group * 4 + kl) != K - rem) return;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) ragged_tail(f.a[i], rem);
+      if constexpr (kTransB) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) ragged_tail(f.b[j], rem);
+      }
+    }
+  };
+  auto compute = [&](int kt, int stage) {
     Frag f;
     load(stage, f);
+    fix(kt, f);
     mma(f);
   };
-
-  const int k_tiles = static_cast<int>((K + BKT - 1) / BKT);
+  // A [k, n] B whose last row ends inside a chunk of this tile: lanes 0 .. 2
+  // hold the columns of that chunk and write them once the last k tile has
+  // landed and before any wave reads it.
+  const int cut_n = static_cast<int>(N & 3);
+  const bool cut = kRagged && !kTransB && cut_n != 0 && n0 + 64 > N;
+  float cut_value = 0.F;
+  if constexpr (kRagged && !kTransB) {
+    if (cut && tid < cut_n) cut_value = B[K * N - cut_n + tid];
+  }
+  auto patch = [&](int stage) {
+    if constexpr (kRagged && !kTransB) {
+      if (!cut) return;
+      if (tid < cut_n) {
+        const int kr = static_cast<int>((K - 1) % BKT), c = static_cast<int>(N - cut_n - n0) / 4;
+        Bs[stage][kr][4 * (c ^ (8 * ((kr >> 2) & 1))) + tid] = cut_value;
+      }
+      __syncthreads();
+    }
+  };
   if constexpr (BM == 32) {
     // One k-tile per barrier over three stages, two tiles in flight: the
     // barrier of tile kt frees the stage of tile kt - 1 for tile kt + 2. The
@@ -932,7 +988,8 @@ __global__ __launch_bounds__(16 * BM) __attribute__((amdgpu_waves_per_eu(4, 8)))
       else __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
       if (kt + 2 < k_tiles) issue((kt + 2) % kStages, (kt + 2) * BKT);
-      compute(kt % kStages);
+      if (kt == k_tiles - 1) patch(kt % kStages);
+      compute(kt, kt % kStages);
     }
   } else {
   // Two k-tiles per barrier over four stages: tiles kt and kt + 1 are read
@@ -949,10 +1006,10 @@ __global__ __launch_bounds__(16 * BM) __attribute__((amdgpu_waves_per_eu(4, 8)))
     // 1000^3 24.2 -> 24.0 us, 1024^3 23.5 -> 23.1 us).
     __builtin_amdgcn_s_waitcnt(0x0F76);  // vmcnt(6): tile 0
     __syncthreads();
-    compute(0);
+    compute(0, 0);
     __builtin_amdgcn_s_waitcnt(0x0F74);  // vmcnt(4): tile 1
     __syncthreads();
-    compute(1);
+    compute(1, 1);
     __builtin_amdgcn_s_waitcnt(0);  // tiles 2 and 3
     __syncthreads();
     kt0 = 2;
@@ -970,9 +1027,12 @@ __global__ __launch_bounds__(16 * BM) __attribute__((amdgpu_waves_per_eu(4, 8)))
     // Both tiles' fragment reads go out before the first MFMA (the stage of
     // a missing odd tile is read but not used): the second tile's reads land
     // under the first tile's MFMAs (1000^3: 23.8 -> 23.55 us).
+    if (kt + 2 >= k_tiles) patch((k_tiles - 1) % kStages);
     Frag f0, f1;
     load(kt % kStages, f0);
     load((kt + 1) % kStages, f1);
+    fix(kt, f0);
+    fix(kt + 1, f1);
     __builtin_amdgcn_sched_barrier(0);
     mma(f0);
     if (kt + 1 < k_tiles) mma(f1);
@@ -1026,34 +1086,35 @@ __global__ __launch_bounds__(16 * BM) __attribute__((amdgpu_waves_per_eu(4, 8)))
   }
 }
 
-// True when gemm_f32_direct64_kernel can take the problem: 16-byte rows
-// (k and n multiples of 4, 16-byte aligned operands, checked by the caller)
-// and every byte offset into a panel, a tile's 64 rows included, below 2^31.
+// True when gemm_f32_direct64_kernel can take the problem: rows of at least
+// four k and every byte offset into a panel, a tile's 64 rows included, below
+// 2^31.
 inline bool direct64_fits(std::int64_t m, std::int64_t n, std::int64_t k) {
   constexpr double kLimit = 2147483647.0;
   const double rows_m = static_cast<double>(m < 64 ? 64 : m), rows_n = static_cast<double>(n < 64 ? 64 : n);
-  return m > 0 && n > 0 && k > 0 && k % 4 == 0 && n % 4 == 0 && rows_m * k * 4 < kLimit &&
-         rows_n * k * 4 < kLimit && (static_cast<double>(k) + 64) * n * 4 < kLimit;
+  return m > 0 && n > 0 && k >= 4 && rows_m * k * 4 < kLimit && rows_n * k * 4 < kLimit &&
+         (static_cast<double>(k) + 64) * n * 4 < kLimit;
 }
 
-// half: 32x64 tiles instead of 64x64.
-inline int launch_direct64(GemmArgs& args, bool trans_b, bool half, hipStream_t stream) {
+// half: 32x64 tiles instead of 64x64. vec: 16-byte rows (k and n multiples of
+// 4, 16-byte aligned operands).
+inline int launch_direct64(GemmArgs& args, bool trans_b, bool half, bool vec, hipStream_t stream) {
   if (!direct64_fits(args.m, args.n, args.k))
-    return fail(TCX_INTERNAL, "direct 64x64 gemm needs 16-byte rows and 31-bit panel offsets");
+    return fail(TCX_INTERNAL, "direct 64x64 gemm needs rows of four k and 31-bit panel offsets");
   const int bm = half ? 32 : 64;
   args.tiles_m = (args.m + bm - 1) / bm;
   args.tiles_n = (args.n + 63) / 64;
   args.total_tiles = args.tiles_m * args.tiles_n * args.total_tiles;  // caller passes the batch count
   if (args.total_tiles > 0x7fffffff) return fail(TCX_INVALID_ARGUMENT, "gemm grid is too large");
   const dim3 grid(static_cast<unsigned>(args.total_tiles)), block(16 * bm);
-  if (half && trans_b)
-    hipLaunchKernelGGL((gemm_f32_direct64_kernel<true, 32>), grid, block, 0, stream, args);
-  else if (half)
-    hipLaunchKernelGGL((gemm_f32_direct64_kernel<false, 32>), grid, block, 0, stream, args);
-  else if (trans_b)
-    hipLaunchKernelGGL((gemm_f32_direct64_kernel<true, 64>), grid, block, 0, stream, args);
-  else
-    hipLaunchKernelGGL((gemm_f32_direct64_kernel<false, 64>), grid, block, 0, stream, args);
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, stream, args); };
+  if (vec) {
+    if (half) go(trans_b ? gemm_f32_direct64_kernel<true, 32, false> : gemm_f32_direct64_kernel<false, 32, false>);
+    else go(trans_b ? gemm_f32_direct64_kernel<true, 64, false> : gemm_f32_direct64_kernel<false, 64, false>);
+  } else {
+    if (half) go(trans_b ? gemm_f32_direct64_kernel<true, 32, true> : gemm_f32_direct64_kernel<false, 32, true>);
+    else go(trans_b ? gemm_f32_direct64_kernel<true, 64, true> : gemm_f32_direct64_kernel<false, 64, true>);
+  }
   return check(hipGetLastError(), "gemm_f32 direct 64-column tile launch");
 }
 
@@ -1072,7 +1133,10 @@ inline int launch_direct64(GemmArgs& args, bool trans_b, bool half, hipStream_t 
 // operand panels, so rows past M or N read zero; lanes past K, [k, n] B
 // columns past N and chunks past the wave's run take an out-of-range offset
 // (zero, no memory access), so every group issues the same loads.
-template <bool kTransB, int KS, int kG>
+//   kRagged as in gemm_f32_direct64_kernel: loads cut by K start at K - 4 and
+// pass ragged_tail; a [k, n] B's pair of columns cut by N starts a column early
+// (142x320x739 transposed 14.7 -> 7.5 us, 128x431x1408 22.9 -> 14.2).
+template <bool kTransB, int KS, int kG, bool kRagged>
 __global__ __launch_bounds__(64 * KS) void gemm_f32_small_kernel(GemmArgs a) {
   const std::int64_t per_batch = a.tiles_m * a.tiles_n;
   const std::int64_t grid = a.total_tiles;
@@ -1109,14 +1173,19 @@ __global__ __launch_bounds__(64 * KS) void gemm_f32_small_kernel(GemmArgs a) {
   };
   // The launcher checks that every panel spans less than 2^31 bytes.
   const auto a_rsrc = rsrc_of(a.lhs + lhs_off + m0 * K, (M - m0) * K * 4);
-  const auto b_rsrc = kTransB ? rsrc_of(a.rhs + rhs_off + n0 * K, (N - n0) * K * 4)
-                              : rsrc_of(a.rhs + rhs_off + n0, (K * N - n0) * 4);
+  // (Ragged: from the matrix's first column, as a pair may start before n0.)
+  const auto b_rsrc = kTransB   ? rsrc_of(a.rhs + rhs_off + n0 * K, (N - n0) * K * 4)
+                      : kRagged ? rsrc_of(a.rhs + rhs_off, K * N * 4)
+                                : rsrc_of(a.rhs + rhs_off + n0, (K * N - n0) * 4);
   constexpr int kOut = 0x7fffffff;
   const int Ki = static_cast<int>(K), Ni = static_cast<int>(N);
   // This wave's chunks: [c_begin, c_end), at least one when KS <= chunks.
   const int chunks = (Ki + 15) / 16;
   const int c_begin = wave * chunks / KS, c_end = (wave + 1) * chunks / KS;
   const bool b_col_in = n0 + 2 * r < N;
+  const bool b_odd = kRagged && n0 + 2 * r + 1 == N;  // the pair's second column is past N
+  const int b_col = 2 * r + (kRagged ? static_cast<int>(n0) - (b_odd ? 1 : 0) : 0);
+  const int rem = Ki & 3;
 
   struct Frag {
     float4_t a[2], b[2];
@@ -1124,23 +1193,25 @@ __global__ __launch_bounds__(64 * KS) void gemm_f32_small_kernel(GemmArgs a) {
   auto load = [&](int c, Frag& f) {
     const int k = 16 * c + 4 * kl;
     const bool k_in = c < c_end && k < Ki;
+    const int kf = kRagged ? min(k, Ki - 4) : k;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
       f.a[i] = __builtin_bit_cast(
-          float4_t, __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, k_in ? ((16 * i + r) * Ki + k) * 4 : kOut, 0, 0));
+          float4_t, __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, k_in ? ((16 * i + r) * Ki + kf) * 4 : kOut, 0, 0));
     if constexpr (kTransB) {
 #pragma unroll
       for (int j = 0; j < 2; ++j)
         f.b[j] = __builtin_bit_cast(
-            float4_t, __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, k_in ? ((16 * j + r) * Ki + k) * 4 : kOut, 0, 0));
+            float4_t, __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, k_in ? ((16 * j + r) * Ki + kf) * 4 : kOut, 0, 0));
     } else {
       using float2v = float __attribute__((ext_vector_type(2)));
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const bool in = c < c_end && k + q < Ki && b_col_in;
         const float2v v = __builtin_bit_cast(
-            float2v, __builtin_amdgcn_raw_buffer_load_b64(b_rsrc, in ? ((k + q) * Ni + 2 * r) * 4 : kOut, 0, 0));
-        f.b[0][q] = v.x;
+            float2v, __builtin_amdgcn_raw_buffer_load_b64(
+                         b_rsrc, in ? ((k + q) * Ni + b_col) * 4 : kOut, 0, 0));
+        f.b[0][q] = kRagged && b_odd ? v.y : v.x;
         f.b[1][q] = v.y;
       }
     }
@@ -1166,10 +1237,22 @@ __global__ __launch_bounds__(64 * KS) void gemm_f32_small_kernel(GemmArgs a) {
 #pragma unroll
     for (int u = 0; u < kG; ++u) load(c0 + u, f[u]);
   };
-  auto mma_group = [&](int c0, const Frag (&f)[kG]) {
+  auto mma_group = [&](int c0, Frag (&f)[kG]) {
 #pragma unroll
     for (int u = 0; u < kG; ++u)
-      if (c0 + u < c_end) mma(f[u]);
+      if (c0 + u < c_end) {
+        if constexpr (kRagged) {
+          if (rem != 0 && c0 + u == chunks - 1 && 16 * (c0 + u) + 4 * kl == Ki - rem) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) ragged_tail(f[u].a[i], rem);
+            if constexpr (kTransB) {
+#pragma unroll
+              for (int j = 0; j < 2; ++j) ragged_tail(f[u].b[j], rem);
+            }
+          }
+        }
+        mma(f[u]);
+      }
   };
   load_group(c_begin, f0);
   for (int c0 = c_begin; c0 < c_end; c0 += 2 * kG) {
@@ -1214,29 +1297,33 @@ __global__ __launch_bounds__(64 * KS) void gemm_f32_small_kernel(GemmArgs a) {
   }
 }
 
-// True when gemm_f32_small_kernel can take the problem: 16-byte rows and
-// every byte offset into a panel below 2^31 (rows of a 32-row tile included).
+// True when gemm_f32_small_kernel can take the problem: rows of at least four k
+// (and two n) and every byte offset into a panel below 2^31 (rows of a 32-row
+// tile included).
 inline bool small_fits(std::int64_t m, std::int64_t n, std::int64_t k) {
   constexpr double kLimit = 2147483647.0;
   const double rows_m = static_cast<double>(m < 32 ? 32 : m), rows_n = static_cast<double>(n < 32 ? 32 : n);
-  return m > 0 && n > 0 && k > 0 && k % 4 == 0 && n % 4 == 0 && rows_m * k * 4 < kLimit &&
-         rows_n * k * 4 < kLimit && (static_cast<double>(k) + 16) * n * 4 < kLimit;
+  return m > 0 && n >= 2 && k >= 4 && rows_m * k * 4 < kLimit && rows_n * k * 4 < kLimit &&
+         (static_cast<double>(k) + 16) * n * 4 < kLimit;
 }
 
 template <bool kTransB, int KS>
-void launch_small_as(GemmArgs& args, hipStream_t stream) {
+void launch_small_as(GemmArgs& args, bool vec, hipStream_t stream) {
   // Two groups of four chunks in flight (160 VGPRs) up to two waves per SIMD
   // (KS <= 8); two chunks per group at 16 waves per block.
   constexpr int kG = KS <= 8 ? 4 : 2;
-  hipLaunchKernelGGL((gemm_f32_small_kernel<kTransB, KS, kG>), dim3(static_cast<unsigned>(args.total_tiles)),
-                     dim3(64 * KS), 0, stream, args);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(args.total_tiles)), dim3(64 * KS), 0, stream, args);
+  };
+  go(vec ? gemm_f32_small_kernel<kTransB, KS, kG, false> : gemm_f32_small_kernel<kTransB, KS, kG, true>);
 }
 
 // KS: enough waves for about sixteen per CU over the launch (512^3: 8.4
 // against 9.5 us with eight), at most one per 16-k chunk and at most 16.
-inline int launch_small(GemmArgs& args, bool trans_b, hipStream_t stream) {
+// vec: 16-byte rows, as for launch_direct64.
+inline int launch_small(GemmArgs& args, bool trans_b, bool vec, hipStream_t stream) {
   if (!small_fits(args.m, args.n, args.k))
-    return fail(TCX_INTERNAL, "small gemm needs 16-byte rows and 31-bit panel offsets");
+    return fail(TCX_INTERNAL, "small gemm needs rows of four k and 31-bit panel offsets");
   args.tiles_m = (args.m + 31) / 32;
   args.tiles_n = (args.n + 31) / 32;
   args.total_tiles = args.tiles_m * args.tiles_n * args.total_tiles;  // caller passes the batch count
@@ -1245,11 +1332,11 @@ inline int launch_small(GemmArgs& args, bool trans_b, hipStream_t stream) {
   int ks = 1;
   while (ks < 16 && ks * 2 <= chunks && args.total_tiles * ks < 4096) ks *= 2;
   switch (ks) {
-    case 1: trans_b ? launch_small_as<true, 1>(args, stream) : launch_small_as<false, 1>(args, stream); break;
-    case 2: trans_b ? launch_small_as<true, 2>(args, stream) : launch_small_as<false, 2>(args, stream); break;
-    case 4: trans_b ? launch_small_as<true, 4>(args, stream) : launch_small_as<false, 4>(args, stream); break;
-    case 8: trans_b ? launch_small_as<true, 8>(args, stream) : launch_small_as<false, 8>(args, stream); break;
-    default: trans_b ? launch_small_as<true, 16>(args, stream) : launch_small_as<false, 16>(args, stream); break;
+    case 1: trans_b ? launch_small_as<true, 1>(args, vec, stream) : launch_small_as<false, 1>(args, vec, stream); break;
+    case 2: trans_b ? launch_small_as<true, 2>(args, vec, stream) : launch_small_as<false, 2>(args, vec, stream); break;
+    case 4: trans_b ? launch_small_as<true, 4>(args, vec, stream) : launch_small_as<false, 4>(args, vec, stream); break;
+    case 8: trans_b ? launch_small_as<true, 8>(args, vec, stream) : launch_small_as<false, 8>(args, vec, stream); break;
+    default: trans_b ? launch_small_as<true, 16>(args, vec, stream) : launch_small_as<false, 16>(args, vec, stream); break;
   }
   return check(hipGetLastError(), "gemm_f32 small launch");
 }
@@ -1271,8 +1358,9 @@ inline int launch_small(GemmArgs& args, bool trans_b, hipStream_t stream) {
 // groups in flight. The KS partial tiles meet in LDS and are added in wave
 // order with the bias and activation. Rows of W past I, rows of X past J and
 // k past K read zero through the buffer range checks and an out-of-range
-// offset.
-template <bool kXCols, bool kOutJI, int kMB, int KS, int kG>
+// offset. kRagged as in gemm_f32_small_kernel (8x438x707 transposed on scalar
+// tiles 14.4, here 4.2 us).
+template <bool kXCols, bool kOutJI, int kMB, int KS, int kG, bool kRagged>
 __global__ __launch_bounds__(64 * KS) void gemm_f32_stream_kernel(GemmArgs a) {
   const std::int64_t M = a.m, N = a.n, K = a.k;
   const std::int64_t I = kOutJI ? N : M, J = kOutJI ? M : N;
@@ -1314,19 +1402,22 @@ __global__ __launch_bounds__(64 * KS) void gemm_f32_stream_kernel(GemmArgs a) {
   auto load = [&](int c, Frag& f) {
     const int k = 16 * c + 4 * kl;
     const bool k_in = c < c_end && k < Ki;
-    f.w = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, k_in ? (r * Ki + k) * 4 : kOut,
+    const int kf = kRagged ? min(k, Ki - 4) : k;
+    f.w = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, k_in ? (r * Ki + kf) * 4 : kOut,
                                                                              0, 0));
 #pragma unroll
     for (int g = 0; g < kMB; ++g) {
       const int j = 16 * g + r;
       if constexpr (kXCols) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+        for (int q = 0; q < 4; ++q) {
+          const bool in = k_in && j < Ji && (!kRagged || k + q < Ki);
           f.x[g][q] = __builtin_bit_cast(
-              float, __builtin_amdgcn_raw_buffer_load_b32(x_rsrc, k_in && j < Ji ? ((k + q) * Ji + j) * 4 : kOut, 0, 0));
+              float, __builtin_amdgcn_raw_buffer_load_b32(x_rsrc, in ? ((k + q) * Ji + j) * 4 : kOut, 0, 0));
+        }
       } else {
         f.x[g] = __builtin_bit_cast(
-            float4_t, __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, k_in && j < Ji ? (j * Ki + k) * 4 : kOut, 0, 0));
+            float4_t, __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, k_in && j < Ji ? (j * Ki + kf) * 4 : kOut, 0, 0));
       }
     }
   };
@@ -1345,10 +1436,22 @@ __global__ __launch_bounds__(64 * KS) void gemm_f32_stream_kernel(GemmArgs a) {
 #pragma unroll
     for (int u = 0; u < kG; ++u) load(c0 + u, f[u]);
   };
-  auto mma_group = [&](int c0, const Frag (&f)[kG]) {
+  const int rem = Ki & 3;
+  auto mma_group = [&](int c0, Frag (&f)[kG]) {
 #pragma unroll
     for (int u = 0; u < kG; ++u)
-      if (c0 + u < c_end) mma(f[u]);
+      if (c0 + u < c_end) {
+        if constexpr (kRagged) {
+          if (rem != 0 && c0 + u == chunks - 1 && 16 * (c0 + u) + 4 * kl == Ki - rem) {
+            ragged_tail(f[u].w, rem);
+            if constexpr (!kXCols) {
+#pragma unroll
+              for (int g = 0; g < kMB; ++g) ragged_tail(f[u].x[g], rem);
+            }
+          }
+        }
+        mma(f[u]);
+      }
   };
   load_group(c_begin, f0);
   for (int c0 = c_begin; c0 < c_end; c0 += 2 * kG) {
@@ -1404,7 +1507,9 @@ __global__ __launch_bounds__(64 * KS) void gemm_f32_stream_kernel(GemmArgs a) {
 // Against gemm_f32_stream_kernel on MI355X: 16x4096x4096 20.8 -> 16.2 us,
 // 32x4096x4096 28.5 -> 19.3, 16x14336x4096 66.2 -> 54.4, 32x11008x4096
 // 76.1 -> 54.0, 24x2048x2048 13.7 -> 10.7.
-template <int kMB, int KS>
+// kRagged: 4-byte aligned rows by the same DMA, a chunk cut by K loaded from
+// K - 4 on and put right as it is read (last span only).
+template <int kMB, int KS, bool kRagged>
 __global__ __launch_bounds__(64 * KS) void gemm_f32_stream_lds_kernel(GemmArgs a) {
   constexpr int kStages = 3, kSpan = 64, kTile = 16 * kSpan;
   constexpr int kPer = (1 + kMB) * kTile;  // floats of one stage: W, then kMB row groups of X
@@ -1462,12 +1567,13 @@ __global__ __launch_bounds__(64 * KS) void gemm_f32_stream_lds_kernel(GemmArgs a
     for (int u = 0; u < 4; ++u) {
       const int row = 4 * u + lane / 16;
       const int k = k0 + 4 * (slot ^ row);
-      const bool k_in = k < Ki;  // K % 4 == 0: a chunk is whole or past K
-      dma16(w_rsrc, lds_of(base) + u * 1024, k_in ? (row * Ki + k) * 4 : kOut);
+      const bool k_in = k < Ki;
+      const int kf = kRagged ? min(k, Ki - 4) : k;
+      dma16(w_rsrc, lds_of(base) + u * 1024, k_in ? (row * Ki + kf) * 4 : kOut);
 #pragma unroll
       for (int g = 0; g < kMB; ++g) {
         const int j = 16 * g + row;
-        dma16(x_rsrc, lds_of(base + (1 + g) * kTile) + u * 1024, k_in && j < Ji ? (j * Ki + k) * 4 : kOut);
+        dma16(x_rsrc, lds_of(base + (1 + g) * kTile) + u * 1024, k_in && j < Ji ? (j * Ki + kf) * 4 : kOut);
       }
     }
   };
@@ -1476,15 +1582,23 @@ __global__ __launch_bounds__(64 * KS) void gemm_f32_stream_lds_kernel(GemmArgs a
   for (int h = 0; h < 2; ++h)
 #pragma unroll
     for (int g = 0; g < kMB; ++g) acc[h][g] = floatx4{0.F, 0.F, 0.F, 0.F};
-  auto compute = [&](int stage) {
+  const int rem = Ki & 3;
+  auto compute = [&](int s, int stage) {
     const float* const base = mine + stage * kPer;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       const int off = r * kSpan + 4 * ((4 * c + kl) ^ r);
-      const float4_t w = *reinterpret_cast<const float4_t*>(base + off);
+      float4_t w = *reinterpret_cast<const float4_t*>(base + off);
       float4_t x[kMB];
 #pragma unroll
       for (int g = 0; g < kMB; ++g) x[g] = *reinterpret_cast<const float4_t*>(base + (1 + g) * kTile + off);
+      if constexpr (kRagged) {
+        if (rem != 0 && s == spans - 1 && s * kSpan + 4 * (4 * c + kl) == Ki - rem) {
+          ragged_tail(w, rem);
+#pragma unroll
+          for (int g = 0; g < kMB; ++g) ragged_tail(x[g], rem);
+        }
+      }
 #pragma unroll
       for (int q = 0; q < 4; ++q)
 #pragma unroll
@@ -1500,7 +1614,7 @@ __global__ __launch_bounds__(64 * KS) void gemm_f32_stream_lds_kernel(GemmArgs a
     if (s + 1 < s_end) __builtin_amdgcn_s_waitcnt(0x0F70 | kInst);
     else __builtin_amdgcn_s_waitcnt(0x0F70);
     asm volatile("" ::: "memory");  // the stage's LDS reads stay after the wait
-    compute((s - s_begin) % kStages);
+    compute(s, (s - s_begin) % kStages);
     // The stage of span s - 1, whose reads this wave has consumed.
     if (s + 2 < s_end) issue(s + 2, (s + 2 - s_begin) % kStages);
   }
@@ -1547,6 +1661,12 @@ __global__ __launch_bounds__(64 * KS) void gemm_f32_stream_lds_kernel(GemmArgs a
 // contiguous (a row of x, or the column of a [k, 1] b); y_stride is the
 // element stride of y in the output; bias is per row (bias_per_row) or one
 // value.
+// 16 bytes at a 4-byte aligned address, read once.
+using float4_u = float __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float4_t stream_load4(const float* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const float4_u*>(p));
+}
+
 template <int KW>
 __global__ __launch_bounds__(256) void gemv_f32_kernel(const float* __restrict__ R, const float* __restrict__ v,
                                                        float* __restrict__ y, const float* __restrict__ bias,
@@ -1565,25 +1685,28 @@ __global__ __launch_bounds__(256) void gemv_f32_kernel(const float* __restrict__
     const float* __restrict__ rp = R + batch * r_batch + i * K;
     const float* __restrict__ vp = v + batch * v_batch;
     // This wave's run of K: whole 1024-element strides first, 4-element
-    // groups after (K % 4 == 0).
+    // groups after, from rows at any 4-byte address; the last K % 4 elements
+    // are single words of the last wave.
+    const std::int64_t K4 = K & ~std::int64_t{3};
     const std::int64_t run = (K / 4 + KW - 1) / KW * 4;
-    const std::int64_t k_begin = part * run, k_end = min(K, k_begin + run);
+    const std::int64_t k_begin = part * run, k_end = min(K4, k_begin + run);
     float s[8] = {};
     std::int64_t k = k_begin + 4 * lane;
     for (; k + 7 * 256 < k_end; k += 8 * 256) {
       float4_t w[8], x[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) w[u] = stream_load(reinterpret_cast<const float4_t*>(rp + k + 256 * u));
+      for (int u = 0; u < 8; ++u) w[u] = stream_load4(rp + k + 256 * u);
 #pragma unroll
-      for (int u = 0; u < 8; ++u) x[u] = *reinterpret_cast<const float4_t*>(vp + k + 256 * u);
+      for (int u = 0; u < 8; ++u) x[u] = *reinterpret_cast<const float4_u*>(vp + k + 256 * u);
 #pragma unroll
       for (int u = 0; u < 8; ++u) s[u] += (w[u].x * x[u].x + w[u].y * x[u].y) + (w[u].z * x[u].z + w[u].w * x[u].w);
     }
     for (; k < k_end; k += 256) {
-      const float4_t w = stream_load(reinterpret_cast<const float4_t*>(rp + k));
-      const float4_t x = *reinterpret_cast<const float4_t*>(vp + k);
+      const float4_t w = stream_load4(rp + k);
+      const float4_t x = *reinterpret_cast<const float4_u*>(vp + k);
       s[0] += (w.x * x.x + w.y * x.y) + (w.z * x.z + w.w * x.w);
     }
+    if (part == KW - 1 && K4 + lane < K) s[1] += rp[K4 + lane] * vp[K4 + lane];
     sum = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
   }
   sum = wave_sum(sum);
@@ -2071,26 +2194,29 @@ constexpr std::int64_t kStreamMaxSkinny = 32;
 // and kStreamMaxSkinny rows of K floats (the skinny operand's buffer range)
 // below 2^31 bytes.
 inline bool stream_fits(std::int64_t k) {
-  return k > 0 && k % 4 == 0 && static_cast<double>(kStreamMaxSkinny) * static_cast<double>(k) * 4 < 2147483647.0;
+  return k >= 4 && static_cast<double>(kStreamMaxSkinny) * static_cast<double>(k) * 4 < 2147483647.0;
 }
 
 template <bool kXCols, bool kOutJI, int kMB, int KS>
-void launch_stream_as(const GemmArgs& args, std::int64_t blocks, hipStream_t stream) {
+void launch_stream_as(const GemmArgs& args, bool vec, std::int64_t blocks, hipStream_t stream) {
   // Two groups of four chunks in flight for one row group of X, of two
   // chunks for two (the registers of four waves per SIMD at KS = 16).
   constexpr int kG = kMB == 1 ? 4 : 2;
-  hipLaunchKernelGGL((gemm_f32_stream_kernel<kXCols, kOutJI, kMB, KS, kG>), dim3(static_cast<unsigned>(blocks)),
-                     dim3(64 * KS), 0, stream, args);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(64 * KS), 0, stream, args);
+  };
+  go(vec ? gemm_f32_stream_kernel<kXCols, kOutJI, kMB, KS, kG, false>
+         : gemm_f32_stream_kernel<kXCols, kOutJI, kMB, KS, kG, true>);
 }
 
 template <bool kXCols, bool kOutJI, int kMB>
-void launch_stream_ks(const GemmArgs& args, std::int64_t blocks, int ks, hipStream_t stream) {
+void launch_stream_ks(const GemmArgs& args, bool vec, std::int64_t blocks, int ks, hipStream_t stream) {
   switch (ks) {
-    case 1: launch_stream_as<kXCols, kOutJI, kMB, 1>(args, blocks, stream); break;
-    case 2: launch_stream_as<kXCols, kOutJI, kMB, 2>(args, blocks, stream); break;
-    case 4: launch_stream_as<kXCols, kOutJI, kMB, 4>(args, blocks, stream); break;
-    case 8: launch_stream_as<kXCols, kOutJI, kMB, 8>(args, blocks, stream); break;
-    default: launch_stream_as<kXCols, kOutJI, kMB, 16>(args, blocks, stream); break;
+    case 1: launch_stream_as<kXCols, kOutJI, kMB, 1>(args, vec, blocks, stream); break;
+    case 2: launch_stream_as<kXCols, kOutJI, kMB, 2>(args, vec, blocks, stream); break;
+    case 4: launch_stream_as<kXCols, kOutJI, kMB, 4>(args, vec, blocks, stream); break;
+    case 8: launch_stream_as<kXCols, kOutJI, kMB, 8>(args, vec, blocks, stream); break;
+    default: launch_stream_as<kXCols, kOutJI, kMB, 16>(args, vec, blocks, stream); break;
   }
 }
 
@@ -2098,8 +2224,9 @@ void launch_stream_ks(const GemmArgs& args, std::int64_t blocks, int ks, hipStre
 // most 32 columns of B, kXCols when B is [k, n]). args.total_tiles holds the
 // batch count. KS as for the small kernel: about sixteen waves per CU over
 // the launch, at most one per 16-k chunk and at most 16.
+// vec: K a multiple of 4 and 16-byte rows of the operands read along K.
 template <bool kXCols, bool kOutJI>
-int launch_stream(GemmArgs& args, hipStream_t stream) {
+int launch_stream(GemmArgs& args, bool vec, hipStream_t stream) {
   const std::int64_t I = kOutJI ? args.n : args.m, J = kOutJI ? args.m : args.n;
   if (J > kStreamMaxSkinny || !stream_fits(args.k))
     return fail(TCX_INTERNAL, "streaming gemm needs at most 32 skinny rows");
@@ -2118,12 +2245,16 @@ int launch_stream(GemmArgs& args, hipStream_t stream) {
       auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(64 * waves), 0, stream, args);
       };
-      if (J <= 16)
-        go(waves == 1 ? gemm_f32_stream_lds_kernel<1, 1>
-                      : waves == 2 ? gemm_f32_stream_lds_kernel<1, 2> : gemm_f32_stream_lds_kernel<1, 4>);
-      else
-        go(waves == 1 ? gemm_f32_stream_lds_kernel<2, 1>
-                      : waves == 2 ? gemm_f32_stream_lds_kernel<2, 2> : gemm_f32_stream_lds_kernel<2, 4>);
+      auto pick = [&]<bool kRagged>(std::bool_constant<kRagged>) {
+        if (J <= 16)
+          go(waves == 1 ? gemm_f32_stream_lds_kernel<1, 1, kRagged>
+                        : waves == 2 ? gemm_f32_stream_lds_kernel<1, 2, kRagged> : gemm_f32_stream_lds_kernel<1, 4, kRagged>);
+        else
+          go(waves == 1 ? gemm_f32_stream_lds_kernel<2, 1, kRagged>
+                        : waves == 2 ? gemm_f32_stream_lds_kernel<2, 2, kRagged> : gemm_f32_stream_lds_kernel<2, 4, kRagged>);
+      };
+      if (vec) pick(std::false_type{});
+      else pick(std::true_type{});
       return check(hipGetLastError(), "gemm_f32 streaming launch");
     }
   }
@@ -2131,9 +2262,9 @@ int launch_stream(GemmArgs& args, hipStream_t stream) {
   int ks = 1;
   while (ks < 16 && ks * 2 <= chunks && blocks * ks < 4096) ks *= 2;
   if (J <= 16)
-    launch_stream_ks<kXCols, kOutJI, 1>(args, blocks, ks, stream);
+    launch_stream_ks<kXCols, kOutJI, 1>(args, vec, blocks, ks, stream);
   else
-    launch_stream_ks<kXCols, kOutJI, 2>(args, blocks, ks, stream);
+    launch_stream_ks<kXCols, kOutJI, 2>(args, vec, blocks, ks, stream);
   return check(hipGetLastError(), "gemm_f32 streaming launch");
 }
 

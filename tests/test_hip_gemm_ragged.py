@@ -1,0 +1,139 @@
+"""Matrix products whose rows are not 16-byte: K or N no multiple of four, or
+operands off a 16-byte boundary, on every kernel that takes them. The bar is
+the matmul bar against float64; infinities in neighbouring rows and columns
+must not leak into an output that does not use them."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from conftest import require_gpu
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def capi():
+    require_gpu()
+    import tensorcx_hip_capi
+    return tensorcx_hip_capi
+
+
+def shifted(capi, array, shift):
+    """A device copy that starts `shift` floats past an aligned address."""
+    store = capi.DeviceArray.from_numpy(np.concatenate([np.full(shift, np.nan, np.float32), array.reshape(-1)]))
+    return store, store.ptr + 4 * shift
+
+
+def product(capi, a, b, trans, bias=None, shift=0, workspace=False):
+    batch = a.shape[:-2]
+    m, k = a.shape[-2:]
+    n = b.shape[-2] if trans else b.shape[-1]
+    held_a, pa = shifted(capi, a, shift)
+    held_b, pb = shifted(capi, b, shift)
+    out = capi.DeviceArray((shift + int(np.prod(batch, dtype=np.int64)) * m * n + 8,))
+    capi.check(capi.lib().tcx_hip_fill(0, out.ptr, out.size, -7.0, capi.stream()), "fill")
+    held_bias = capi.DeviceArray.from_numpy(bias) if bias is not None else None
+    desc = capi.gemm_desc(m, n, k, batch_shape=batch, lhs_batch_strides=(m * k,) * len(batch),
+                          rhs_batch_strides=(k * n,) * len(batch), rhs_transposed=trans,
+                          bias=held_bias.ptr if held_bias is not None else None)
+    ws = capi.gemm_workspace(desc) if workspace else None
+    capi.gemm(pa, pb, out.ptr + 4 * shift, desc, workspace=ws)
+    capi.synchronize()
+    got = out.numpy()
+    assert (got[:shift] == -7.0).all() and (got[-8:] == -7.0).all()  # nothing outside the output
+    return got[shift:-8].reshape(batch + (m, n))
+
+
+def reference(a, b, trans, bias):
+    with np.errstate(all="ignore"):
+        y = a.astype(np.float64) @ (np.swapaxes(b, -1, -2) if trans else b).astype(np.float64)
+    return y if bias is None else y + bias
+
+
+def check(capi, m, n, k, trans, *, batch=(), shift=0, workspace=False, leak=True):
+    rng = np.random.default_rng(m * 7 + n * 3 + k)
+    a = rng.standard_normal(batch + (m, k)).astype(np.float32)
+    b = rng.standard_normal(batch + ((n, k) if trans else (k, n))).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float32)
+    what = f"{batch} {m}x{n}x{k} trans={trans} shift={shift}"
+    got = product(capi, a, b, trans, bias, shift, workspace)
+    error = np.abs(got - reference(a, b, trans, bias)).max()
+    assert error <= 1e-4 * np.sqrt(k), f"{what}: {error}"
+    if not leak or m < 3 or n < 3:
+        return
+    # A row of A and a row of W (a column of B) of infinities and NaN.
+    a[..., 1, :] = np.inf
+    if trans:
+        b[..., 1, :] = np.nan
+    else:
+        b[..., :, 0] = np.inf
+        b[..., :, n - 1] = np.nan
+    got = product(capi, a, b, trans, bias, shift, workspace)
+    clean = np.ones((m, n), bool)
+    clean[1] = False
+    if trans:
+        clean[:, 1] = False
+    else:
+        clean[:, 0] = clean[:, n - 1] = False
+    expected = reference(a, b, trans, bias)
+    error = np.abs(got[..., clean] - expected[..., clean]).max()
+    assert error <= 1e-4 * np.sqrt(k), f"{what} next to infinities: {error}"
+    assert not np.isfinite(got[..., ~clean]).any(), what
+
+
+@pytest.mark.parametrize("trans", [False, True])
+@pytest.mark.parametrize("k", [5, 6, 7, 63, 65, 66, 67, 127, 129, 191, 194, 255, 321])
+def test_direct_tiles(capi, trans, k):
+    """64x64 tiles (9 x 15 of them): k tiles of 64 cut at every remainder, from
+    one to six of them; and the 32x64 tiles of a short last round."""
+    check(capi, 130, 261, k, trans, batch=(9,))
+    check(capi, 130, 261, k, trans, batch=(19,), leak=False)
+
+
+@pytest.mark.parametrize("trans", [False, True])
+@pytest.mark.parametrize("n", [705, 706, 707, 708, 641])
+@pytest.mark.parametrize("k", [128, 130])
+def test_direct_columns(capi, trans, n, k):
+    check(capi, 700, n, k, trans)
+
+
+@pytest.mark.parametrize("trans", [False, True])
+def test_direct_many_tiles(capi, trans):
+    check(capi, 2050, 2049, 70, trans)
+    check(capi, 2050, 2048, 71, trans, leak=False)
+    check(capi, 1030, 1027, 4099, trans, workspace=True, leak=False)  # padded copies in the workspace
+
+
+@pytest.mark.parametrize("trans", [False, True])
+@pytest.mark.parametrize("m,n", [(64, 64), (33, 65), (97, 31), (142, 321), (200, 2), (5, 7), (40, 33), (64, 129)])
+@pytest.mark.parametrize("k", [5, 17, 30, 225, 739, 1030])
+def test_small_tiles(capi, trans, m, n, k):
+    check(capi, m, n, k, trans)
+
+
+@pytest.mark.parametrize("m", [2, 3, 16, 17, 32])
+@pytest.mark.parametrize("k", [6, 61, 65, 707, 2049, 4098])
+def test_skinny(capi, m, k):
+    """At most 32 rows of A against W, and at most 32 columns of B."""
+    for n in (256, 438, 5001):
+        check(capi, m, n, k, True)
+    check(capi, 300, m, k, False)
+    check(capi, 300, m, k, True)
+
+
+@pytest.mark.parametrize("k", [64, 65, 255, 1025, 3245, 9999])
+def test_vectors(capi, k):
+    for n in (1, 3, 264, 1001):
+        check(capi, 1, n, k, True, leak=False)
+    check(capi, 517, 1, k, False, leak=False)
+    check(capi, 1, 37, k, True, batch=(5,), leak=False)
+
+
+@pytest.mark.parametrize("shift", [1, 2, 3])
+@pytest.mark.parametrize("trans", [False, True])
+def test_unaligned_operands(capi, trans, shift):
+    """Sizes of 16-byte rows at addresses between them."""
+    for m, n, k in ((700, 704, 128), (64, 64, 256), (16, 512, 1024), (1, 300, 512), (1100, 1100, 260)):
+        check(capi, m, n, k, trans, shift=shift, leak=False)
