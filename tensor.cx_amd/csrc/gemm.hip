@@ -124,7 +124,8 @@ bool full_rounds_128(std::int64_t m, std::int64_t n, std::int64_t batches) {
 // Measured on MI355X, padded against ragged 64x64 tiles: 4096 x 4095 x 4096 1064
 // against 1253 us, 8191 x 2047 x 300 135 / 154, 4096 x 4096 x 525 200 / 225; but
 // without full rounds 2048 x 2049 x 2048 242 / 204, 3000 x 3001 x 1000 237 / 205,
-// 3441 x 4096 x 525 transposed 240 / 183. Around 10^9 multiply-adds the copies
+// 3441 x 4096 x 525 transposed 240 / 183: those leave the workspace that the
+// query offers unused. Around 10^9 multiply-adds the copies
 // and three extra launches cost more than they bring.
 constexpr std::int64_t kPadMinWork = std::int64_t{1} << 32;
 constexpr std::int64_t kPadAlign = 64;  // floats: 256-byte aligned regions
@@ -136,9 +137,7 @@ struct PadPlan {
 
 PadPlan pad_plan(const tcx_hip_gemm_desc_t* d) {
   PadPlan p{false, 0, 0, 0, 0, 0};
-  if (d->batch_rank != 0 || (d->k % 4 == 0 && d->n % 4 == 0) || d->m * d->n * d->k < kPadMinWork ||
-      !full_rounds_128(d->m, d->n, 1))
-    return p;
+  if (d->batch_rank != 0 || (d->k % 4 == 0 && d->n % 4 == 0) || d->m * d->n * d->k < kPadMinWork) return p;
   auto up = [](std::int64_t v, std::int64_t q) { return (v + q - 1) / q * q; };
   p.pad = true;
   p.k4 = up(d->k, 4);
@@ -228,7 +227,7 @@ extern "C" int tcx_hip_gemm_f32_ws(const float* lhs, const float* rhs, float* ou
   for (int i = 0; i < d->batch_rank; ++i) batches *= d->batch_shape[i];
   if (batches != d->batch_count) return fail(TCX_INVALID_ARGUMENT, "gemm batch_count mismatch");
   if (d->m == 0 || d->n == 0 || batches == 0) return TCX_OK;
-  if (const PadPlan pad = pad_plan(d); pad.pad && d->k > 0 && lhs != nullptr && rhs != nullptr && out != nullptr &&
+  if (const PadPlan pad = pad_plan(d); pad.pad && full_rounds_128(d->m, d->n, 1) && d->k > 0 && lhs != nullptr && rhs != nullptr && out != nullptr &&
       workspace != nullptr && aligned16(workspace) &&
       workspace_bytes >= static_cast<size_t>(pad.a_floats + pad.b_floats + pad.c_floats) * sizeof(float)) {
     const int status = ready();
