@@ -316,6 +316,10 @@ int tcx_hip_gather_strided(int elem_bytes, const void* in, void* out, int32_t ra
  * input copied into out at out[o * out_block + dst_offset + j]. */
 int tcx_hip_copy_blocks(int elem_bytes, const void* in, void* out, int64_t outer, int64_t block, int64_t out_block,
                         int64_t dst_offset, tcx_stream_t stream);
+/* kConcat whole (cpu_backend.cpp:317-339): `count` contiguous [outer, blocks[i]]
+ * inputs side by side in out [outer, sum of blocks], up to eight in a launch. */
+int tcx_hip_concat(int elem_bytes, const void* const* in, const int64_t* blocks, int32_t count, void* out, int64_t outer,
+                   tcx_stream_t stream);
 /* kCast (cpu_backend.cpp:834-876) between TCX_FLOAT32 / TCX_INT32 / TCX_BOOL:
  * to/from bool tests value != 0; float32 -> int32 truncates toward zero after
  * every value was checked finite and inside [-2^31, 2^31) (else

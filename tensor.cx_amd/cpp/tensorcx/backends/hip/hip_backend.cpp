@@ -1082,17 +1082,17 @@ Tensor concat(const OpDesc& op, std::span<const Tensor> inputs, Stream& s) {
   const ConcatPlan plan = make_concat_plan(shapes, op.axis);
   Tensor out = make_tensor(inputs[0].dtype, plan.output_shape);
   if (numel(plan.output_shape) == 0) return out;
-  const Dim out_block = plan.output_shape[plan.axis] * plan.inner;
   Dim outer = 1;
   for (std::size_t a = 0; a < plan.axis; ++a) outer *= plan.output_shape[a];
-  Dim offset = 0;
+  std::vector<const void*> sources;
+  std::vector<std::int64_t> blocks;
   for (const Tensor& t : inputs) {
-    const Dim block = t.shape[plan.axis] * plan.inner;
-    ok_or_throw(tcx_hip_copy_blocks(element_bytes(t.dtype), device_ptr(t), out_ptr(out), outer, block, out_block,
-                                    offset, s),
-                "HIP concat");
-    offset += block;
+    sources.push_back(device_ptr(t));
+    blocks.push_back(t.shape[plan.axis] * plan.inner);
   }
+  ok_or_throw(tcx_hip_concat(element_bytes(inputs[0].dtype), sources.data(), blocks.data(),
+                             static_cast<int32_t>(inputs.size()), out_ptr(out), outer, s),
+              "HIP concat");
   return out;
 }
 

@@ -56,6 +56,42 @@ int refuse_forked() { return fail(TCX_UNAVAILABLE, "HIP requires a fresh process
 
 int ready() { return tcx_hip_init(); }
 
+namespace {
+std::mutex flags_mutex;
+// Flags not in use; as many exist as calls have ever run at once. Never
+// destroyed, like the retired blocks below.
+std::vector<std::int32_t*>& free_flags() {
+  static auto* flags = new std::vector<std::int32_t*>;
+  return *flags;
+}
+}  // namespace
+
+std::int32_t* acquire_host_flag() {
+  {
+    std::lock_guard lock(flags_mutex);
+    if (!free_flags().empty()) {
+      std::int32_t* const flag = free_flags().back();
+      free_flags().pop_back();
+      return flag;
+    }
+  }
+  void* flag = nullptr;
+  if (hipHostMalloc(&flag, sizeof(std::int32_t), hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  return static_cast<std::int32_t*>(flag);
+}
+
+void release_host_flag(std::int32_t* flag) {
+  try {
+    std::lock_guard lock(flags_mutex);
+    free_flags().push_back(flag);
+  } catch (...) {
+    (void)hipHostFree(flag);
+  }
+}
+
 }  // namespace tcx
 
 // ------------------------------------------------------------ bounded pool
