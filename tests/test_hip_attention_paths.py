@@ -125,6 +125,31 @@ def test_masks(cx, d, rows, cols, causal, kind):
 
 @pytest.mark.parametrize("d", [32, 64, 128])
 @pytest.mark.parametrize("kind", ["bool", "additive"])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("rows", [40, 130])
+def test_hidden_ends(cx, d, kind, causal, rows):
+    """Key masks that hide whole tiles in front and behind, all keys, or all but
+    one; values there that are not finite show as NaN all the same. The few
+    queries of 16 matrices also split the keys."""
+    cols = 700
+    q, k, v = f32((8, 2, rows, d), 32), f32((8, 2, cols, d), 33), f32((8, 2, cols, d), 34)
+    shown = np.zeros((8, 1, 1, cols), bool)
+    for b, (first, end) in enumerate([(0, 700), (0, 31), (0, 64), (0, 65), (300, 500), (699, 700), (0, 0), (95, 97)]):
+        shown[b, 0, 0, first:end] = True
+    shown[4, 0, 0, 350:400] = False
+    mask = shown if kind == "bool" else np.where(shown, np.float32(0.5), np.float32(-np.inf))
+    check(cx, q, k, v, mask, causal)
+    v[1, 0, 699, 3] = np.nan
+    v[1, 1, 33, 4] = np.inf
+    v[4, 0, 0, 5] = -np.inf
+    v[4, 1, 550, 6] = np.nan
+    v[5, 0, 10, 7] = np.inf
+    v[6, 1, 640, 8] = np.nan
+    check(cx, q, k, v, mask, causal)
+
+
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("kind", ["bool", "additive"])
 def test_mask_special_values(cx, d, kind):
     rng = np.random.default_rng(3)
     q, k, v = f32((2, 90, d), 14), f32((2, 110, d), 15), f32((2, 110, d), 16)
