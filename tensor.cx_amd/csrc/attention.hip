@@ -955,25 +955,31 @@ FlashPlan flash_plan(std::int64_t batch, std::int64_t rows, std::int64_t cols, s
     // at D = 128 64 KB of LDS, so that two blocks share a CU, under causal
     // masking a heavy and a light one (89 TFLOP/s at 16 x 2048 x 128 against
     // 86 for a register-staged 4-wave kernel, 92 against 71 at 32 x 2048 x 64).
-    // Unmasked at D = 64 and 128 also eight waves and 64-key tiles (one block
-    // per CU): 281 against 291 us at 16 x 2048 x 128, but 78 against 53 at 16 x
-    // 1024 x 64, where its blocks are too few; at D = 32 94 against 90 TFLOP/s
-    // for the small tiles. Up to 16 queries one wave holds them all: 60 us
-    // against 81 for 512 matrices of 16 queries and 512 keys at D = 128.
-    const int d = features == 128 ? 2 : features == 64 ? 1 : 0;
+    // At D = 32 and 64 also 64-key tiles, with half the barriers and softmax
+    // chains and half the blocks a CU (16 x 1024 x 64 53 -> 47 us, x 32 36 -> 30,
+    // causal 32 x 512 x 64 31.2 -> 27.9, 160 x 320 x 64 40.7 -> 36.8); with 1024
+    // causal blocks and more, 32 keys stay ahead (32 x 2048 x 64 170 against
+    // 184). Unmasked at D = 128
+    // eight waves and 64-key tiles, one block per CU, where there are enough
+    // (16 x 2048 281 against 291 us). Up to 16 queries one wave holds them all:
+    // 60 us against 81 for 512 matrices of 16 queries and 512 keys at D = 128.
     static constexpr FlashForm kFour[] = {{4, 32, 1.0, 0.8, 5}, {4, 32, 1.53, 1.27, 4}, {4, 32, 2.65, 2.27, 2}};
-    static constexpr FlashForm kEight[] = {{}, {8, 64, 4.6, 4.6, 1}, {8, 64, 8.7, 8.7, 1}};
+    static constexpr FlashForm kLong[] = {{4, 64, 1.64, 1.25, 4}, {4, 64, 2.71, 2.35, 2}}, kEight128{8, 64, 8.7, 8.7, 1};
     static constexpr FlashForm kOne[] = {{1, 32, 1.0, 0.4, 8}, {1, 32, 1.7, 0.6, 5}, {1, 32, 2.85, 1.9, 2}};
+    const int d = features == 128 ? 2 : features == 64 ? 1 : 0;
     const bool plain = !causal && mask_kind == TCX_MASK_NONE;
     FlashForm form = plain && rows <= 16 ? kOne[d] : kFour[d];
     double time = best_split(form, batch, rows, cols, features, causal, p.splits);
-    if (plain && rows > 64 && features >= 64) {
+    auto consider = [&](const FlashForm& other) {
       std::int64_t splits;
-      if (best_split(kEight[d], batch, rows, cols, features, false, splits) < time) {
-        form = kEight[d];
-        p.splits = splits;
-      }
-    }
+      const double t = best_split(other, batch, rows, cols, features, causal, splits);
+      if (t >= time) return;
+      time = t;
+      form = other;
+      p.splits = splits;
+    };
+    if (features <= 64 && form.waves == 4 && (!causal || ceil_div(rows, 64) * batch < 1024)) consider(kLong[d]);
+    if (features == 128 && plain && rows > 64) consider(kEight128);
     p.waves = form.waves;
     p.keys = form.keys;
     p.split_keys = std::max<std::int64_t>(ceil_div(ceil_div(cols, p.keys), p.splits), 1) * p.keys;
@@ -1022,21 +1028,33 @@ int launch_decode(const FlashArgs& a, hipStream_t s) {
   return check(hipGetLastError(), "decode attention launch");
 }
 
+template <int D, bool kCausal, int kMask>
+int launch_tiles(const FlashArgs& a, const FlashPlan& p, hipStream_t s) {
+  constexpr bool kPlain = !kCausal && kMask == TCX_MASK_NONE;
+  if constexpr (kPlain) {
+    if (p.waves == 1) return launch_flash<D, 1, 32, false, TCX_MASK_NONE>(a, s);
+  }
+  if constexpr (kPlain && D == 128) {
+    if (p.waves == 8) return launch_flash<D, 8, 64, false, TCX_MASK_NONE>(a, s);
+  }
+  if constexpr (D <= 64) {
+    if (p.keys == 64) return launch_flash<D, 4, 64, kCausal, kMask>(a, s);
+  }
+  return launch_flash<D, 4, 32, kCausal, kMask>(a, s);
+}
+
 template <int D, bool kCausal>
-int launch_masked(const FlashArgs& a, hipStream_t s) {
-  if (a.mask_kind == TCX_MASK_BOOL) return launch_flash<D, 4, 32, kCausal, TCX_MASK_BOOL>(a, s);
-  return launch_flash<D, 4, 32, kCausal, TCX_MASK_ADDITIVE>(a, s);
+int launch_mask_kind(const FlashArgs& a, const FlashPlan& p, hipStream_t s) {
+  if (a.mask_kind == TCX_MASK_BOOL) return launch_tiles<D, kCausal, TCX_MASK_BOOL>(a, p, s);
+  if (a.mask_kind == TCX_MASK_ADDITIVE) return launch_tiles<D, kCausal, TCX_MASK_ADDITIVE>(a, p, s);
+  return launch_tiles<D, kCausal, TCX_MASK_NONE>(a, p, s);
 }
 
 template <int D>
 int launch_features(const FlashArgs& a, const FlashPlan& p, hipStream_t s) {
-  int rc;
-  if (p.decode) rc = launch_decode<D>(a, s);
-  else if (a.mask_kind != TCX_MASK_NONE) rc = a.causal ? launch_masked<D, true>(a, s) : launch_masked<D, false>(a, s);
-  else if (a.causal) rc = launch_flash<D, 4, 32, true, TCX_MASK_NONE>(a, s);
-  else if (p.waves == 1) rc = launch_flash<D, 1, 32, false, TCX_MASK_NONE>(a, s);
-  else if (D == 32 || p.waves == 4) rc = launch_flash<D, 4, 32, false, TCX_MASK_NONE>(a, s);
-  else rc = launch_flash<D >= 64 ? D : 64, 8, 64, false, TCX_MASK_NONE>(a, s);
+  const int rc = p.decode   ? launch_decode<D>(a, s)
+                 : a.causal ? launch_mask_kind<D, true>(a, p, s)
+                            : launch_mask_kind<D, false>(a, p, s);
   if (rc != TCX_OK || a.splits == 1) return rc;
   hipLaunchKernelGGL((flash_combine_kernel<D>), dim3(grid_for(a.batch * a.rows, 4, kStrideBlocks)), dim3(256), 0, s, a);
   return check(hipGetLastError(), "attention combine launch");

@@ -78,6 +78,15 @@ def test_few_queries_many_batch_matrices(cx):
     check(cx, q, k, v)
 
 
+@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("rows,cols", [(64, 64), (65, 63), (130, 129), (200, 320), (256, 191)])
+def test_both_tile_lengths(cx, d, causal, rows, cols):
+    """32- and 64-key tiles: causal calls of 1024 blocks and more, and few."""
+    for batch in (5, 520):
+        check(cx, f32((batch, rows, d), 35), f32((batch, cols, d), 36), f32((batch, cols, d), 37), None, causal)
+
+
 # (batch matrices, rows, cols): one wave for up to 16 queries; four or eight
 # waves, whole or split, with splits that end in the middle of a key tile and
 # causal parts that are empty.
