@@ -959,10 +959,10 @@ FlashPlan flash_plan(std::int64_t batch, std::int64_t rows, std::int64_t cols, s
     // chains and half the blocks a CU (16 x 1024 x 64 53 -> 47 us, x 32 36 -> 30,
     // causal 32 x 512 x 64 31.2 -> 27.9, 160 x 320 x 64 40.7 -> 36.8); with 1024
     // causal blocks and more, 32 keys stay ahead (32 x 2048 x 64 170 against
-    // 184). Unmasked at D = 128
-    // eight waves and 64-key tiles, one block per CU, where there are enough
-    // (16 x 2048 281 against 291 us). Up to 16 queries one wave holds them all:
-    // 60 us against 81 for 512 matrices of 16 queries and 512 keys at D = 128.
+    // 184). Unmasked at D = 128 eight waves and 64-key tiles, one block per CU,
+    // where there are enough (16 x 2048 281 against 291 us). Up to 16 queries
+    // one wave holds them all: 60 us against 81 for 512 matrices of 16 queries
+    // and 512 keys at D = 128.
     static constexpr FlashForm kFour[] = {{4, 32, 1.0, 0.8, 5}, {4, 32, 1.53, 1.27, 4}, {4, 32, 2.65, 2.27, 2}};
     static constexpr FlashForm kLong[] = {{4, 64, 1.64, 1.25, 4}, {4, 64, 2.71, 2.35, 2}}, kEight128{8, 64, 8.7, 8.7, 1};
     static constexpr FlashForm kOne[] = {{1, 32, 1.0, 0.4, 8}, {1, 32, 1.7, 0.6, 5}, {1, 32, 2.85, 1.9, 2}};
