@@ -459,8 +459,11 @@ int tcx_hip_flash_attention_f32(const float* q, const float* k, const float* v, 
                                 int64_t rows, int64_t cols, int64_t features, float scale, int causal,
                                 tcx_stream_t stream);
 
+/* 1 when tcx_hip_flash_attention_f32_ws handles these feature sizes
+ * (features == value_features, a multiple of 8 from 16 to 128), else 0. */
+int tcx_hip_flash_attention_ws_supported(int64_t features, int64_t value_features);
 typedef struct {
-  int64_t batch, rows, cols, features; /* as for tcx_hip_flash_attention_f32 */
+  int64_t batch, rows, cols, features; /* as for tcx_hip_flash_attention_f32, more sizes */
   float scale;
   int32_t causal;
   int32_t mask_kind; /* TCX_MASK_* */

@@ -87,6 +87,38 @@ def test_both_tile_lengths(cx, d, causal, rows, cols):
         check(cx, f32((batch, rows, d), 35), f32((batch, cols, d), 36), f32((batch, cols, d), 37), None, causal)
 
 
+# Padded kernels: multiples of eight features, the first and last of each
+# kernel's range among them; 8, 66 and 136 keep the unfused route.
+@pytest.mark.parametrize("d", [16, 24, 40, 56, 72, 80, 120, 8, 66, 136])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("batch,rows,cols", [(3, 1, 700), (3, 4, 33), (2, 37, 1500), (5, 130, 129), (300, 64, 64)])
+def test_padded_features(cx, d, causal, batch, rows, cols):
+    q, k, v = f32((batch, rows, d), 41), f32((batch, cols, d), 42), f32((batch, cols, d), 43)
+    check(cx, q, k, v, None, causal)
+    rng = np.random.default_rng(d)
+    for kind in ("bool", "additive"):
+        mask = masks(kind, (batch, 1, cols), rng)
+        mask[..., cols // 2:] = False if kind == "bool" else -np.inf
+        check(cx, q, k, v, mask, causal)
+
+
+@pytest.mark.parametrize("d", [16, 48, 80])
+@pytest.mark.parametrize("rows", [2, 70])
+def test_padded_features_special_values(cx, d, rows):
+    """Infinities in the first chunk (which padding lanes read) and the last."""
+    q, k, v = f32((4, rows, d), 44), f32((4, 900, d), 45), f32((4, 900, d), 46)
+    k[0, 5, 0] = np.inf
+    k[1, 800, d - 1] = -np.inf
+    v[2, 850, 0] = np.inf
+    v[3, 3, d - 1] = np.nan
+    q[3, 1, 0] = np.inf
+    for causal in (False, True):
+        check(cx, q, k, v, None, causal)
+    mask = np.ones((4, 1, 900), dtype=bool)
+    mask[:, :, 600:] = False
+    check(cx, q, k, v, mask)
+
+
 # (batch matrices, rows, cols): one wave for up to 16 queries; four or eight
 # waves, whole or split, with splits that end in the middle of a key tile and
 # causal parts that are empty.
