@@ -128,8 +128,9 @@ __device__ __forceinline__ float exp_attention_exact(float x) {
 }
 
 // K/V tiles are loaded straight into LDS (buffer_load ... lds) and the loop
-// is pipelined so that matrix cores stay busy through the softmax: while the scores of key tile j go through the softmax (VALU), the
-// same wave's MFMAs already compute the scores of tile j + 1. K therefore runs
+// is pipelined so that matrix cores stay busy through the softmax: while the
+// scores of key tile j go through the softmax (VALU), the same wave's MFMAs
+// already compute the scores of tile j + 1. K therefore runs
 // one tile ahead of V: iteration j reads K tile j + 1 and V tile j, and loads
 // K tile j + 2 and V tile j + 1 into the other halves of two-stage buffers,
 // with one barrier per tile. Rows are unpadded and their 16-byte chunks
@@ -683,8 +684,8 @@ __device__ __forceinline__ void flash_store(const FlashArgs& a, const int* bad_c
 
 // One block per query tile and split of the keys.
 template <int D, int kWaves, int kKeys, bool kCausal, int kMask, bool kPad>
-__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWaves == 1 ? 1 : 2, 8))) void flash_attention_kernel(
-    FlashArgs a) {
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWaves == 1 ? 1 : 2, 8))) void
+flash_attention_kernel(FlashArgs a) {
   constexpr int kQTile = 16 * kWaves;
   __shared__ float ks[2][kKeys * D];
   __shared__ float vs[2][kKeys * D];
@@ -1068,7 +1069,9 @@ FlashPlan flash_plan(std::int64_t batch, std::int64_t rows, std::int64_t cols, s
       form = other;
       p.splits = splits;
     };
-    if (!padded && mask_kind == TCX_MASK_NONE && features <= 64 && form.waves == 4 && (!causal || ceil_div(rows, 64) * batch < 1024)) consider(kLong[d]);
+    if (!padded && mask_kind == TCX_MASK_NONE && features <= 64 && form.waves == 4 &&
+        (!causal || ceil_div(rows, 64) * batch < 1024))
+      consider(kLong[d]);
     if (d == 2 && plain && rows > 64) consider(kEight128);
     p.waves = form.waves;
     p.keys = form.keys;

@@ -227,7 +227,8 @@ extern "C" int tcx_hip_gemm_f32_ws(const float* lhs, const float* rhs, float* ou
   for (int i = 0; i < d->batch_rank; ++i) batches *= d->batch_shape[i];
   if (batches != d->batch_count) return fail(TCX_INVALID_ARGUMENT, "gemm batch_count mismatch");
   if (d->m == 0 || d->n == 0 || batches == 0) return TCX_OK;
-  if (const PadPlan pad = pad_plan(d); pad.pad && full_rounds_128(d->m, d->n, 1) && d->k > 0 && lhs != nullptr && rhs != nullptr && out != nullptr &&
+  if (const PadPlan pad = pad_plan(d); pad.pad && full_rounds_128(d->m, d->n, 1) && d->k > 0 &&
+      lhs != nullptr && rhs != nullptr && out != nullptr &&
       workspace != nullptr && aligned16(workspace) &&
       workspace_bytes >= static_cast<size_t>(pad.a_floats + pad.b_floats + pad.c_floats) * sizeof(float)) {
     const int status = ready();
