@@ -33,7 +33,8 @@ __global__ __launch_bounds__(256) void embedding_check_kernel(const std::int32_t
 
 // Rows of `width` units T (16 bytes, or one word), checked and copied in one
 // pass: a block takes 256 units of a row (blockIdx.x) and strides over the rows,
-// so that no index is divided. Out-of-range rows are never read.
+// so that no index is divided; where the grid is too short for a row (2^28
+// units), it strides over the columns as well. Out-of-range rows are never read.
 template <typename T>
 __global__ __launch_bounds__(256) void embedding_kernel(const std::int32_t* __restrict__ indices,
                                                         const T* __restrict__ weight, T* __restrict__ out,
@@ -41,15 +42,18 @@ __global__ __launch_bounds__(256) void embedding_kernel(const std::int32_t* __re
                                                         int per_block, std::int32_t* __restrict__ flag) {
   // Narrow rows share a block: per_block of them, 256 / per_block lanes each.
   const int lanes = 256 / per_block, sub = threadIdx.x / lanes;
-  const std::int64_t c = static_cast<std::int64_t>(blockIdx.x) * lanes + threadIdx.x % lanes;
-  if (c >= width) return;
+  const std::int64_t first = static_cast<std::int64_t>(blockIdx.x) * lanes + threadIdx.x % lanes;
+  const std::int64_t step = static_cast<std::int64_t>(gridDim.x) * lanes;
   for (std::int64_t i = static_cast<std::int64_t>(blockIdx.y) * per_block + sub; i < count;
        i += static_cast<std::int64_t>(gridDim.y) * per_block) {
     const std::int32_t id = indices[i];
-    T v{};
-    if (id >= 0 && id < vocabulary) v = weight[id * width + c];
-    else flag_bad(flag);
-    out[i * width + c] = v;
+    const bool in = id >= 0 && id < vocabulary;
+    if (!in) flag_bad(flag);
+    for (std::int64_t c = first; c < width; c += step) {
+      T v{};
+      if (in) v = weight[id * width + c];
+      out[i * width + c] = v;
+    }
   }
 }
 

@@ -95,3 +95,26 @@ def test_embedding_many_rows(cx):
     ids[1_100_001] = 50
     with pytest.raises(ValueError):
         cx.embedding(cx.tensor(ids, device="hip"), h)
+
+
+def test_embedding_row_wider_than_the_grid():
+    """A table of one row of 2^28 + 5 words (its grid covers 2^28): the last
+    columns are copied too."""
+    require_gpu()
+    import ctypes
+
+    import tensorcx_hip_capi as capi
+    lib, vp, i64 = capi.lib(), ctypes.c_void_p, ctypes.c_int64
+    width, marks = (1 << 28) + 5, np.arange(1, 17, dtype=np.float32)
+    table, out, flag = (capi.DeviceBuffer(4 * n) for n in (width, width, 1))
+    capi.check(lib.tcx_hip_fill(0, table.ptr, width, 2.0, capi.stream()), "fill")
+    capi.check(lib.tcx_hip_fill(0, out.ptr, width, -7.0, capi.stream()), "fill")
+    tail = 4 * (width - marks.size)
+    capi.check(lib.tcx_hip_memcpy_h2d(table.address + tail, marks.ctypes.data, marks.nbytes, capi.stream()), "h2d")
+    ids = capi.DeviceArray.from_numpy(np.zeros(1, np.int32))
+    capi.check(lib.tcx_hip_embedding_f32(vp(ids.ptr), table.ptr, out.ptr, i64(1), i64(1), i64(width), flag.ptr,
+                                         vp(capi.stream())), "embedding")
+    got = np.empty_like(marks)
+    for start, expected in ((tail, marks), (0, np.full(16, 2, np.float32)), (tail // 8 * 4, np.full(16, 2, np.float32))):
+        capi.check(lib.tcx_hip_memcpy_d2h(got.ctypes.data, out.address + start, got.nbytes, capi.stream()), "d2h")
+        np.testing.assert_array_equal(got, expected)
