@@ -11,23 +11,24 @@
 // Short rows with few elements asked for take a wave each (topk_wave_kernel).
 // Otherwise a block works on one row at a time:
 //   * rows of at most kThreads elements: every element is a candidate;
+//   * k = 1, or 2 in 256 threads: a pass for each (select_rounds);
 //   * k <= kThreads / 4: each thread takes the largest key of its share of the
 //     row. The lower bound T of the k-th key is the smallest, over the waves,
 //     of a wave's ceil(k / waves)-th largest thread maximum: at least k keys
 //     are >= T. A second pass over the row collects the keys >= T, a few
 //     times k of them for values in no special order;
-//   * otherwise, or when more than kCandidates keys are >= T (long runs of
-//     equal values): a radix selection of the k-th key, 8 bits a pass, and a
-//     compaction in index order.
+//   * otherwise, or when too many keys are >= T (long runs of equal values,
+//     ordered rows): a radix selection of the k-th key, 8 bits a pass, and a
+//     compaction in index order, or for k <= kFewK a pass for each.
 // Candidates in LDS are put in order by counting, for each, those before it:
 // no barriers, and the counts of one candidate are shared by several lanes.
 //
 // What bounds it: the row is read once from HBM and once more from L2 (the
 // selection reads nothing else), so a row costs two passes at the rate that
-// one CU draws: 100 us for 1024 rows of 50257 with k = 40. With a workspace,
-// fewer rows than CUs are cut into parts (launch_topk_parts): 21 us for 32 rows
+// one CU draws: 66 us for 1024 rows of 50257 with k = 50. With a workspace,
+// fewer rows than CUs are cut into parts (launch_topk_parts): 22 us for 32 rows
 // of 128256 with k = 50. One pass over the row for each of the k elements, as
-// before, took 5.84 and 11.40 ms.
+// before, took 5.84 ms (k = 40) and 11.40.
 
 #include <algorithm>
 
@@ -37,6 +38,19 @@ namespace tcx {
 namespace {
 
 constexpr int kCandidates = 1024;  // in LDS: 16 bytes each
+// Few elements asked for have a kernel without the radix selection. It runs
+// select_rounds straight away up to k = kRoundsK, by which it reads the row no
+// more often than the bound and the candidates do, and where more than
+// kRankedFew candidates show that the bound was a poor one: ties, rows that are
+// in order already. There the radix selection (every count in one bin) and the
+// ordering of a thousand candidates cost more than kFewK passes: with k = 1,
+// 1024 equal rows of 50257 took 820 us and take 36, 65536 ordered rows of 1025
+// took 3370 and take 185; with k = 3, 3380 and 529. Ordering more than half of
+// kCandidates also costs more than the radix selection of at most kShort
+// elements.
+constexpr int kFewK = 12, kRankedFew = 256, kShort = 4096;
+template <int kThreads>
+constexpr int kRoundsK = kThreads == 256 ? 2 : 1;
 
 struct TopkArgs {
   const std::uint32_t* x;
@@ -359,8 +373,56 @@ __device__ void select_span(TopkShared<kThreads>& s, const TopkArgs& a, const To
   else sort_output<kThreads, kFp>(a, span.values, span.indices);
 }
 
+// k rounds over the row for few k, each for the first element after the one
+// before, whatever the values are.
 template <int kThreads, bool kFp, bool kParts>
-__global__ __launch_bounds__(kThreads) void topk_kernel(TopkArgs a) {
+__device__ void select_rounds(TopkShared<kThreads>& s, const TopkArgs& a, const TopkSpan& span) {
+  constexpr int kWaves = kThreads / kWave;
+  const bool largest = a.largest != 0;
+  const int t = threadIdx.x, k = static_cast<int>(span.k);
+  std::uint64_t last = 0;
+  for (int j = 0; j < k; ++j) {
+    std::uint64_t best = 0;  // below every element's place
+    scan_row<kThreads>(span.x, span.n, a.inner, [&](std::uint32_t w, std::int64_t i) {
+      const std::uint64_t place = place_of(topk_key<kFp>(w, largest), span.first + i);
+      if ((j == 0 || place < last) && place > best) best = place;
+    });
+#pragma unroll
+    for (int offset = 32; offset > 0; offset >>= 1) {
+      const std::uint64_t other = __shfl_xor(static_cast<unsigned long long>(best), offset, kWave);
+      best = other > best ? other : best;
+    }
+    __syncthreads();  // the previous round's maxima have been read
+    if ((t & 63) == 0) s.place[t >> 6] = best;
+    __syncthreads();
+    for (int v = 0; v < kWaves; ++v) best = s.place[v] > best ? s.place[v] : best;
+    last = best;
+    if (t == 0) {
+      if constexpr (kParts) {
+        span.places[j] = best;
+      } else {
+        const std::int32_t index = index_of(best);
+        const std::uint32_t word = span.x[index * a.inner];
+        if (a.sorted) {
+          span.values[j * a.inner] = word;
+          span.indices[j * a.inner] = index;
+        } else {  // emit_by_index takes them behind the waves' maxima
+          s.place[kWaves + j] = best;
+          s.word[kWaves + j] = word;
+          s.chosen[j] = kWaves + j;
+        }
+      }
+    }
+  }
+  if (kParts || a.sorted) return;
+  __syncthreads();
+  emit_by_index<kThreads>(s, a, span);
+}
+
+// kFew: k <= kFewK.
+template <int kThreads, bool kFp, bool kParts, bool kFew>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kThreads == 256 && kFew ? 5 : 4, 8))) void
+topk_kernel(TopkArgs a) {
   constexpr int kWaves = kThreads / kWave;
   __shared__ TopkShared<kThreads> s;
   const bool largest = a.largest != 0;
@@ -391,9 +453,16 @@ __global__ __launch_bounds__(kThreads) void topk_kernel(TopkArgs a) {
       emit_candidates<kThreads, kParts>(s, a, span, static_cast<int>(span.n));
       continue;
     }
-    if (span.k > kThreads / 4) {
-      select_span<kThreads, kFp, kParts>(s, a, span);
-      continue;
+    if constexpr (kFew) {
+      if (span.k <= kRoundsK<kThreads>) {
+        select_rounds<kThreads, kFp, kParts>(s, a, span);
+        continue;
+      }
+    } else {
+      if (span.k > kThreads / 4) {
+        select_span<kThreads, kFp, kParts>(s, a, span);
+        continue;
+      }
     }
     std::uint32_t best = 0;
     scan_row<kThreads>(span.x, span.n, a.inner, [&](std::uint32_t w, std::int64_t) {
@@ -417,7 +486,9 @@ __global__ __launch_bounds__(kThreads) void topk_kernel(TopkArgs a) {
       }
     });
     __syncthreads();
-    if (s.count <= kCandidates) emit_candidates<kThreads, kParts>(s, a, span, static_cast<int>(s.count));
+    if (s.count <= (kFew ? kRankedFew : span.n <= kShort ? kCandidates / 2 : kCandidates))
+      emit_candidates<kThreads, kParts>(s, a, span, static_cast<int>(s.count));
+    else if constexpr (kFew) select_rounds<kThreads, kFp, kParts>(s, a, span);
     else select_span<kThreads, kFp, kParts>(s, a, span);
   }
 }
@@ -529,8 +600,9 @@ void launch_topk_wave(const TopkArgs& a, hipStream_t s) {
 template <int kThreads, bool kFp>
 void launch_topk(const TopkArgs& a, hipStream_t s) {
   const std::int64_t cap = kMaxLaunchWorkItems / kThreads;
-  hipLaunchKernelGGL((topk_kernel<kThreads, kFp, false>), dim3(static_cast<unsigned>(a.rows < cap ? a.rows : cap)),
-                     dim3(kThreads), 0, s, a);
+  const dim3 grid(static_cast<unsigned>(a.rows < cap ? a.rows : cap));
+  if (a.k <= kFewK) hipLaunchKernelGGL((topk_kernel<kThreads, kFp, false, true>), grid, dim3(kThreads), 0, s, a);
+  else hipLaunchKernelGGL((topk_kernel<kThreads, kFp, false, false>), grid, dim3(kThreads), 0, s, a);
 }
 
 // The number of parts to cut a row into (1: whole). Fewer rows than the 256 CUs
@@ -545,21 +617,27 @@ std::int64_t topk_parts(std::int64_t rows, std::int64_t reduce, std::int64_t k) 
 // CU reads; one row of 128256 20 against 29 us.
 template <bool kFp>
 void launch_topk_parts(const TopkArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL((topk_kernel<1024, kFp, true>), dim3(static_cast<unsigned>(a.rows * a.parts)), dim3(1024), 0, s, a);
+  const dim3 grid(static_cast<unsigned>(a.rows * a.parts));
+  if (a.k <= kFewK) hipLaunchKernelGGL((topk_kernel<1024, kFp, true, true>), grid, dim3(1024), 0, s, a);
+  else hipLaunchKernelGGL((topk_kernel<1024, kFp, true, false>), grid, dim3(1024), 0, s, a);
   hipLaunchKernelGGL(topk_join_kernel, dim3(static_cast<unsigned>(a.rows)), dim3(1024), 0, s, a);
 }
 
 // A wave a row up to kWaveRow elements and k = kWaveK: with k = 1, 14.7 us for
 // 65536 rows of 32 and 5.4 us for 4096 rows of 1000, against 144 and 22.7 us
-// with a block a row. Else 1024 threads where a row is long enough to keep them
-// reading, or where 256 would send k to the radix selection.
+// with a block a row. Else 256 threads, of which a CU holds four or five blocks
+// (1024 rows of 50257 with k = 3 64 us, with 1024 threads 98; 8192 rows of 8193
+// 90 and 322; 1024 rows of 8193 16 and 42), and 1024 where one row has a CU to
+// itself and is long enough to keep them reading (one row of 50257 17 us,
+// of 1000000 148; with 256 threads 22 and 306; 255 rows of 50257 the same), or
+// where 256 would send k to the radix selection.
 template <bool kFp>
 void launch_topk_rows(const TopkArgs& a, hipStream_t s) {
   if (a.reduce <= kWaveRow && a.k <= kWaveK) {
     if (a.reduce <= 64) launch_topk_wave<1, kFp>(a, s);
     else if (a.reduce <= 256) launch_topk_wave<4, kFp>(a, s);
     else launch_topk_wave<16, kFp>(a, s);
-  } else if (a.reduce > 8192 || (a.reduce > 256 && a.k > 64)) {
+  } else if ((a.reduce > 20000 && a.rows < 256) || (a.reduce > 256 && a.k > 64)) {
     launch_topk<1024, kFp>(a, s);
   } else {
     launch_topk<256, kFp>(a, s);

@@ -101,3 +101,41 @@ def test_more_rows_than_one_per_compute_unit(cx):
     rng = np.random.default_rng(7)
     check(cx, values_of("special", (3000, 70), rng), -1, 5, True, True)
     check(cx, values_of("ties", (700, 1100), rng), -1, 20, True, False)
+
+
+# Up to 12 elements: k = 1 (and 2 in 256 threads) in passes, more of them when
+# many candidates pass the bound, from rows in one block of 256 or 1024 threads
+# and in parts; 13 leave that kernel. 255 rows of 20001 take 1024 threads.
+@pytest.mark.parametrize("kind", ["special", "equal", "ordered", "int32"])
+@pytest.mark.parametrize("rows,n", [(5, 257), (300, 1025), (255, 20001), (256, 20001), (3, 16389)])
+def test_few_elements(cx, rows, n, kind):
+    rng = np.random.default_rng(n)
+    x = np.sort(values_of("special", (rows, n), rng), axis=-1) if kind == "ordered" else values_of(kind, (rows, n), rng)
+    for k in (1, 2, 3, 12, 13):
+        check(cx, x, -1, k, True, True)
+        check(cx, x, -1, k, False, False)
+
+
+@pytest.mark.parametrize("k", [1, 3])
+def test_ordered_rows_take_little_longer(k):
+    """Rows in order pass every bound: they took 14 times as long as rows in no
+    order (now at most twice)."""
+    require_gpu()
+    import ctypes
+
+    import tensorcx_hip_capi as capi
+    i64, rows, n = ctypes.c_int64, 4096, 1025
+    values, indices = capi.DeviceArray((rows, k)), capi.DeviceArray((rows, k), np.int32)
+    start, end, took = capi.Event(), capi.Event(), []
+    for x in (np.random.default_rng(1).standard_normal((rows, n), np.float32), np.tile(np.arange(n, dtype=np.float32), (rows, 1))):
+        held, best = capi.DeviceArray.from_numpy(x), np.inf
+        for _ in range(5):
+            start.record()
+            for _ in range(10):
+                capi.check(capi.lib().tcx_hip_topk(0, *(ctypes.c_void_p(t.ptr) for t in (held, values, indices)), i64(rows),
+                                                   i64(n), i64(1), i64(k), 1, 1, ctypes.c_void_p(capi.stream())), "topk")
+            end.record()
+            end.synchronize()
+            best = min(best, start.elapsed_ms(end))
+        took.append(best)
+    assert took[1] < 5 * took[0], took
