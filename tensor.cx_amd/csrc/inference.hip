@@ -32,27 +32,42 @@ __global__ __launch_bounds__(256) void embedding_check_kernel(const std::int32_t
 }
 
 // Rows of `width` units T (16 bytes, or one word), checked and copied in one
-// pass: a block takes 256 units of a row (blockIdx.x) and strides over the rows,
-// so that no index is divided; where the grid is too short for a row (2^28
-// units), it strides over the columns as well. Out-of-range rows are never read.
-template <typename T>
+// pass: a block takes up to 256 units of a row (blockIdx.x), or several narrow
+// rows, and strides over the rows, so that no index is divided; where the grid
+// is too short for a row (2^28 units), it strides over the columns as well. A
+// thread takes kEach rows at a time, their loads ahead of their stores: four
+// where there are enough of them (a call on 10^6 rows of 36 floats 50 us with
+// one, 32 with four). Out-of-range rows are never read.
+template <typename T, int kEach>
 __global__ __launch_bounds__(256) void embedding_kernel(const std::int32_t* __restrict__ indices,
                                                         const T* __restrict__ weight, T* __restrict__ out,
                                                         std::int64_t count, std::int64_t vocabulary, std::int64_t width,
-                                                        int per_block, std::int32_t* __restrict__ flag) {
-  // Narrow rows share a block: per_block of them, 256 / per_block lanes each.
-  const int lanes = 256 / per_block, sub = threadIdx.x / lanes;
+                                                        int lanes, int per_block, std::int32_t* __restrict__ flag) {
+  const int sub = threadIdx.x / lanes;
+  if (sub >= per_block) return;
   const std::int64_t first = static_cast<std::int64_t>(blockIdx.x) * lanes + threadIdx.x % lanes;
-  const std::int64_t step = static_cast<std::int64_t>(gridDim.x) * lanes;
-  for (std::int64_t i = static_cast<std::int64_t>(blockIdx.y) * per_block + sub; i < count;
-       i += static_cast<std::int64_t>(gridDim.y) * per_block) {
-    const std::int32_t id = indices[i];
-    const bool in = id >= 0 && id < vocabulary;
-    if (!in) flag_bad(flag);
-    for (std::int64_t c = first; c < width; c += step) {
-      T v{};
-      if (in) v = weight[id * width + c];
-      out[i * width + c] = v;
+  const std::int64_t column_step = static_cast<std::int64_t>(gridDim.x) * lanes;
+  const std::int64_t row_step = static_cast<std::int64_t>(gridDim.y) * per_block;
+  for (std::int64_t i = static_cast<std::int64_t>(blockIdx.y) * per_block + sub; i < count; i += kEach * row_step) {
+    std::int32_t id[kEach];
+    bool in[kEach];
+#pragma unroll
+    for (int u = 0; u < kEach; ++u) id[u] = indices[std::min(i + u * row_step, count - 1)];
+#pragma unroll
+    for (int u = 0; u < kEach; ++u) {
+      in[u] = id[u] >= 0 && id[u] < vocabulary;
+      if (!in[u]) flag_bad(flag);
+    }
+    for (std::int64_t c = first; c < width; c += column_step) {
+      T v[kEach];
+#pragma unroll
+      for (int u = 0; u < kEach; ++u) {
+        v[u] = T{};
+        if (in[u]) v[u] = weight[id[u] * width + c];
+      }
+#pragma unroll
+      for (int u = 0; u < kEach; ++u)
+        if (i + u * row_step < count) out[(i + u * row_step) * width + c] = v[u];
     }
   }
 }
@@ -60,12 +75,59 @@ __global__ __launch_bounds__(256) void embedding_kernel(const std::int32_t* __re
 template <typename T>
 void launch_embedding(const std::int32_t* indices, const float* weight, float* out, std::int64_t count,
                       std::int64_t vocabulary, std::int64_t width, std::int32_t* flag, hipStream_t s) {
-  int per_block = 1;
-  while (per_block < 16 && width * per_block * 2 <= 256) per_block *= 2;
-  const unsigned gx = grid_for(width, 256 / per_block, 1 << 20);
-  const unsigned gy = grid_for(count, per_block, std::min<std::int64_t>(65535, std::max<std::int64_t>(1, (1 << 20) / gx)));
-  hipLaunchKernelGGL((embedding_kernel<T>), dim3(gx, gy), dim3(256), 0, s, indices, reinterpret_cast<const T*>(weight),
-                     reinterpret_cast<T*>(out), count, vocabulary, width, per_block, flag);
+  const int lanes = static_cast<int>(std::min<std::int64_t>(width, 256)), per_block = 256 / lanes;
+  const unsigned gx = grid_for(width, lanes, 1 << 20);
+  auto go = [&](auto kernel, int each) {
+    const unsigned gy =
+        grid_for(count, per_block * each, std::min<std::int64_t>(65535, std::max<std::int64_t>(1, (1 << 20) / gx)));
+    hipLaunchKernelGGL(kernel, dim3(gx, gy), dim3(256), 0, s, indices, reinterpret_cast<const T*>(weight),
+                       reinterpret_cast<T*>(out), count, vocabulary, width, lanes, per_block, flag);
+  };
+  // Four rows a thread from 2048 blocks of them on.
+  if (grid_for(count, 4 * per_block) * gx >= 2048) go(embedding_kernel<T, 4>, 4);
+  else go(embedding_kernel<T, 1>, 1);
+}
+
+// The same by words where rows have no 16-byte units: a flat index over the
+// output, so that stores are whole lines wherever the rows start (10^6 rows of
+// 129 words 407 us by rows, 33 words 103).
+template <int kEach>
+__global__ __launch_bounds__(256) void embedding_words_kernel(const std::int32_t* __restrict__ indices,
+                                                              const std::uint32_t* __restrict__ weight,
+                                                              std::uint32_t* __restrict__ out, std::uint32_t n,
+                                                              std::int64_t vocabulary, FastDiv width,
+                                                              std::int32_t* __restrict__ flag) {
+  const std::uint32_t first = blockIdx.x * (256U * kEach) + threadIdx.x;
+  std::uint32_t column[kEach], v[kEach];
+  std::int32_t id[kEach];
+#pragma unroll
+  for (int u = 0; u < kEach; ++u) {
+    const std::uint32_t e = min(first + 256U * u, n - 1), i = width(e);
+    column[u] = e - i * width.divisor;
+    id[u] = indices[i];
+  }
+#pragma unroll
+  for (int u = 0; u < kEach; ++u) {
+    const bool in = id[u] >= 0 && id[u] < vocabulary;
+    if (!in) flag_bad(flag);
+    v[u] = 0;
+    if (in) v[u] = weight[static_cast<std::int64_t>(id[u]) * width.divisor + column[u]];
+  }
+#pragma unroll
+  for (int u = 0; u < kEach; ++u)
+    if (first + 256U * u < n) out[first + 256U * u] = v[u];
+}
+
+void launch_embedding_words(const std::int32_t* indices, const float* weight, float* out, std::int64_t count,
+                            std::int64_t vocabulary, std::int64_t width, std::int32_t* flag, hipStream_t s) {
+  const std::int64_t n = count * width;
+  auto go = [&](auto kernel, int each) {
+    hipLaunchKernelGGL(kernel, dim3(grid_for(n, 256 * each, 1 << 23)), dim3(256), 0, s, indices,
+                       reinterpret_cast<const std::uint32_t*>(weight), reinterpret_cast<std::uint32_t*>(out),
+                       static_cast<std::uint32_t>(n), vocabulary, FastDiv(static_cast<std::uint32_t>(width)), flag);
+  };
+  if (n >= 256 * 1024) go(embedding_words_kernel<4>, 4);
+  else go(embedding_words_kernel<1>, 1);
 }
 
 struct SoftmaxMeta {
@@ -162,6 +224,8 @@ int tcx_hip_embedding_f32(const int32_t* indices, const float* weight, float* ou
                          vocabulary, where);
     else if (width % 4 == 0 && ((at(weight) | at(out)) & 15U) == 0)
       launch_embedding<float4_t>(indices, weight, out, count, vocabulary, width / 4, where, s);
+    else if (count < (std::int64_t{1} << 31) / width)  // FastDiv's range
+      launch_embedding_words(indices, weight, out, count, vocabulary, width, where, s);
     else
       launch_embedding<std::uint32_t>(indices, weight, out, count, vocabulary, width, where, s);
     if (int rc = check(hipGetLastError(), "embedding launch"); rc != TCX_OK) return rc;

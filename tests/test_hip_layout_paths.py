@@ -97,15 +97,16 @@ def test_embedding_many_rows(cx):
         cx.embedding(cx.tensor(ids, device="hip"), h)
 
 
-def test_embedding_row_wider_than_the_grid():
-    """A table of one row of 2^28 + 5 words (its grid covers 2^28): the last
-    columns are copied too."""
+@pytest.mark.parametrize("width", [(1 << 28) + 5, (1 << 30) + 8])
+def test_embedding_row_wider_than_the_grid(width):
+    """A table of one row of more than 2^28 units, words or 16 bytes (the grid
+    of whole rows covers 2^28): the last columns are copied too."""
     require_gpu()
     import ctypes
 
     import tensorcx_hip_capi as capi
     lib, vp, i64 = capi.lib(), ctypes.c_void_p, ctypes.c_int64
-    width, marks = (1 << 28) + 5, np.arange(1, 17, dtype=np.float32)
+    marks = np.arange(1, 17, dtype=np.float32)
     table, out, flag = (capi.DeviceBuffer(4 * n) for n in (width, width, 1))
     capi.check(lib.tcx_hip_fill(0, table.ptr, width, 2.0, capi.stream()), "fill")
     capi.check(lib.tcx_hip_fill(0, out.ptr, width, -7.0, capi.stream()), "fill")
@@ -115,6 +116,20 @@ def test_embedding_row_wider_than_the_grid():
     capi.check(lib.tcx_hip_embedding_f32(vp(ids.ptr), table.ptr, out.ptr, i64(1), i64(1), i64(width), flag.ptr,
                                          vp(capi.stream())), "embedding")
     got = np.empty_like(marks)
-    for start, expected in ((tail, marks), (0, np.full(16, 2, np.float32)), (tail // 8 * 4, np.full(16, 2, np.float32))):
+    for start, expected in ((tail, marks), (0, np.full(16, 2, np.float32)), (tail // 32 * 16, np.full(16, 2, np.float32))):
         capi.check(lib.tcx_hip_memcpy_d2h(got.ctypes.data, out.address + start, got.nbytes, capi.stream()), "d2h")
         np.testing.assert_array_equal(got, expected)
+
+
+# Rows by 16 bytes and by words, one and four of them a thread, in blocks that
+# they do not fill.
+@pytest.mark.parametrize("count,width", [(257, 1), (300_001, 1), (100_003, 3), (70_001, 5), (1023, 255), (1030, 257),
+                                         (700_001, 4), (600_001, 12), (2049, 1032), (5000, 1036)])
+def test_embedding_packed_rows(cx, count, width):
+    rng = np.random.default_rng(count)
+    table, ids = values((19, width), "float32"), rng.integers(0, 19, count).astype(np.int32)
+    h = cx.tensor(table, device="hip")
+    same(cx.embedding(cx.tensor(ids, device="hip"), h).numpy(), table[ids], f"{count} {width}")
+    ids[count - 2] = 19
+    with pytest.raises(ValueError):
+        cx.embedding(cx.tensor(ids, device="hip"), h)
