@@ -88,10 +88,11 @@ void tcx_hip_release(void* ptr, size_t bytes, tcx_hip_pool_t* owner);
  * that was exposed to another framework (DLPack export, copies included) may
  * still be read by work on streams this library cannot see (the reference's
  * exported-buffer rule, bindings/dlpack.cpp:204-206 and cuda_buffer.h:35). The
- * block is freed, which waits for the device, or kept (at most 16 blocks and
- * 512 MiB in all) for an allocation of the same size that waits for the device
- * first; blocks kept are freed when device memory runs out and when any pool
- * is trimmed or left. */
+ * block is freed, which waits for the device; or an active pool keeps it apart
+ * for an allocation of the same size, which waits for the device first. Blocks
+ * kept so count towards the pool's limits beside the cached ones (not in its
+ * cached_bytes and cached_blocks), are freed to make room for those, and are
+ * given back with them: on trim, exit, and when device memory runs out. */
 void tcx_hip_release_uncached(void* ptr, size_t bytes, tcx_hip_pool_t* owner);
 
 /* Checks memory handed over by another framework before a tensor borrows it

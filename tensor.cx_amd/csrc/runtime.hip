@@ -6,7 +6,6 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <iterator>
 #include <mutex>
 #include <new>
 #include <string>
@@ -59,7 +58,7 @@ int ready() { return tcx_hip_init(); }
 namespace {
 std::mutex flags_mutex;
 // Flags not in use; as many exist as calls have ever run at once. Never
-// destroyed, like the retired blocks below.
+// destroyed: at process end the runtime that would free them may be gone already.
 std::vector<std::int32_t*>& free_flags() {
   static auto* flags = new std::vector<std::int32_t*>;
   return *flags;
@@ -95,6 +94,21 @@ void release_host_flag(std::int32_t* flag) {
 }  // namespace tcx
 
 // ------------------------------------------------------------ bounded pool
+
+// Exported storage after its release, kept by the pool it came from. Another
+// framework may still read it by work that is queued on streams this library
+// cannot see, so a block is handed out again only after hipDeviceSynchronize,
+// which hipFree would have made its releaser wait for as well. Mapping and
+// unmapping a result of 2 MiB and more for each exchange cost 40 to 280 us of a
+// call.
+struct Exported {
+  void* ptr;
+  size_t bytes;
+  int device;
+  std::uint64_t number;  // of its release
+  bool idle;             // the device has been waited for since
+};
+
 struct tcx_hip_pool {
   std::mutex mutex;
   std::atomic<long> refs{1};
@@ -102,129 +116,20 @@ struct tcx_hip_pool {
   bool default_runtime{true};
   tcx_hip_pool_stats_t stats{};
   std::vector<std::pair<void*, size_t>> cached;
+  // Exact sizes, the newest last; they count towards the pool's limits beside
+  // the cached blocks and make room for those, the oldest first.
+  std::vector<Exported> exported;
+  size_t exported_bytes{0};
+  std::uint64_t exports{0};  // released so far
   bool used{false};
 };
 
 namespace {
 thread_local tcx_hip_pool* active_pool = nullptr;
 
-// Exported storage after its release. Another framework may still read it by
-// work that is queued on streams this library cannot see, so a block is handed
-// out again only after hipDeviceSynchronize, which hipFree would have made its
-// releaser wait for as well. Mapping and unmapping a result of 2 MiB and more
-// for each exchange cost 40 to 280 us of a call. Exact sizes, the newest first;
-// at most kRetiredBlocks blocks and kRetiredBytes bytes, the oldest freed for a
-// new one; all freed when device memory runs out and when a pool is trimmed or
-// left. One list for all threads: a block belongs to no stream once the device
-// has been waited for.
-struct Retired {
-  void* ptr;
-  size_t bytes;
-  int device;
-  std::uint64_t number;  // of its release
-  bool idle;             // the device has been waited for since
-};
-constexpr size_t kRetiredBlocks = 16, kRetiredBytes = size_t{512} << 20;
-std::mutex retired_mutex;
-std::uint64_t releases = 0;  // under retired_mutex
-
-// Never destroyed: at process end the runtime that would free the blocks may
-// be gone already.
-std::vector<Retired>& retired() {
-  static auto* blocks = new std::vector<Retired>;
-  return *blocks;
-}
-
-void free_retired() {
-  std::vector<Retired> blocks;
-  {
-    std::lock_guard lock(retired_mutex);
-    blocks.swap(retired());
-  }
-  for (const Retired& b : blocks) (void)hipFree(b.ptr);
-}
-
-// Takes a released block over; false where it has to be freed instead.
-bool retire(void* ptr, size_t bytes) noexcept {
-  int device = 0;
-  hipPointerAttribute_t attributes{};
-  if (bytes > kRetiredBytes / 2 || hipGetDevice(&device) != hipSuccess ||
-      hipPointerGetAttributes(&attributes, ptr) != hipSuccess) {
-    (void)hipGetLastError();
-    return false;
-  }
-  if (attributes.device != device) return false;  // another device's work is not waited for here
-  try {
-    std::vector<Retired> old;
-    {
-      std::lock_guard lock(retired_mutex);
-      auto& blocks = retired();
-      size_t held = bytes;
-      for (const Retired& b : blocks) held += b.bytes;
-      size_t drop = 0;
-      while (drop < blocks.size() && (blocks.size() - drop >= kRetiredBlocks || held > kRetiredBytes))
-        held -= blocks[drop++].bytes;
-      old.assign(blocks.begin(), blocks.begin() + static_cast<std::ptrdiff_t>(drop));
-      blocks.reserve(2 * kRetiredBlocks);
-      blocks.erase(blocks.begin(), blocks.begin() + static_cast<std::ptrdiff_t>(drop));
-      blocks.push_back({ptr, bytes, device, ++releases, false});
-    }
-    for (const Retired& b : old) (void)hipFree(b.ptr);
-  } catch (...) {
-    return false;
-  }
-  return true;
-}
-
-// A retired block of this size, once the device has finished all work queued
-// before now; null when there is none (or the device cannot be waited for, as
-// during a stream capture). The wait is outside the lock.
-void* reuse_retired(size_t bytes) {
-  int device = 0;
-  if (hipGetDevice(&device) != hipSuccess) return nullptr;
-  Retired block{};
-  std::uint64_t until = 0;
-  {
-    std::lock_guard lock(retired_mutex);
-    auto& blocks = retired();
-    const auto found = std::find_if(blocks.rbegin(), blocks.rend(),
-                                    [&](const Retired& b) { return b.bytes == bytes && b.device == device; });
-    if (found == blocks.rend()) return nullptr;
-    block = *found;
-    until = releases;
-    blocks.erase(std::next(found).base());
-  }
-  if (block.idle) return block.ptr;
-  const bool waited = hipDeviceSynchronize() == hipSuccess;
-  if (!waited) (void)hipGetLastError();
-  std::lock_guard lock(retired_mutex);
-  if (!waited) {
-    retired().push_back(block);  // the room it left is reserved
-    return nullptr;
-  }
-  for (Retired& b : retired()) b.idle = b.idle || (b.device == device && b.number <= until);
-  return block.ptr;
-}
-
-hipError_t device_malloc(void** ptr, size_t bytes) {
-  if (void* const again = reuse_retired(bytes)) {
-    *ptr = again;
-    return hipSuccess;
-  }
-  hipError_t error = hipMalloc(ptr, bytes);
-  if (error != hipErrorOutOfMemory) return error;
-  {
-    std::lock_guard lock(retired_mutex);
-    if (retired().empty()) return error;
-  }
-  (void)hipGetLastError();
-  free_retired();
-  return hipMalloc(ptr, bytes);
-}
-
 int hip_allocate(void** ptr, size_t bytes) {
   if (tcx::forked()) return tcx::refuse_forked();
-  const hipError_t error = device_malloc(ptr, bytes);
+  const hipError_t error = hipMalloc(ptr, bytes);
   if (error == hipErrorOutOfMemory) {
     tcx::set_error("hipMalloc: out of memory");
     return TCX_POOL_OOM;
@@ -242,31 +147,100 @@ int hip_clear_error() {
 void pool_unref(tcx_hip_pool* pool) {
   if (pool->refs.fetch_sub(1) == 1) {
     for (auto& [ptr, bytes] : pool->cached) pool->runtime.free(ptr);
+    for (const Exported& b : pool->exported) pool->runtime.free(b.ptr);
     delete pool;
   }
 }
 
-// Frees every cached block; keeps going after a failure and reports it.
+// Gives a block back to the runtime; a failure is counted and reported.
+int pool_free_locked(tcx_hip_pool* pool, void* ptr, size_t bytes) {
+  ++pool->stats.free_calls;
+  const int rc = pool->runtime.free(ptr);
+  if (rc != TCX_OK) {
+    ++pool->stats.free_failures;
+    pool->stats.failed_free_bytes += bytes;
+  }
+  return rc;
+}
+
+// True when `bytes` more fit the pool's limits, once the oldest exported blocks
+// have been freed as far as that takes.
+bool pool_room_locked(tcx_hip_pool* pool, size_t bytes) {
+  const auto& s = pool->stats;
+  if (!s.active || pool->cached.size() >= s.max_cached_blocks || bytes > s.max_cached_bytes - s.cached_bytes) return false;
+  while (!pool->exported.empty() && (pool->cached.size() + pool->exported.size() >= s.max_cached_blocks ||
+                                     bytes > s.max_cached_bytes - s.cached_bytes - pool->exported_bytes)) {
+    const Exported oldest = pool->exported.front();
+    pool->exported.erase(pool->exported.begin());
+    pool->exported_bytes -= oldest.bytes;
+    (void)pool_free_locked(pool, oldest.ptr, oldest.bytes);
+  }
+  return true;
+}
+
+// Takes a released exported block over; false where it has to be freed instead.
+bool pool_keep_exported_locked(tcx_hip_pool* pool, void* ptr, size_t bytes) {
+  int device = 0;
+  hipPointerAttribute_t attributes{};
+  if (!pool->default_runtime || !pool_room_locked(pool, bytes)) return false;
+  if (hipGetDevice(&device) != hipSuccess || hipPointerGetAttributes(&attributes, ptr) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  if (attributes.device != device) return false;
+  pool->exported.push_back({ptr, bytes, device, ++pool->exports, false});  // within the room reserved for max_cached_blocks
+  pool->exported_bytes += bytes;
+  return true;
+}
+
+// An exported block of this size, once the device has finished all work queued
+// before now; null when there is none, or when the device cannot be waited for
+// (during a stream capture). The lock is given up for the wait: other threads
+// may release blocks meanwhile, which stay marked as not waited for.
+void* pool_take_exported(tcx_hip_pool* pool, size_t bytes, std::unique_lock<std::mutex>& lock) {
+  auto& blocks = pool->exported;
+  int device = 0;
+  if (blocks.empty() || tcx::forked() || hipGetDevice(&device) != hipSuccess) return nullptr;
+  const auto found = std::find_if(blocks.rbegin(), blocks.rend(),
+                                  [&](const Exported& b) { return b.bytes == bytes && b.device == device; });
+  if (found == blocks.rend()) return nullptr;
+  const std::uint64_t number = found->number, until = pool->exports;
+  if (!found->idle) {
+    // Meanwhile the block stays listed: only this thread, the pool's owner,
+    // takes blocks, but a release on another may free it to make room.
+    lock.unlock();
+    const bool waited = hipDeviceSynchronize() == hipSuccess;
+    if (!waited) (void)hipGetLastError();
+    lock.lock();
+    if (!waited) return nullptr;
+    for (Exported& b : blocks) b.idle = b.idle || (b.device == device && b.number <= until);
+  }
+  // (Freed meanwhile to make room, or with the whole pool.)
+  const auto at = std::find_if(blocks.begin(), blocks.end(), [&](const Exported& b) { return b.number == number; });
+  if (at == blocks.end()) return nullptr;
+  void* const ptr = at->ptr;
+  blocks.erase(at);
+  pool->exported_bytes -= bytes;
+  return ptr;
+}
+
+// Frees every cached and every exported block; keeps going after a failure and reports it.
 int pool_trim_locked(tcx_hip_pool* pool) {
   int status = TCX_OK;
-  for (auto& [ptr, bytes] : pool->cached) {
-    ++pool->stats.free_calls;
-    const int rc = pool->runtime.free(ptr);
-    if (rc != TCX_OK) {
-      ++pool->stats.free_failures;
-      pool->stats.failed_free_bytes += bytes;
-      status = TCX_INTERNAL;
-    }
-  }
+  for (auto& [ptr, bytes] : pool->cached)
+    if (pool_free_locked(pool, ptr, bytes) != TCX_OK) status = TCX_INTERNAL;
+  for (const Exported& b : pool->exported)
+    if (pool_free_locked(pool, b.ptr, b.bytes) != TCX_OK) status = TCX_INTERNAL;
   pool->cached.clear();
+  pool->exported.clear();
+  pool->exported_bytes = 0;
   pool->stats.cached_bytes = 0;
   pool->stats.cached_blocks = 0;
   if (status != TCX_OK) return tcx::fail(status, "HIP pool failed to free cached blocks");
   return TCX_OK;
 }
 
-int pool_allocate(tcx_hip_pool* pool, size_t bytes, void** ptr) {
-  std::lock_guard lock(pool->mutex);
+int pool_allocate_locked(tcx_hip_pool* pool, size_t bytes, void** ptr, std::unique_lock<std::mutex>& lock) {
   if (!pool->stats.active || !bytes)
     return tcx::fail(TCX_INVALID_ARGUMENT, "inactive pool or zero-byte allocation");
   auto found = std::find_if(pool->cached.begin(), pool->cached.end(),
@@ -276,12 +250,17 @@ int pool_allocate(tcx_hip_pool* pool, size_t bytes, void** ptr) {
     pool->cached.erase(found);
     pool->stats.cached_bytes -= bytes;
     ++pool->stats.hits;
+  } else if (void* const again = pool_take_exported(pool, bytes, lock)) {
+    *ptr = again;
+    ++pool->stats.hits;
+  } else if (!pool->stats.active) {  // left while the lock was given up
+    return tcx::fail(TCX_INVALID_ARGUMENT, "inactive pool or zero-byte allocation");
   } else {
     ++pool->stats.misses;
     ++pool->stats.allocation_calls;
     int rc = pool->runtime.allocate(ptr, bytes);
-    if (rc == TCX_POOL_OOM && !pool->cached.empty()) {
-      // Recover only from out-of-memory: drain the cache and retry once.
+    if (rc == TCX_POOL_OOM && !(pool->cached.empty() && pool->exported.empty())) {
+      // Recover only from out-of-memory: drain the pool and retry once.
       const int pending = pool->runtime.clear_error();
       if (pending != TCX_OK && pending != TCX_POOL_OOM) {
         ++pool->stats.allocation_failures;
@@ -304,16 +283,23 @@ int pool_allocate(tcx_hip_pool* pool, size_t bytes, void** ptr) {
   pool->stats.cached_blocks = pool->cached.size();
   pool->stats.in_use_bytes += bytes;
   pool->stats.peak_in_use_bytes = std::max(pool->stats.peak_in_use_bytes, pool->stats.in_use_bytes);
-  pool->refs.fetch_add(1);
   return TCX_OK;
+}
+
+int pool_allocate(tcx_hip_pool* pool, size_t bytes, void** ptr) {
+  pool->refs.fetch_add(1);  // the block's; it also holds the pool while its lock is given up
+  std::unique_lock lock(pool->mutex);
+  const int rc = pool_allocate_locked(pool, bytes, ptr, lock);
+  lock.unlock();
+  if (rc != TCX_OK) pool_unref(pool);
+  return rc;
 }
 
 void pool_release(tcx_hip_pool* pool, void* ptr, size_t bytes, bool allow_cache) {
   {
     std::lock_guard lock(pool->mutex);
     pool->stats.in_use_bytes -= bytes;
-    bool cache = allow_cache && pool->stats.active && pool->cached.size() < pool->stats.max_cached_blocks &&
-                 bytes <= pool->stats.max_cached_bytes - pool->stats.cached_bytes;
+    bool cache = allow_cache && pool_room_locked(pool, bytes);
     if (cache && pool->default_runtime && tcx::thread_stream != nullptr &&
         hipStreamQuery(tcx::thread_stream) != hipSuccess) {
       // Never cache a block that queued work may still touch.
@@ -327,12 +313,7 @@ void pool_release(tcx_hip_pool* pool, void* ptr, size_t bytes, bool allow_cache)
       pool->stats.peak_cached_bytes = std::max(pool->stats.peak_cached_bytes, pool->stats.cached_bytes);
     } else {
       ++pool->stats.uncached_returns;
-      ++pool->stats.free_calls;
-      const bool kept = !allow_cache && pool->default_runtime && retire(ptr, bytes);
-      if (!kept && pool->runtime.free(ptr) != TCX_OK) {
-        ++pool->stats.free_failures;
-        pool->stats.failed_free_bytes += bytes;
-      }
+      if (allow_cache || !pool_keep_exported_locked(pool, ptr, bytes)) (void)pool_free_locked(pool, ptr, bytes);
     }
   }
   pool_unref(pool);
@@ -426,7 +407,7 @@ int tcx_hip_allocate(size_t bytes, void** ptr, tcx_hip_pool_t** owner) {
   }
   const int status = tcx::ready();
   if (status != TCX_OK) return status;
-  return tcx::check(device_malloc(ptr, bytes), "hipMalloc");
+  return tcx::check(hipMalloc(ptr, bytes), "hipMalloc");
 }
 
 void tcx_hip_release(void* ptr, size_t bytes, tcx_hip_pool_t* owner) {
@@ -444,7 +425,7 @@ void tcx_hip_release_uncached(void* ptr, size_t bytes, tcx_hip_pool_t* owner) {
     pool_release(owner, ptr, bytes, false);
     return;
   }
-  if (!retire(ptr, bytes)) (void)hipFree(ptr);
+  (void)hipFree(ptr);
 }
 
 int tcx_hip_borrow_check(const void* ptr, size_t bytes) {
@@ -511,7 +492,8 @@ int tcx_hip_pool_create(size_t max_cached_bytes, size_t max_cached_blocks,
   }
   p->stats.max_cached_bytes = max_cached_bytes;
   p->stats.max_cached_blocks = max_cached_blocks;
-  p->cached.reserve(max_cached_blocks);  // caching a block never allocates host memory
+  p->cached.reserve(max_cached_blocks);  // keeping a block never allocates host memory
+  if (p->default_runtime) p->exported.reserve(max_cached_blocks);
   *pool = p;
   return TCX_OK;
 }
@@ -535,14 +517,12 @@ int tcx_hip_pool_exit(tcx_hip_pool_t* pool) {
   if (active_pool != pool)
     return tcx::fail(TCX_INVALID_ARGUMENT, "memory pool must exit on its owning thread");
   active_pool = nullptr;
-  if (pool->default_runtime) free_retired();
   std::lock_guard lock(pool->mutex);
   pool->stats.active = 0;
   return pool_trim_locked(pool);
 }
 
 int tcx_hip_pool_trim(tcx_hip_pool_t* pool) {
-  if (pool->default_runtime) free_retired();
   std::lock_guard lock(pool->mutex);
   return pool_trim_locked(pool);
 }
