@@ -117,16 +117,6 @@ __device__ __forceinline__ float exp_attention(float x) {
   return __builtin_amdgcn_exp2f(x * kLog2e);
 }
 
-// exp(x) for x <= 0 (or NaN) with the rounding of x log2 e made good: the
-// product's remainder r enters as 2^r = 1 + r ln 2 (x = -inf: 0, r unused).
-__device__ __forceinline__ float exp_attention_exact(float x) {
-  constexpr float kLog2e = 1.44269502F, kLog2eLow = 1.92596299e-8F;  // their sum is log2 e to 49 bits
-  const float h = x * kLog2e;
-  const float r = fmaf(x, kLog2e, -h) + x * kLog2eLow;
-  const float y = __builtin_amdgcn_exp2f(h);
-  return x > -104.F ? fmaf(y, r * 0.693147182F, y) : y;  // past it 0, and r may not be finite
-}
-
 // K/V tiles are loaded straight into LDS (buffer_load ... lds) and the loop
 // is pipelined so that matrix cores stay busy through the softmax: while the
 // scores of key tile j go through the softmax (VALU), the same wave's MFMAs
@@ -219,12 +209,13 @@ __device__ __forceinline__ void flash_segment(const FlashArgs& a, float (&ks)[2]
     }
   }
   mfma_acc (&o)[kT] = st.o;
-  // Masked and padded kernels sum in shorter chains and round the exponent's
-  // argument once less, so that their error against 64 bits is no larger than
-  // that of the two products and the softmax of the unfused route (with one
-  // chain it was up to twice that; now 0.8 of it in the mean, at most 1.01):
-  // the scores in eight accumulators, four at D = 32 (step (t, e) in number
-  // 4t + e), and P V of a tile apart (tile_o).
+  // Masked and padded kernels sum in shorter chains and take expf, so that
+  // their error against 64 bits is no larger than that of the two products and
+  // the softmax of the unfused route (with one chain it was up to twice that;
+  // now 0.70 of it in the mean over 16 to 128 features and 5 to 2048 keys, for
+  // these kernels at most 0.97): the scores in eight accumulators, four at D =
+  // 32 (step (t, e) in number 4t + e), and P V of a tile apart, its steps in
+  // two by turns (tile_o).
   constexpr int kParts = !kExact ? 1 : D >= 64 ? 8 : 4;
   mfma_acc s_part[kParts][kB];
   auto clear_parts = [&] {
@@ -398,7 +389,7 @@ __device__ __forceinline__ void flash_segment(const FlashArgs& a, float (&ks)[2]
       tmax = fmaxf(tmax, xor32(tmax));
       m_new = fmaxf(m, tmax);
       m_sub = m_new == neg_inf ? 0.F : m_new;
-      alpha = kExact ? exp_attention_exact(m - m_sub) : exp_attention(m - m_sub);
+      alpha = kExact ? expf(m - m_sub) : exp_attention(m - m_sub);
     } else if constexpr (I == kB + 1) {
 #pragma unroll
       for (int v = 0; v < 4; ++v)
@@ -410,7 +401,7 @@ __device__ __forceinline__ void flash_segment(const FlashArgs& a, float (&ks)[2]
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const float x = s[I - kB - 2 - kT][v] - m_sub;
-        const float p = kExact ? exp_attention_exact(x) : exp_attention(x);
+        const float p = kExact ? expf(x) : exp_attention(x);
         s[I - kB - 2 - kT][v] = p;
         psum += p;
       }
@@ -429,16 +420,16 @@ __device__ __forceinline__ void flash_segment(const FlashArgs& a, float (&ks)[2]
   // each reading the next step's V operands before its own MFMAs.
   auto accumulate = [&]<int... I>(const float* __restrict__ vt_, const mfma_acc (&p)[kB], float (&vv)[2][kT],
                                   std::integer_sequence<int, I...>) {
-    mfma_acc tile_o[kExact ? kT : 1];
+    mfma_acc tile_o[2][kExact ? kT : 1];
     if constexpr (kExact) {
 #pragma unroll
-      for (int t = 0; t < kT; ++t) tile_o[t] = mfma_acc{0.F, 0.F, 0.F, 0.F};
+      for (int t = 0; t < kT; ++t) tile_o[0][t] = tile_o[1][t] = mfma_acc{0.F, 0.F, 0.F, 0.F};
     }
     auto one = [&]<int J>() {
       if constexpr (J + 1 < 4 * kB) read_v(vt_, J + 1, vv[(J + 1) & 1]);
 #pragma unroll
       for (int t = 0; t < kT; ++t) {
-        mfma_acc& to = kExact ? tile_o[kExact ? t : 0] : o[t];
+        mfma_acc& to = kExact ? tile_o[J & 1][kExact ? t : 0] : o[t];
         to = __builtin_amdgcn_mfma_f32_16x16x4f32(p[J / 4][J % 4], vv[J & 1][t], to, 0, 0, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -446,7 +437,7 @@ __device__ __forceinline__ void flash_segment(const FlashArgs& a, float (&ks)[2]
     (one.template operator()<I>(), ...);
     if constexpr (kExact) {
 #pragma unroll
-      for (int t = 0; t < kT; ++t) o[t] += tile_o[t];
+      for (int t = 0; t < kT; ++t) o[t] += tile_o[0][t] + tile_o[1][t];
     }
   };
 
@@ -776,7 +767,7 @@ template <int N>
 __device__ __forceinline__ void join_state(float& m, float& l, float (&o)[N], float m2, float l2, const float (&o2)[N]) {
   const float top = fmaxf(m, m2);
   const float at = top == -__builtin_inff() ? 0.F : top;
-  const float f = exp_attention(m - at), f2 = exp_attention(m2 - at);
+  const float f = expf(m - at), f2 = expf(m2 - at);
   m = top;
   l = l * f + l2 * f2;
 #pragma unroll
@@ -789,6 +780,8 @@ __device__ __forceinline__ void join_state(float& m, float& l, float (&o)[N], fl
 // each lane kC 16-byte chunks of its rows; kEach keys a group and pass, so that
 // 16 loads a lane are in flight. Every group keeps an online softmax of its own
 // (no exchange between groups in the loop); the groups are joined at the end.
+// The exponentials are expf here, as in the unfused route: the loop is bound by
+// memory, and the sums are as short as to keep the error below that route's too.
 // 32 heads of one query and 4096 keys, D = 128 (134 MB): 24.1 us with the
 // combine (5.6 TB/s), against 537 us for one block of flash_attention_kernel
 // per head.
@@ -870,14 +863,14 @@ __global__ __launch_bounds__(256) void flash_decode_kernel(FlashArgs a) {
         top = fmaxf(top, s[u]);
       }
       const float at = top == neg_inf ? 0.F : top;  // as in flash_segment: every key so far hidden
-      const float f = exp_attention(m[r] - at);
+      const float f = expf(m[r] - at);
       m[r] = top;
       l[r] *= f;
 #pragma unroll
       for (int e = 0; e < 4 * kC; ++e) o[r][e] *= f;
 #pragma unroll
       for (int u = 0; u < kEach; ++u) {
-        const float p = exp_attention(s[u] - at);
+        const float p = expf(s[u] - at);
         l[r] += p;
 #pragma unroll
         for (int c = 0; c < kC; ++c)
@@ -948,7 +941,7 @@ __global__ __launch_bounds__(256) void flash_combine_kernel(FlashArgs a) {
 #pragma unroll
     for (int offset = 32; offset > 0; offset >>= 1) top = fmaxf(top, __shfl_xor(top, offset, kWave));
     const float at = top == neg_inf ? 0.F : top;
-    const float weight = exp_attention(ml.x - at);
+    const float weight = expf(ml.x - at);
     const float sum = wave_sum(ml.y * weight);
     const int d = lane * kE;
     float y[kE] = {};

@@ -266,3 +266,76 @@ def test_without_a_workspace(cx, rows):
     assert_close(out.numpy(), oracle.attention(q, k, v), 2e-4, 2e-5, "no workspace")
     assert lib.tcx_hip_flash_attention_f32_ws(None, None, None, None, None, None, None, ctypes.c_size_t(0),
                                               None) == capi.TCX_INVALID_ARGUMENT
+
+
+# With q = 0 the additive mask holds the scores, exactly: one key at 0, one at
+# -x, the others hidden. The output is then exp(-x) / (1 + exp(-x)): two to four
+# ulp of expf, the sum and the division. Both keys in one tile, and so far apart
+# that the states of lane groups, tiles or splits have to be joined.
+@pytest.mark.parametrize("d", [16, 64, 128])
+@pytest.mark.parametrize("rows", [1, 4, 5, 40])
+@pytest.mark.parametrize("cols", [2, 90, 700, 4100])
+def test_exponentials(cx, d, rows, cols):
+    x = np.linspace(0.3, 87, 48).astype(np.float32)
+    q, k, v = np.zeros((48, rows, d), np.float32), f32((48, cols, d), 47), np.zeros((48, cols, d), np.float32)
+    for first, last in ((0, cols - 1), (cols - 1, 0)):
+        mask = np.full((48, 1, cols), -np.inf, np.float32)
+        mask[:, 0, first], mask[:, 0, last] = 0, -x
+        v[:] = 0
+        v[:, last, 1:] = 1
+        got = cx.attention(*(cx.tensor(t, device="hip") for t in (q, k, v)), cx.tensor(mask, device="hip")).numpy()
+        p = np.exp(-x.astype(np.float64))
+        expected = np.broadcast_to((p / (1 + p))[:, None, None], (48, rows, d - 1))
+        assert np.abs(got[:, :, 1:] / expected - 1).max() <= 8 * 2.0**-24, (first, last)
+        assert not got[:, :, 0].any()
+        # Below the normal numbers a probability is still no zero to an
+        # infinite value, down to the last one that expf gives.
+        mask[:, 0, last] = -np.linspace(87.4, 103, 48).astype(np.float32)
+        v[:, last, 3] = np.inf
+        got = cx.attention(*(cx.tensor(t, device="hip") for t in (q, k, v)), cx.tensor(mask, device="hip")).numpy()
+        assert (got[:, :, 3] == np.inf).all() and np.isfinite(got[:, :, :3]).all()
+
+
+class SoftmaxDesc(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int64 * 8) for n in ("shape", "score_strides", "mask_strides")] + [
+        ("rank", ctypes.c_int32), ("mask_kind", ctypes.c_int32), ("causal", ctypes.c_int32), ("scale", ctypes.c_float)]
+
+
+def unfused(capi, q, k, v, mask, scale):
+    """The two products and the softmax between them."""
+    batch, rows, d = q.shape
+    cols = k.shape[1]
+    dq, dk, dv, dm = (capi.DeviceArray.from_numpy(t) for t in (q, k, v, mask))
+    scores, out = capi.DeviceArray((batch, rows, cols)), capi.DeviceArray(q.shape)
+    capi.gemm(dq.ptr, dk.ptr, scores.ptr, capi.gemm_desc(rows, cols, d, batch_shape=(batch,), lhs_batch_strides=(rows * d,),
+                                                         rhs_batch_strides=(cols * d,), rhs_transposed=True))
+    desc = SoftmaxDesc(rank=3, mask_kind=2, scale=scale)
+    for i, (n, stride) in enumerate(zip(scores.shape, (rows * cols, cols, 1))):
+        desc.shape[i], desc.score_strides[i], desc.mask_strides[i] = n, stride, stride
+    capi.check(capi.lib().tcx_hip_attention_softmax_f32(*(ctypes.c_void_p(t.ptr) for t in (scores, dm, scores)),
+                                                        ctypes.byref(desc), ctypes.c_void_p(capi.stream())), "softmax")
+    capi.gemm(scores.ptr, dv.ptr, out.ptr, capi.gemm_desc(rows, d, cols, batch_shape=(batch,), lhs_batch_strides=(rows * cols,),
+                                                          rhs_batch_strides=(cols * d,)))
+    capi.synchronize()
+    return out.numpy()
+
+
+@pytest.mark.parametrize("d", [16, 32, 48, 64, 80, 128])
+def test_masked_error_against_64_bits(cx, d):
+    """The masked and padded kernels are no less exact than the products and
+    the softmax that they replace: relative errors (2-norm) over at least 25000
+    outputs of each shape, whose ratio one sample moves by 2 % or so."""
+    import tensorcx_hip_capi as capi
+    ratios = []
+    for batch, rows, cols in ((1500, 1, 100), (1500, 1, 700), (500, 3, 300), (100, 16, 200), (50, 40, 128), (20, 130, 600)):
+        rng = np.random.default_rng(rows + cols + d)
+        q, k, v = f32((batch, rows, d), 51), f32((batch, cols, d), 52), f32((batch, cols, d), 53)
+        mask = rng.standard_normal((batch, rows, cols)).astype(np.float32)
+        mask[rng.random(mask.shape) < 0.2] = -np.inf
+        scale = np.float32(1 / np.sqrt(d))
+        s = q.astype(np.float64) @ np.swapaxes(k, 1, 2) * scale + mask
+        p = np.exp(s - s.max(-1, keepdims=True))
+        exact = p / p.sum(-1, keepdims=True) @ v.astype(np.float64)
+        got = cx.attention(*(cx.tensor(t, device="hip") for t in (q, k, v)), cx.tensor(mask, device="hip")).numpy()
+        ratios.append(np.linalg.norm(got - exact) / np.linalg.norm(unfused(capi, q, k, v, mask, scale) - exact))
+    assert max(ratios) <= 1.03 and np.mean(ratios) <= 0.9, ratios
