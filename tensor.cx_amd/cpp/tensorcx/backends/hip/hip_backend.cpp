@@ -945,10 +945,11 @@ Tensor attention(const OpDesc& op, std::span<const Tensor> inputs, Stream& s) {
   for (const Tensor& t : inputs) (void)device_ptr(t);
   if (numel(shape) == 0) return make_tensor(DType::kFloat32, shape);
   // Attention over matching batches with a multiple of eight features from
-  // 16 to 128: the fused kernels, scores never materialised.
+  // 16 to 128: the fused kernels, scores never materialised (their grid holds
+  // 2^24 - 1 tiles of 64 queries of a matrix).
   const Shape qb(q.shape.begin(), q.shape.end() - 2);
   if (qb == Shape(k.shape.begin(), k.shape.end() - 2) && qb == Shape(v.shape.begin(), v.shape.end() - 2) &&
-      tcx_hip_flash_attention_ws_supported(features, v.shape.back()) && aligned16(device_ptr(q)) &&
+      tcx_hip_flash_attention_ws_supported(features, v.shape.back()) && rows <= (Dim{1} << 30) - 64 && aligned16(device_ptr(q)) &&
       aligned16(device_ptr(k)) && aligned16(device_ptr(v))) {
     tcx_hip_flash_attention_desc_t d{};
     d.batch = numel(qb);

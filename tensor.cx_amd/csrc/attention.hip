@@ -50,6 +50,7 @@ struct FlashArgs {
   std::int64_t rows, cols;
   std::int64_t features;       // of a row; the kernels' D where they are not padded
   std::int64_t qtiles, batch;  // work items: qtiles query tiles of each batch matrix
+  std::int64_t first_batch;    // of this launch, in the whole call (for the mask)
   float scale;
   int causal;
   int xcd_blocks;   // group the blocks of one batch matrix on one XCD
@@ -71,6 +72,7 @@ struct FlashArgs {
 // Offset of batch matrix b in the mask (its leading axes, row-major).
 __device__ __forceinline__ std::int64_t mask_offset(const FlashArgs& a, std::int64_t b) {
   std::int64_t offset = 0;
+  b += a.first_batch;
   for (int i = a.mask_rank - 1; i >= 0; --i) {
     offset += b % a.mask_shape[i] * a.mask_stride[i];
     b /= a.mask_shape[i];
@@ -1079,7 +1081,6 @@ template <int D, int kWaves, int kKeys, bool kCausal, int kMask, bool kPad = fal
 int launch_flash(FlashArgs a, hipStream_t s) {
   constexpr int kQTile = 16 * kWaves;
   a.qtiles = ceil_div(a.rows, kQTile);
-  if (a.qtiles > 0x7fffffff / a.batch / a.splits) return fail(TCX_INVALID_ARGUMENT, "attention grid is too large");
   const std::int64_t items = a.qtiles * a.batch;
   const std::int64_t blocks = items * a.splits;
   // Causal blocks keep their heavy/light order instead.
@@ -1106,7 +1107,6 @@ int launch_flash(FlashArgs a, hipStream_t s) {
 
 template <int D, bool kPad>
 int launch_decode(const FlashArgs& a, hipStream_t s) {
-  if (a.batch > 0x7fffffff / a.splits) return fail(TCX_INVALID_ARGUMENT, "attention grid is too large");
   const dim3 grid(static_cast<unsigned>(a.batch * a.splits));
   if (a.rows == 1) hipLaunchKernelGGL((flash_decode_kernel<D, 1, kPad>), grid, dim3(256), 0, s, a);
   else if (a.rows == 2) hipLaunchKernelGGL((flash_decode_kernel<D, 2, kPad>), grid, dim3(256), 0, s, a);
@@ -1215,14 +1215,13 @@ int tcx_hip_flash_attention_f32_ws(const float* q, const float* k, const float* 
     p.split_keys *= p.splits;
     p.splits = 1;
   }
-  a.q = q;
-  a.k = k;
-  a.v = v;
-  a.out = out;
+  // Blocks of one batch matrix, and as many matrices a launch as HIP counts work-items for.
+  const std::int64_t blocks = (p.decode ? 1 : ceil_div(d.rows, 16 * p.waves)) * p.splits;
+  const std::int64_t per_launch = kMaxLaunchWorkItems / (p.decode ? 256 : 64 * p.waves) / blocks;
+  if (per_launch == 0) return fail(TCX_INVALID_ARGUMENT, "attention grid is too large");
   a.rows = d.rows;
   a.cols = d.cols;
   a.features = d.features;
-  a.batch = d.batch;
   a.scale = d.scale;
   a.causal = d.causal != 0;
   a.splits = p.splits;
@@ -1232,12 +1231,25 @@ int tcx_hip_flash_attention_f32_ws(const float* q, const float* k, const float* 
     a.part_ml = a.part + p.splits * d.batch * d.rows * d.features;
   }
   const auto s = static_cast<hipStream_t>(stream);
-  if (d.features == 32) return launch_features<32, false>(a, p, s);
-  if (d.features == 64) return launch_features<64, false>(a, p, s);
-  if (d.features == 128) return launch_features<128, false>(a, p, s);
-  if (d.features < 32) return launch_features<32, true>(a, p, s);
-  if (d.features < 64) return launch_features<64, true>(a, p, s);
-  return launch_features<128, true>(a, p, s);
+  auto launch = [&] {
+    if (d.features == 32) return launch_features<32, false>(a, p, s);
+    if (d.features == 64) return launch_features<64, false>(a, p, s);
+    if (d.features == 128) return launch_features<128, false>(a, p, s);
+    if (d.features < 32) return launch_features<32, true>(a, p, s);
+    if (d.features < 64) return launch_features<64, true>(a, p, s);
+    return launch_features<128, true>(a, p, s);
+  };
+  // (Splits have few matrices: their states are not cut.)
+  for (std::int64_t first = 0; first < d.batch; first += per_launch) {
+    a.first_batch = first;
+    a.batch = std::min(per_launch, d.batch - first);
+    a.q = q + first * d.rows * d.features;
+    a.k = k + first * d.cols * d.features;
+    a.v = v + first * d.cols * d.features;
+    a.out = out + first * d.rows * d.features;
+    if (int rc = launch(); rc != TCX_OK) return rc;
+  }
+  return TCX_OK;
 }
 
 int tcx_hip_flash_attention_f32(const float* q, const float* k, const float* v, float* out, int64_t batch,

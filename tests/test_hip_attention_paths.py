@@ -339,3 +339,33 @@ def test_masked_error_against_64_bits(cx, d):
         got = cx.attention(*(cx.tensor(t, device="hip") for t in (q, k, v)), cx.tensor(mask, device="hip")).numpy()
         ratios.append(np.linalg.norm(got - exact) / np.linalg.norm(unfused(capi, q, k, v, mask, scale) - exact))
     assert max(ratios) <= 1.03 and np.mean(ratios) <= 0.9, ratios
+
+
+@pytest.mark.parametrize("rows", [1, 5])
+def test_more_matrices_than_a_launch_holds(rows):
+    """2^24 + 5 matrices of one key (HIP counts 2^32 work-items a launch), on the
+    streaming and on the matrix kernel; the last ones under the last entries of
+    a mask with an axis of its own for each half of them."""
+    require_gpu()
+    import tensorcx_hip_capi as capi
+    lib, vp, n, tail, d = capi.lib(), ctypes.c_void_p, (1 << 24) + 6, 64, 16
+    q, out = capi.DeviceBuffer(4 * n * rows * d), capi.DeviceBuffer(4 * n * rows * d)
+    k, v, mask = capi.DeviceBuffer(4 * n * d), capi.DeviceBuffer(4 * n * d), capi.DeviceBuffer(n)
+    for t, size, value in ((q, n * rows * d, 1.0), (k, n * d, 1.0), (v, n * d, 2.0), (out, n * rows * d, -7.0)):
+        capi.check(lib.tcx_hip_fill(0, t.ptr, size, value, capi.stream()), "fill")
+    capi.check(lib.tcx_hip_fill(2, mask.ptr, n, 1.0, capi.stream()), "fill")
+    marks, shown = f32((tail, d), 61), np.arange(tail) % 3 != 0
+    for t, host, at in ((v, marks, 4 * (n - tail) * d), (mask, shown.astype(np.uint8), n - tail)):
+        capi.check(lib.tcx_hip_memcpy_h2d(t.address + at, host.ctypes.data, host.nbytes, capi.stream()), "h2d")
+    desc = Desc(batch=n, rows=rows, cols=1, features=d, scale=0.25, mask_kind=1, mask_rank=2, mask_row_stride=0, mask_col_stride=1)
+    desc.mask_shape[0], desc.mask_shape[1], desc.mask_strides[0], desc.mask_strides[1] = 2, n // 2, n // 2, 1
+    capi.check(lib.tcx_hip_flash_attention_f32_ws(q.ptr, k.ptr, v.ptr, out.ptr, mask.ptr, ctypes.byref(desc), None,
+                                                  ctypes.c_size_t(0), vp(capi.stream())), "attention")
+    got = np.empty((tail, rows, d), np.float32)
+    expected = np.repeat(np.where(shown[:, None], marks, np.float32(0))[:, None], rows, 1)
+    for first, want in ((n - tail, expected), (0, np.full_like(got, 2)), ((1 << 24) - tail, np.full_like(got, 2))):
+        capi.check(lib.tcx_hip_memcpy_d2h(got.ctypes.data, out.address + 4 * first * rows * d, got.nbytes, capi.stream()), "d2h")
+        want = want.copy()
+        if first != n - tail and first + tail > n - tail:
+            want[n - tail - first:] = expected[:first + tail - (n - tail)]
+        np.testing.assert_array_equal(got, want)
