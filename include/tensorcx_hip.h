@@ -480,11 +480,22 @@ typedef struct {
  * when there are too few queries to fill the GPU, so that the keys are split
  * over blocks whose states land in the workspace; 0 otherwise. */
 size_t tcx_hip_flash_attention_workspace_bytes(const tcx_hip_flash_attention_desc_t* desc);
+/* How the call would run with a workspace of that many bytes: on the kernel that
+ * streams the keys past few queries (decode) or on the one with matrix
+ * instructions, with `waves` waves a block of 16 queries each, key tiles of
+ * `keys` (decode: 0) and the keys in `splits` parts, whose states take
+ * workspace_bytes (0 for one part). */
+typedef struct {
+  int32_t decode, waves, keys, splits;
+  size_t workspace_bytes;
+} tcx_hip_flash_attention_plan_t;
+int tcx_hip_flash_attention_plan(const tcx_hip_flash_attention_desc_t* desc, size_t workspace_bytes,
+                                 tcx_hip_flash_attention_plan_t* plan);
 /* tcx_hip_flash_attention_f32 with a mask (kAttention's, core/inference.cpp:
  * 123-161: false or -inf hides a key, other additive entries are added to the
- * scaled score) and with that workspace (16-byte aligned; with NULL or fewer
- * bytes than the query it runs unsplit). The workspace must stay allocated
- * until the stream has run the call. */
+ * scaled score) and with that workspace (16-byte aligned; the keys are split
+ * as far as it has room, without one not at all). The workspace must stay
+ * allocated until the stream has run the call. */
 int tcx_hip_flash_attention_f32_ws(const float* q, const float* k, const float* v, float* out, const void* mask,
                                    const tcx_hip_flash_attention_desc_t* desc, void* workspace,
                                    size_t workspace_bytes, tcx_stream_t stream);

@@ -993,20 +993,25 @@ struct FlashForm {
   int resident;  // blocks a CU holds
 };
 
+std::size_t split_bytes(std::int64_t splits, std::int64_t batch, std::int64_t rows, std::int64_t features) {
+  return splits > 1 ? static_cast<std::size_t>(splits * batch * rows) * (features + 2) * sizeof(float) : 0;
+}
+
 // The split of the keys that is expected to end first, with its time in
 // microseconds. A block's time is its tiles on the busiest of 256 CUs and 4 us
 // of start and end a round; a split call also runs the combine (4 us and the
 // states written and read at 4 TB/s). Under causal masking almost half of the
 // parts of a split are empty. Within 15 % of what MI355X took for 20 shapes of
 // 3 to 512 matrices, 5 to 2048 queries and 128 to 4096 keys; a split has to
-// promise 8 %.
+// promise 8 %, and room in the workspace.
 double best_split(const FlashForm& f, std::int64_t batch, std::int64_t rows, std::int64_t cols, std::int64_t features,
-                  bool causal, std::int64_t& splits) {
+                  bool causal, std::size_t limit, std::int64_t& splits) {
   const std::int64_t items = ceil_div(rows, 16 * f.waves) * batch, tiles = std::max<std::int64_t>(ceil_div(cols, f.keys), 1);
   double best = 0;
   splits = 1;
   for (const std::int64_t n : kSplits) {
-    if (n > 1 && (n > tiles || items * n > 2048)) break;
+    const std::size_t bytes = split_bytes(n, batch, rows, features);
+    if (n > 1 && (n > tiles || items * n > 2048 || bytes > limit)) break;
     const std::int64_t per = ceil_div(tiles, n);
     if (n > 1 && ceil_div(tiles, per) != n) continue;  // another count cuts the tiles the same way
     const double blocks = static_cast<double>(causal && n > 1 ? items * (n + 1) : items * n) * (causal && n > 1 ? 0.6 : 1.0);
@@ -1023,7 +1028,7 @@ double best_split(const FlashForm& f, std::int64_t batch, std::int64_t rows, std
 }
 
 FlashPlan flash_plan(std::int64_t batch, std::int64_t rows, std::int64_t cols, std::int64_t features, bool causal,
-                     int mask_kind) {
+                     int mask_kind, std::size_t limit) {
   FlashPlan p{};
   if (rows <= kDecodeRows && !causal && cols > 0) {
     // Up to 256 blocks of at least 128 keys (8 splits of 32 x 4096 x 128 24.1
@@ -1032,7 +1037,8 @@ FlashPlan flash_plan(std::int64_t batch, std::int64_t rows, std::int64_t cols, s
     p.decode = true;
     std::int64_t splits = 1;
     for (const std::int64_t n : kSplits)
-      if (n * batch <= 256 && n * 128 <= cols && cols >= 512) splits = n;
+      if (n * batch <= 256 && n * 128 <= cols && cols >= 512 && split_bytes(n, batch, rows, features) <= limit)
+        splits = n;
     p.split_keys = ceil_div(ceil_div(cols, splits), 64) * 64;
     p.splits = ceil_div(cols, p.split_keys);
   } else {
@@ -1055,10 +1061,10 @@ FlashPlan flash_plan(std::int64_t batch, std::int64_t rows, std::int64_t cols, s
     const int d = features > 64 ? 2 : features > 32 ? 1 : 0;
     const bool padded = features != 32 << d, plain = !padded && !causal && mask_kind == TCX_MASK_NONE;
     FlashForm form = plain && rows <= 16 ? kOne[d] : kFour[d];
-    double time = best_split(form, batch, rows, cols, features, causal, p.splits);
+    double time = best_split(form, batch, rows, cols, features, causal, limit, p.splits);
     auto consider = [&](const FlashForm& other) {
       std::int64_t splits;
-      const double t = best_split(other, batch, rows, cols, features, causal, splits);
+      const double t = best_split(other, batch, rows, cols, features, causal, limit, splits);
       if (t >= time) return;
       time = t;
       form = other;
@@ -1073,7 +1079,7 @@ FlashPlan flash_plan(std::int64_t batch, std::int64_t rows, std::int64_t cols, s
     p.split_keys = std::max<std::int64_t>(ceil_div(ceil_div(cols, p.keys), p.splits), 1) * p.keys;
     p.splits = std::max<std::int64_t>(ceil_div(cols, p.split_keys), 1);
   }
-  if (p.splits > 1) p.bytes = static_cast<std::size_t>(p.splits * batch * rows) * (features + 2) * sizeof(float);
+  p.bytes = split_bytes(p.splits, batch, rows, features);
   return p;
 }
 
@@ -1163,11 +1169,22 @@ int tcx_hip_flash_attention_ws_supported(int64_t features, int64_t value_feature
   return features == value_features && features >= 16 && features <= 128 && features % 8 == 0 ? 1 : 0;
 }
 
-size_t tcx_hip_flash_attention_workspace_bytes(const tcx_hip_flash_attention_desc_t* desc) {
-  if (desc == nullptr || desc->batch <= 0 || desc->rows <= 0 || desc->cols < 0 ||
+int tcx_hip_flash_attention_plan(const tcx_hip_flash_attention_desc_t* desc, size_t workspace_bytes,
+                                 tcx_hip_flash_attention_plan_t* plan) {
+  using namespace tcx;
+  if (desc == nullptr || plan == nullptr) return fail(TCX_INVALID_ARGUMENT, "attention plan or descriptor is null");
+  if (desc->batch <= 0 || desc->rows <= 0 || desc->cols < 0 ||
       !tcx_hip_flash_attention_ws_supported(desc->features, desc->features))
-    return 0;
-  return tcx::flash_plan(desc->batch, desc->rows, desc->cols, desc->features, desc->causal != 0, desc->mask_kind).bytes;
+    return fail(TCX_INVALID_ARGUMENT, "no fused attention for these extents");
+  const FlashPlan p = flash_plan(desc->batch, desc->rows, desc->cols, desc->features, desc->causal != 0,
+                                 desc->mask_kind, workspace_bytes);
+  *plan = {p.decode ? 1 : 0, p.decode ? 4 : p.waves, p.keys, static_cast<std::int32_t>(p.splits), p.bytes};
+  return TCX_OK;
+}
+
+size_t tcx_hip_flash_attention_workspace_bytes(const tcx_hip_flash_attention_desc_t* desc) {
+  tcx_hip_flash_attention_plan_t plan{};
+  return tcx_hip_flash_attention_plan(desc, SIZE_MAX, &plan) == TCX_OK ? plan.workspace_bytes : 0;
 }
 
 int tcx_hip_flash_attention_f32_ws(const float* q, const float* k, const float* v, float* out, const void* mask,
@@ -1208,13 +1225,10 @@ int tcx_hip_flash_attention_f32_ws(const float* q, const float* k, const float* 
     a.mask_col = d.mask_col_stride;
   }
   if (int rc = ready(); rc != TCX_OK) return rc;
-  FlashPlan p = flash_plan(d.batch, d.rows, d.cols, d.features, d.causal != 0, a.mask_kind);
-  if (p.splits > 1 && (workspace == nullptr || workspace_bytes < p.bytes ||
-                       (reinterpret_cast<std::uintptr_t>(workspace) & 15U) != 0)) {
-    // No room for the splits' states: one block takes all keys.
-    p.split_keys *= p.splits;
-    p.splits = 1;
-  }
+  // The best plan that the workspace has room for.
+  const bool usable = workspace != nullptr && (reinterpret_cast<std::uintptr_t>(workspace) & 15U) == 0;
+  const FlashPlan p = flash_plan(d.batch, d.rows, d.cols, d.features, d.causal != 0, a.mask_kind,
+                                 usable ? workspace_bytes : 0);
   // Blocks of one batch matrix, and as many matrices a launch as HIP counts work-items for.
   const std::int64_t blocks = (p.decode ? 1 : ceil_div(d.rows, 16 * p.waves)) * p.splits;
   const std::int64_t per_launch = kMaxLaunchWorkItems / (p.decode ? 256 : 64 * p.waves) / blocks;

@@ -1,0 +1,68 @@
+"""How fused attention would run a call (tcx_hip_flash_attention_plan): the
+kernel, its form and its split of the keys. No kernel runs here."""
+
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+
+import tensorcx_hip_capi as capi
+
+
+class Desc(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int64) for n in ("batch", "rows", "cols", "features")] + [
+        ("scale", ctypes.c_float), ("causal", ctypes.c_int32), ("mask_kind", ctypes.c_int32),
+        ("mask_rank", ctypes.c_int32), ("mask_shape", ctypes.c_int64 * 8), ("mask_strides", ctypes.c_int64 * 8),
+        ("mask_row_stride", ctypes.c_int64), ("mask_col_stride", ctypes.c_int64)]
+
+
+class Plan(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int32) for n in ("decode", "waves", "keys", "splits")] + [
+        ("workspace_bytes", ctypes.c_size_t)]
+
+
+ANY = ctypes.c_size_t(-1).value
+
+
+def plan(batch, rows, cols, features, causal=False, mask=0, limit=ANY):
+    out = Plan()
+    desc = Desc(batch=batch, rows=rows, cols=cols, features=features, causal=int(causal), mask_kind=mask)
+    capi.check(capi.lib().tcx_hip_flash_attention_plan(ctypes.byref(desc), ctypes.c_size_t(limit), ctypes.byref(out)), "plan")
+    return out
+
+
+def test_no_plan_without_a_fused_kernel():
+    assert capi.lib().tcx_hip_flash_attention_plan(None, 0, ctypes.byref(Plan())) == capi.TCX_INVALID_ARGUMENT
+    for shape in ((0, 4, 4, 64), (1, 0, 4, 64), (1, 4, -1, 64), (1, 4, 4, 20)):
+        with pytest.raises(capi.HipError):
+            plan(*shape)
+
+
+@pytest.mark.parametrize("batch,rows,cols,features", [(4, 256, 256, 64), (16, 512, 512, 32), (2, 64, 4096, 128), (32, 1, 4096, 128),
+                                                      (3, 17, 1000, 80), (8, 1024, 1024, 64)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_split_as_far_as_the_workspace_goes(batch, rows, cols, features, causal):
+    """No more splits than the workspace has room for; without one, the form
+    that is best for whole rows of keys, which is the one of a call that no
+    split would help."""
+    full = plan(batch, rows, cols, features, causal)
+    assert (full.workspace_bytes > 0) == (full.splits > 1)
+    assert full.workspace_bytes == (full.splits > 1) * full.splits * batch * rows * (features + 2) * 4
+    for share in (2, 3, 10):
+        part = plan(batch, rows, cols, features, causal, limit=full.workspace_bytes // share)
+        assert part.workspace_bytes <= full.workspace_bytes // share and part.splits <= full.splits
+    none = plan(batch, rows, cols, features, causal, limit=0)
+    assert (none.splits, none.workspace_bytes) == (1, 0)
+
+
+def test_form_without_a_workspace():
+    """8 x 128 queries and 640 keys of 128 features are split over four-wave
+    blocks; whole, as many matrices as fill the CUs take the eight-wave form,
+    with a workspace at hand (which it has no use for) and without."""
+    assert plan(40, 500, 500, 128).waves == plan(40, 500, 500, 128, limit=0).waves == 8
+    assert plan(8, 128, 4096, 128).splits > 1
+    whole, few = plan(8, 128, 4096, 128, limit=0), plan(8, 128, 128, 128, limit=0)
+    assert (whole.waves, whole.keys) == (few.waves, few.keys) == (4, 32)
+    # 2 x 64 x 2048 x 64: eight parts of 32-key tiles, or one of 64-key tiles.
+    assert plan(2, 64, 2048, 64).splits > 1 and plan(2, 64, 2048, 64, limit=0).keys == 64

@@ -369,3 +369,26 @@ def test_more_matrices_than_a_launch_holds(rows):
         if first != n - tail and first + tail > n - tail:
             want[n - tail - first:] = expected[:first + tail - (n - tail)]
         np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("batch,rows,cols,d", [(4, 256, 256, 64), (2, 64, 1500, 128), (8, 1, 2100, 32), (3, 17, 1000, 80)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_workspace_with_room_for_some_splits(cx, batch, rows, cols, d, causal):
+    """The keys are split as far as the workspace goes, and what lies behind it
+    stays as it is."""
+    import tensorcx_hip_capi as capi
+    q, k, v = f32((batch, rows, d), 62), f32((batch, cols, d), 63), f32((batch, cols, d), 64)
+    held = [capi.DeviceArray.from_numpy(t) for t in (q, k, v)]
+    desc = Desc(batch=batch, rows=rows, cols=cols, features=d, scale=d ** -0.5, causal=int(causal))
+    query = capi.lib().tcx_hip_flash_attention_workspace_bytes
+    query.restype = ctypes.c_size_t
+    full, expected = query(ctypes.byref(desc)), oracle.attention(q, k, v, None, causal)
+    for nbytes in {full, full // 2, full // 3, 1000, 0}:
+        out = capi.DeviceArray(q.shape)
+        workspace = capi.DeviceArray.from_numpy(np.full(nbytes // 4 + 64, 99, np.float32))
+        capi.check(capi.lib().tcx_hip_flash_attention_f32_ws(
+            *(ctypes.c_void_p(t.ptr) for t in (*held, out)), None, ctypes.byref(desc), ctypes.c_void_p(workspace.ptr),
+            ctypes.c_size_t(nbytes), ctypes.c_void_p(capi.stream())), "attention")
+        capi.synchronize()
+        assert_close(out.numpy(), expected, 2e-4, 2e-5, f"{nbytes} of {full} bytes")
+        assert (workspace.numpy()[nbytes // 4:] == 99).all()
