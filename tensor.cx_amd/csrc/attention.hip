@@ -1003,7 +1003,8 @@ std::size_t split_bytes(std::int64_t splits, std::int64_t batch, std::int64_t ro
 // states written and read at 4 TB/s). Under causal masking almost half of the
 // parts of a split are empty. Within 15 % of what MI355X took for 20 shapes of
 // 3 to 512 matrices, 5 to 2048 queries and 128 to 4096 keys; a split has to
-// promise 8 %, and room in the workspace.
+// promise 8 %, and room in the workspace. `cols` are the keys that the
+// last query sees.
 double best_split(const FlashForm& f, std::int64_t batch, std::int64_t rows, std::int64_t cols, std::int64_t features,
                   bool causal, std::size_t limit, std::int64_t& splits) {
   const std::int64_t items = ceil_div(rows, 16 * f.waves) * batch, tiles = std::max<std::int64_t>(ceil_div(cols, f.keys), 1);
@@ -1030,6 +1031,7 @@ double best_split(const FlashForm& f, std::int64_t batch, std::int64_t rows, std
 FlashPlan flash_plan(std::int64_t batch, std::int64_t rows, std::int64_t cols, std::int64_t features, bool causal,
                      int mask_kind, std::size_t limit) {
   FlashPlan p{};
+  if (causal) cols = std::min(cols, rows);  // the keys after the last query are not run
   if (rows <= kDecodeRows && !causal && cols > 0) {
     // Up to 256 blocks of at least 128 keys (8 splits of 32 x 4096 x 128 24.1
     // us, 32 splits 25.2, one 91.4); short sequences whole, since the combine

@@ -66,3 +66,14 @@ def test_form_without_a_workspace():
     assert (whole.waves, whole.keys) == (few.waves, few.keys) == (4, 32)
     # 2 x 64 x 2048 x 64: eight parts of 32-key tiles, or one of 64-key tiles.
     assert plan(2, 64, 2048, 64).splits > 1 and plan(2, 64, 2048, 64, limit=0).keys == 64
+
+
+@pytest.mark.parametrize("rows", [1, 5, 40, 64, 200])
+@pytest.mark.parametrize("features", [32, 64, 80, 128])
+@pytest.mark.parametrize("mask", [0, 1])
+def test_causal_plans_for_the_visible_keys(rows, features, mask):
+    """Keys after the last query are not run: they call for no split and no
+    longer tiles (4 x 1 x 2651 x 32 was split over blocks without a key)."""
+    visible, all_keys = plan(8, rows, rows, features, True, mask), plan(8, rows, 8000, features, True, mask)
+    assert all_keys.splits == visible.splits and all_keys.workspace_bytes == visible.workspace_bytes
+    assert rows > 64 or all_keys.splits == 1
