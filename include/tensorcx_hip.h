@@ -484,12 +484,14 @@ size_t tcx_hip_flash_attention_workspace_bytes(const tcx_hip_flash_attention_des
  * streams the keys past few queries (decode) or on the one with matrix
  * instructions, with `waves` waves a block of 16 queries each, key tiles of
  * `keys` (decode: 0) and the keys in `splits` parts, whose states take
- * workspace_bytes (0 for one part). */
+ * workspace_bytes (0 for one part). per_call: the workspace is taken from
+ * tcx_hip_allocate for this one call, so that where this thread has no pool that
+ * keeps it, the split also has to be worth the allocation. */
 typedef struct {
   int32_t decode, waves, keys, splits;
   size_t workspace_bytes;
 } tcx_hip_flash_attention_plan_t;
-int tcx_hip_flash_attention_plan(const tcx_hip_flash_attention_desc_t* desc, size_t workspace_bytes,
+int tcx_hip_flash_attention_plan(const tcx_hip_flash_attention_desc_t* desc, size_t workspace_bytes, int per_call,
                                  tcx_hip_flash_attention_plan_t* plan);
 /* tcx_hip_flash_attention_f32 with a mask (kAttention's, core/inference.cpp:
  * 123-161: false or -inf hides a key, other additive entries are added to the

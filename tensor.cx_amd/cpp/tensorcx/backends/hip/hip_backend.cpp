@@ -980,7 +980,9 @@ Tensor attention(const OpDesc& op, std::span<const Tensor> inputs, Stream& s) {
       // With few queries the keys are split over blocks, their states in a
       // workspace held until the stream has finished (without one, when that
       // allocation fails, the keys stay together).
-      const std::size_t ws = tcx_hip_flash_attention_workspace_bytes(&d);
+      tcx_hip_flash_attention_plan_t split{};
+      ok_or_throw(tcx_hip_flash_attention_plan(&d, SIZE_MAX, 1, &split), "HIP attention");
+      const std::size_t ws = split.workspace_bytes;
       std::shared_ptr<HipBuffer> workspace;
       if (ws) {
         auto created = HipBuffer::create(ws);

@@ -993,26 +993,41 @@ struct FlashForm {
   int resident;  // blocks a CU holds
 };
 
+// What the workspace of a split costs the call, in microseconds: nothing where
+// the caller has it, and a mapping of memory where it is allocated for the call
+// and no pool has blocks to give (2.5 us below 2 MiB, 25 from there on).
+double workspace_cost(std::size_t bytes, bool per_call) {
+  if (!per_call || bytes == 0 || allocation_cached(bytes)) return 0.0;
+  return bytes < (std::size_t{2} << 20) ? 2.5 : 25.0;
+}
+
 std::size_t split_bytes(std::int64_t splits, std::int64_t batch, std::int64_t rows, std::int64_t features) {
   return splits > 1 ? static_cast<std::size_t>(splits * batch * rows) * (features + 2) * sizeof(float) : 0;
 }
 
+// What a plan may use: a workspace of at most `bytes`, allocated for the one
+// call or not.
+struct FlashLimit {
+  std::size_t bytes;
+  bool per_call;
+};
+
 // The split of the keys that is expected to end first, with its time in
 // microseconds. A block's time is its tiles on the busiest of 256 CUs and 4 us
 // of start and end a round; a split call also runs the combine (4 us and the
-// states written and read at 4 TB/s). Under causal masking almost half of the
-// parts of a split are empty. Within 15 % of what MI355X took for 20 shapes of
-// 3 to 512 matrices, 5 to 2048 queries and 128 to 4096 keys; a split has to
-// promise 8 %, and room in the workspace. `cols` are the keys that the
+// states written and read at 4 TB/s) and may have to map its workspace. Under
+// causal masking almost half of the parts of a split are empty. Within 15 % of
+// what MI355X took for 20 shapes of 3 to 512 matrices, 5 to 2048 queries and
+// 128 to 4096 keys; a split has to promise 8 %. `cols` are the keys that the
 // last query sees.
 double best_split(const FlashForm& f, std::int64_t batch, std::int64_t rows, std::int64_t cols, std::int64_t features,
-                  bool causal, std::size_t limit, std::int64_t& splits) {
+                  bool causal, FlashLimit limit, std::int64_t& splits) {
   const std::int64_t items = ceil_div(rows, 16 * f.waves) * batch, tiles = std::max<std::int64_t>(ceil_div(cols, f.keys), 1);
   double best = 0;
   splits = 1;
   for (const std::int64_t n : kSplits) {
     const std::size_t bytes = split_bytes(n, batch, rows, features);
-    if (n > 1 && (n > tiles || items * n > 2048 || bytes > limit)) break;
+    if (n > 1 && (n > tiles || items * n > 2048 || bytes > limit.bytes)) break;
     const std::int64_t per = ceil_div(tiles, n);
     if (n > 1 && ceil_div(tiles, per) != n) continue;  // another count cuts the tiles the same way
     const double blocks = static_cast<double>(causal && n > 1 ? items * (n + 1) : items * n) * (causal && n > 1 ? 0.6 : 1.0);
@@ -1021,7 +1036,7 @@ double best_split(const FlashForm& f, std::int64_t batch, std::int64_t rows, std
     if (causal && n == 1 && on_cu > 1)  // the light blocks fill in beside the heavy ones
       time = std::max(static_cast<double>(per) * f.alone, 0.5 * time);
     time += 4.0 * static_cast<double>(ceil_div(on_cu, f.resident));
-    if (n > 1) time += 4.0 + static_cast<double>(n * batch * rows * features) * 2e-6;
+    if (n > 1) time += 4.0 + static_cast<double>(n * batch * rows * features) * 2e-6 + workspace_cost(bytes, limit.per_call);
     if (n == 1) best = time;
     else if (time < 0.92 * best) best = time, splits = n;
   }
@@ -1029,7 +1044,7 @@ double best_split(const FlashForm& f, std::int64_t batch, std::int64_t rows, std
 }
 
 FlashPlan flash_plan(std::int64_t batch, std::int64_t rows, std::int64_t cols, std::int64_t features, bool causal,
-                     int mask_kind, std::size_t limit) {
+                     int mask_kind, FlashLimit limit) {
   FlashPlan p{};
   if (causal) cols = std::min(cols, rows);  // the keys after the last query are not run
   if (rows <= kDecodeRows && !causal && cols > 0) {
@@ -1039,7 +1054,7 @@ FlashPlan flash_plan(std::int64_t batch, std::int64_t rows, std::int64_t cols, s
     p.decode = true;
     std::int64_t splits = 1;
     for (const std::int64_t n : kSplits)
-      if (n * batch <= 256 && n * 128 <= cols && cols >= 512 && split_bytes(n, batch, rows, features) <= limit)
+      if (n * batch <= 256 && n * 128 <= cols && cols >= 512 && split_bytes(n, batch, rows, features) <= limit.bytes)
         splits = n;
     p.split_keys = ceil_div(ceil_div(cols, splits), 64) * 64;
     p.splits = ceil_div(cols, p.split_keys);
@@ -1171,7 +1186,7 @@ int tcx_hip_flash_attention_ws_supported(int64_t features, int64_t value_feature
   return features == value_features && features >= 16 && features <= 128 && features % 8 == 0 ? 1 : 0;
 }
 
-int tcx_hip_flash_attention_plan(const tcx_hip_flash_attention_desc_t* desc, size_t workspace_bytes,
+int tcx_hip_flash_attention_plan(const tcx_hip_flash_attention_desc_t* desc, size_t workspace_bytes, int per_call,
                                  tcx_hip_flash_attention_plan_t* plan) {
   using namespace tcx;
   if (desc == nullptr || plan == nullptr) return fail(TCX_INVALID_ARGUMENT, "attention plan or descriptor is null");
@@ -1179,14 +1194,14 @@ int tcx_hip_flash_attention_plan(const tcx_hip_flash_attention_desc_t* desc, siz
       !tcx_hip_flash_attention_ws_supported(desc->features, desc->features))
     return fail(TCX_INVALID_ARGUMENT, "no fused attention for these extents");
   const FlashPlan p = flash_plan(desc->batch, desc->rows, desc->cols, desc->features, desc->causal != 0,
-                                 desc->mask_kind, workspace_bytes);
+                                 desc->mask_kind, {workspace_bytes, per_call != 0});
   *plan = {p.decode ? 1 : 0, p.decode ? 4 : p.waves, p.keys, static_cast<std::int32_t>(p.splits), p.bytes};
   return TCX_OK;
 }
 
 size_t tcx_hip_flash_attention_workspace_bytes(const tcx_hip_flash_attention_desc_t* desc) {
   tcx_hip_flash_attention_plan_t plan{};
-  return tcx_hip_flash_attention_plan(desc, SIZE_MAX, &plan) == TCX_OK ? plan.workspace_bytes : 0;
+  return tcx_hip_flash_attention_plan(desc, SIZE_MAX, 0, &plan) == TCX_OK ? plan.workspace_bytes : 0;
 }
 
 int tcx_hip_flash_attention_f32_ws(const float* q, const float* k, const float* v, float* out, const void* mask,
@@ -1230,7 +1245,7 @@ int tcx_hip_flash_attention_f32_ws(const float* q, const float* k, const float* 
   // The best plan that the workspace has room for.
   const bool usable = workspace != nullptr && (reinterpret_cast<std::uintptr_t>(workspace) & 15U) == 0;
   const FlashPlan p = flash_plan(d.batch, d.rows, d.cols, d.features, d.causal != 0, a.mask_kind,
-                                 usable ? workspace_bytes : 0);
+                                 {usable ? workspace_bytes : 0, false});
   // Blocks of one batch matrix, and as many matrices a launch as HIP counts work-items for.
   const std::int64_t blocks = (p.decode ? 1 : ceil_div(d.rows, 16 * p.waves)) * p.splits;
   const std::int64_t per_launch = kMaxLaunchWorkItems / (p.decode ? 256 : 64 * p.waves) / blocks;

@@ -80,6 +80,9 @@ struct FastDiv {
 std::int32_t* acquire_host_flag();
 void release_host_flag(std::int32_t* flag);
 
+// True when this thread's tcx_hip_allocate keeps a block of `bytes` from call to call.
+bool allocation_cached(std::size_t bytes);
+
 // Wave-wide butterfly sums: both partners add the same two operands, so every
 // lane ends with identical bits and the order is fixed for a given layout.
 __device__ __forceinline__ float wave_sum(float v) {

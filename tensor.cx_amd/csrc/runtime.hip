@@ -320,6 +320,10 @@ void pool_release(tcx_hip_pool* pool, void* ptr, size_t bytes, bool allow_cache)
 }
 }  // namespace
 
+bool tcx::allocation_cached(std::size_t bytes) {
+  return active_pool != nullptr && active_pool->stats.max_cached_blocks > 0 && bytes <= active_pool->stats.max_cached_bytes;
+}
+
 extern "C" {
 
 const char* tcx_hip_last_error(void) { return tcx::last_error.c_str(); }

@@ -25,15 +25,16 @@ class Plan(ctypes.Structure):
 ANY = ctypes.c_size_t(-1).value
 
 
-def plan(batch, rows, cols, features, causal=False, mask=0, limit=ANY):
+def plan(batch, rows, cols, features, causal=False, mask=0, limit=ANY, per_call=False):
     out = Plan()
     desc = Desc(batch=batch, rows=rows, cols=cols, features=features, causal=int(causal), mask_kind=mask)
-    capi.check(capi.lib().tcx_hip_flash_attention_plan(ctypes.byref(desc), ctypes.c_size_t(limit), ctypes.byref(out)), "plan")
+    capi.check(capi.lib().tcx_hip_flash_attention_plan(ctypes.byref(desc), ctypes.c_size_t(limit), int(per_call),
+                                                       ctypes.byref(out)), "plan")
     return out
 
 
 def test_no_plan_without_a_fused_kernel():
-    assert capi.lib().tcx_hip_flash_attention_plan(None, 0, ctypes.byref(Plan())) == capi.TCX_INVALID_ARGUMENT
+    assert capi.lib().tcx_hip_flash_attention_plan(None, 0, 0, ctypes.byref(Plan())) == capi.TCX_INVALID_ARGUMENT
     for shape in ((0, 4, 4, 64), (1, 0, 4, 64), (1, 4, -1, 64), (1, 4, 4, 20)):
         with pytest.raises(capi.HipError):
             plan(*shape)
@@ -77,3 +78,25 @@ def test_causal_plans_for_the_visible_keys(rows, features, mask):
     visible, all_keys = plan(8, rows, rows, features, True, mask), plan(8, rows, 8000, features, True, mask)
     assert all_keys.splits == visible.splits and all_keys.workspace_bytes == visible.workspace_bytes
     assert rows > 64 or all_keys.splits == 1
+
+
+@pytest.mark.parametrize("batch,rows,features,causal", [(8, 128, 128, True), (16, 256, 64, True), (16, 512, 32, False)])
+def test_allocation_of_the_workspace_counts(batch, rows, features, causal):
+    """A workspace that is allocated for the call costs 25 us from 2 MiB on,
+    which these splits do not bring; in a pool that keeps it, nothing."""
+    kept, once = (plan(batch, rows, rows, features, causal, per_call=c) for c in (False, True))
+    assert kept.workspace_bytes >= 2 << 20 and kept.splits > 1
+    assert once.workspace_bytes < 2 << 20
+    long = plan(1, 64, 8192, 128, per_call=True)
+    assert long.splits > 1  # 700 us of one block's keys pay for it
+
+    fails = capi.PoolRuntime(capi.ALLOCATE_FN(lambda out, n: 1), capi.FREE_FN(lambda ptr: 0), capi.CLEAR_FN(lambda: 0))
+    pool = ctypes.c_void_p()
+    for limit, expected in ((1 << 30, kept), (kept.workspace_bytes, kept), (1 << 20, once)):
+        capi.check(capi.lib().tcx_hip_pool_create(limit, 8, ctypes.byref(fails), ctypes.byref(pool)), "pool")
+        capi.check(capi.lib().tcx_hip_pool_enter(pool), "enter")
+        try:
+            assert plan(batch, rows, rows, features, causal, per_call=True).splits == expected.splits
+        finally:
+            capi.check(capi.lib().tcx_hip_pool_exit(pool), "exit")
+            capi.lib().tcx_hip_pool_destroy(pool)
