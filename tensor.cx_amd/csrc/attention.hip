@@ -653,13 +653,16 @@ __device__ __forceinline__ void flash_store(const FlashArgs& a, const int* bad_c
     const float mv = __shfl(st.m, src, kWave);
     const std::int64_t qrow = q0 + 4 * g + v;
     if (qrow >= a.rows) continue;
+    // A split's outputs by the same code, over 1: a third way out of each of
+    // the divisions below cost a call on 64 x 64 x 128 a microsecond of 12.
+    const float over = parts ? 1.F : lv;
+    const bool hidden = !parts && mv == neg_inf;
     float y[kT];
 #pragma unroll
     for (int t = 0; t < kT; ++t) {
       if (bad_column[output_feature<kT>(r, t)]) y[t] = __builtin_nanf("");
-      else if (parts) y[t] = st.o[t][v];
-      else if (mv == neg_inf) y[t] = st.o[t][v] * 0.F;
-      else y[t] = st.o[t][v] / lv;
+      else if (hidden) y[t] = st.o[t][v] * 0.F;
+      else y[t] = st.o[t][v] / over;
     }
     if (parts && r == 0) *reinterpret_cast<float2_t*>(a.part_ml + (first + qrow) * 2) = float2_t{mv, lv};
     float* const orow = ob + qrow * features;
@@ -686,21 +689,24 @@ flash_attention_kernel(FlashArgs a) {
   const int tid = threadIdx.x;
   // One block per work item on a 1-D grid of n = qtiles x batch blocks; the
   // launch id maps to an item (batch-major by default).
-  const std::int64_t n = a.qtiles * a.batch;
-  const std::int64_t split = blockIdx.x / n, id = blockIdx.x % n;
-  std::int64_t batch = id / a.qtiles, qtile = id % a.qtiles;
+  // The arithmetic is in 32 bits, as a grid's size is: a block of one key tile
+  // waits for each 64-bit division about as long as for its loads.
+  const auto qtiles = static_cast<std::uint32_t>(a.qtiles), batches = static_cast<std::uint32_t>(a.batch);
+  const std::uint32_t n = qtiles * batches;
+  const std::uint32_t split = a.splits > 1 ? blockIdx.x / n : 0, id = blockIdx.x - split * n;
+  std::uint32_t item_batch = id / qtiles, item_tile = id - item_batch * qtiles;
   if (a.xcd_blocks) {
     // Launch id L runs on XCD L % 8: give XCD x the consecutive (batch-major)
     // work items x * n/8 .. (x + 1) * n/8 - 1, so that the query tiles of one
     // batch matrix share its K and V in that XCD's L2 (n % 8 == 0).
-    const std::int64_t item = (id % 8) * (n / 8) + id / 8;
-    batch = item / a.qtiles;
-    qtile = item % a.qtiles;
-    if (kMask != TCX_MASK_NONE && a.batch % 8 == 0) {
+    const std::uint32_t item = (id % 8) * (n / 8) + id / 8;
+    item_batch = item / qtiles;
+    item_tile = item - item_batch * qtiles;
+    if (kMask != TCX_MASK_NONE && batches % 8 == 0) {
       // Masks can make one sequence of a batch much shorter than another, so
       // the XCDs take its matrices in turns: matrix b on XCD b % 8.
-      batch = id % 8 + 8 * (id / 8 / a.qtiles);
-      qtile = id / 8 % a.qtiles;
+      item_batch = id % 8 + 8 * (id / 8 / qtiles);
+      item_tile = id / 8 % qtiles;
     }
   }
   if constexpr (kCausal) {
@@ -712,11 +718,12 @@ flash_attention_kernel(FlashArgs a) {
     // than fit, the grid runs heaviest first throughout, so that the light
     // items fill the CUs the heavy ones leave (longest job first: 16 x 4096 x
     // 128 720 -> 658 us, 48 x 2048 x 128 536 -> 482 us on MI355X).
-    const std::int64_t half = (n + 1) / 2;
-    const std::int64_t rank = a.heavy_first || id < half ? id : n - 1 - (id - half);
-    qtile = a.qtiles - 1 - rank / a.batch;
-    batch = rank % a.batch;
+    const std::uint32_t half = (n + 1) / 2;
+    const std::uint32_t rank = a.heavy_first || id < half ? id : n - 1 - (id - half);
+    item_tile = qtiles - 1 - rank / batches;
+    item_batch = rank % batches;
   }
+  const std::int64_t batch = item_batch, qtile = item_tile;
   const std::int64_t q_last = min(qtile * kQTile + kQTile, a.rows) - 1;
   const std::int64_t tiles = (a.cols + kKeys - 1) / kKeys;
   // Key tiles [first, run): under causal masking tiles past the block's last
