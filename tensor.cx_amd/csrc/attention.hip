@@ -993,10 +993,10 @@ constexpr std::int64_t kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};  
 
 // A form of flash_attention_kernel and what a key tile costs in it, in
 // microseconds of one CU: in a block that has the CU to itself, and for each
-// block where several share it.
+// block where two and where more share it.
 struct FlashForm {
   int waves, keys;
-  double alone, shared;
+  double alone, two, shared;
   int resident;  // blocks a CU holds
 };
 
@@ -1039,7 +1039,7 @@ double best_split(const FlashForm& f, std::int64_t batch, std::int64_t rows, std
     if (n > 1 && ceil_div(tiles, per) != n) continue;  // another count cuts the tiles the same way
     const double blocks = static_cast<double>(causal && n > 1 ? items * (n + 1) : items * n) * (causal && n > 1 ? 0.6 : 1.0);
     const std::int64_t on_cu = ceil_div(static_cast<std::int64_t>(blocks), 256);
-    double time = static_cast<double>(per) * (on_cu > 1 ? static_cast<double>(on_cu) * f.shared : f.alone);
+    double time = static_cast<double>(per) * (on_cu > 2 ? static_cast<double>(on_cu) * f.shared : on_cu > 1 ? 2 * f.two : f.alone);
     if (causal && n == 1 && on_cu > 1)  // the light blocks fill in beside the heavy ones
       time = std::max(static_cast<double>(per) * f.alone, 0.5 * time);
     time += 4.0 * static_cast<double>(ceil_div(on_cu, f.resident));
@@ -1053,8 +1053,13 @@ double best_split(const FlashForm& f, std::int64_t batch, std::int64_t rows, std
 FlashPlan flash_plan(std::int64_t batch, std::int64_t rows, std::int64_t cols, std::int64_t features, bool causal,
                      int mask_kind, FlashLimit limit) {
   FlashPlan p{};
+  const bool mostly_hidden = causal && cols > 2 * rows;
   if (causal) cols = std::min(cols, rows);  // the keys after the last query are not run
-  if (rows <= kDecodeRows && !causal && cols > 0) {
+  // Decoding streams the keys; plain calls of 32 features have too few of them
+  // for that up to 64, or 128 where more queries share them (their states cost
+  // more to join than a tile: 1500 x 4 x 16 x 32 25 us, 8.6 in tiles).
+  const bool few_keys = features == 32 && mask_kind == TCX_MASK_NONE && cols <= (rows == 1 ? 64 : 128);
+  if (rows <= kDecodeRows && !causal && cols > 0 && !few_keys) {
     // Up to 256 blocks of at least 128 keys (8 splits of 32 x 4096 x 128 24.1
     // us, 32 splits 25.2, one 91.4); short sequences whole, since the combine
     // costs more than it brings (16 x 300 x 64 6.6 us, 8.2 in two).
@@ -1071,20 +1076,29 @@ FlashPlan flash_plan(std::int64_t batch, std::int64_t rows, std::int64_t cols, s
     // masking a heavy and a light one (89 TFLOP/s at 16 x 2048 x 128 against
     // 86 for a register-staged 4-wave kernel, 92 against 71 at 32 x 2048 x 64).
     // At D = 32 and 64 also 64-key tiles, with half the barriers and softmax
-    // chains and half the blocks a CU (16 x 1024 x 64 53 -> 47 us, x 32 36 -> 30,
-    // causal 32 x 512 x 64 31.2 -> 27.9, 160 x 320 x 64 40.7 -> 36.8); with 1024
-    // causal blocks and more, 32 keys stay ahead (32 x 2048 x 64 170 against
-    // 184). Unmasked at D = 128 eight waves and 64-key tiles, one block per CU,
+    // chains and half the blocks a CU: 0.83 to 0.9 of the time where a CU has one
+    // block (8 x 1024 x 64 52 -> 46 us), 0.93 to 0.95 with two, 0.97 (D = 32) and
+    // 1.03 (D = 64; causal 1.1) with more (512 x 512 x 64 294 against 314), times
+    // what the last tile adds (200 keys: 256 for 224). Where most keys lie behind
+    // the causal mask, 32-key tiles: 128 x 200 x 8000 at D = 32 64 us against 69.
+    // Unmasked at D = 128 eight waves and 64-key tiles, one block per CU,
     // where there are enough (16 x 2048 281 against 291 us). Up to 16 queries
-    // one wave holds them all: 60 us against 81 for 512 matrices of 16 queries
-    // and 512 keys at D = 128.
-    static constexpr FlashForm kFour[] = {{4, 32, 1.0, 0.8, 5}, {4, 32, 1.53, 1.27, 4}, {4, 32, 2.65, 2.27, 2}};
-    static constexpr FlashForm kLong[] = {{4, 64, 1.64, 1.25, 4}, {4, 64, 2.71, 2.35, 2}}, kEight128{8, 64, 8.7, 8.7, 1};
-    static constexpr FlashForm kOne[] = {{1, 32, 1.0, 0.4, 8}, {1, 32, 1.7, 0.6, 5}, {1, 32, 2.85, 1.9, 2}};
-    // Padded kernels have the general form only.
+    // one wave holds them all where blocks share a CU: 60 us against 81 for 512
+    // matrices of 16 queries and 512 keys at D = 128 (alone 35.5 against 33.4 for
+    // 1000 keys at D = 32).
+    static constexpr FlashForm kFour[] = {
+        {4, 32, 1.0, 0.76, 0.76, 5}, {4, 32, 1.53, 1.27, 1.27, 4}, {4, 32, 2.65, 2.27, 2.27, 2}};
+    static constexpr FlashForm kLong[] = {{4, 64, 1.66, 1.42, 1.49, 5}, {4, 64, 2.71, 2.41, 2.64, 4}};
+    static constexpr FlashForm kOne[] = {
+        {1, 32, 1.06, 0.4, 0.4, 8}, {1, 32, 1.7, 0.6, 0.6, 4}, {1, 32, 2.85, 1.9, 1.9, 2}};
+    static constexpr FlashForm kEight128{8, 64, 8.7, 8.7, 8.7, 1};
+    // Masked and padded kernels have the general form only, and are planned by
+    // the plain kernels' costs: theirs are 1.1 to 2 times as much a tile, with two
+    // or three blocks a CU, but with constants of their own 657 calls took the
+    // same time in the mean (0.77 to 1.23 of it).
     const int d = features > 64 ? 2 : features > 32 ? 1 : 0;
     const bool padded = features != 32 << d, plain = !padded && !causal && mask_kind == TCX_MASK_NONE;
-    FlashForm form = plain && rows <= 16 ? kOne[d] : kFour[d];
+    FlashForm form = kFour[d];
     double time = best_split(form, batch, rows, cols, features, causal, limit, p.splits);
     auto consider = [&](const FlashForm& other) {
       std::int64_t splits;
@@ -1094,7 +1108,8 @@ FlashPlan flash_plan(std::int64_t batch, std::int64_t rows, std::int64_t cols, s
       form = other;
       p.splits = splits;
     };
-    if (!padded && mask_kind == TCX_MASK_NONE && features <= 64 && form.waves == 4 &&
+    if (plain && rows <= 16) consider(kOne[d]);
+    if (!padded && mask_kind == TCX_MASK_NONE && features <= 64 && form.waves == 4 && !mostly_hidden &&
         (!causal || ceil_div(rows, 64) * batch < 1024))
       consider(kLong[d]);
     if (d == 2 && plain && rows > 64) consider(kEight128);

@@ -100,3 +100,30 @@ def test_allocation_of_the_workspace_counts(batch, rows, features, causal):
         finally:
             capi.check(capi.lib().tcx_hip_pool_exit(pool), "exit")
             capi.lib().tcx_hip_pool_destroy(pool)
+
+
+# (batch, rows, cols, features, causal, waves, keys), measured both ways.
+@pytest.mark.parametrize("shape", [
+    (512, 100, 333, 32, False, 4, 32),    # 35.7 us; 64-key tiles 38.5 (333 keys fill 5.2 of them)
+    (64, 200, 200, 32, False, 4, 64),     # one block a CU
+    (512, 512, 512, 64, False, 4, 32),    # 294 us; 64-key tiles 314
+    (64, 512, 512, 64, False, 4, 64),     # 45.0 us; 32-key tiles 47.2
+    (300, 200, 200, 64, True, 4, 32),
+    (8, 16, 1000, 32, False, 4, 64),      # one wave a block where blocks share CUs
+    (512, 16, 512, 128, False, 1, 32),
+    (128, 200, 8000, 64, True, 4, 32),    # the keys behind the mask are most of the work
+    (32, 1000, 1000, 128, False, 8, 64),
+    (64, 300, 300, 128, False, 8, 64),
+    (40, 500, 500, 128, False, 8, 64),
+    (32, 970, 1025, 128, False, 8, 64),
+])
+def test_forms(shape):
+    p = plan(*shape[:5], limit=0)
+    assert (p.decode, p.waves, p.keys) == (0, *shape[5:])
+
+
+@pytest.mark.parametrize("rows,cols,features,mask,decode", [
+    (1, 64, 32, 0, 0), (1, 65, 32, 0, 1), (2, 128, 32, 0, 0), (4, 128, 32, 0, 0), (4, 129, 32, 0, 1), (4, 16, 32, 1, 1),
+    (4, 16, 64, 0, 1), (1, 1, 128, 0, 1), (4, 16, 24, 0, 1), (5, 500, 32, 0, 0), (3, 0, 64, 0, 0)])
+def test_few_queries_and_keys(rows, cols, features, mask, decode):
+    assert plan(300, rows, cols, features, mask=mask).decode == decode

@@ -392,3 +392,20 @@ def test_workspace_with_room_for_some_splits(cx, batch, rows, cols, d, causal):
         capi.synchronize()
         assert_close(out.numpy(), expected, 2e-4, 2e-5, f"{nbytes} of {full} bytes")
         assert (workspace.numpy()[nbytes // 4:] == 99).all()
+
+
+# Eight waves and 64-key tiles (tests of the plan pin that these sizes take
+# them): query and key remainders, and values that are not finite in the last,
+# partial key tile and in rows of every wave.
+@pytest.mark.parametrize("batch,rows,cols", [(64, 300, 300), (32, 1000, 1000), (40, 500, 500), (32, 970, 1025)])
+def test_eight_waves(cx, batch, rows, cols):
+    q, k, v = f32((batch, rows, 128), 65), f32((batch, cols, 128), 66), f32((batch, cols, 128), 67)
+    check(cx, q, k, v)
+    q[0, ::37, 5] = np.nan
+    k[1, cols - 1, 3] = np.inf
+    k[2, 70, 4] = -np.inf
+    v[3, cols - 1, 127] = np.inf
+    v[3, 64, 2] = np.nan
+    v[batch - 1, 0, 0] = -np.inf
+    q[1, rows - 1] = 0
+    check(cx, q, k, v)
