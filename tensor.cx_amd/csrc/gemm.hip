@@ -304,8 +304,10 @@ extern "C" int tcx_hip_gemm_f32_ws(const float* lhs, const float* rhs, float* ou
   // One row of A against a transposed B, or one column of B: a
   // matrix-vector product, the long operand's rows streamed in whole cache
   // lines (one or no batch axis).
-  // (Rows of 64 k at any address; shorter ones only where 16-byte.)
-  if (d->batch_rank <= 1 && (d->k >= 64 || (strides_vec && d->k % 4 == 0 && aligned16(lhs) && aligned16(rhs)))) {
+  // (Rows of 64 k at any address, as many as a launch holds with a wave each;
+  // shorter ones only where 16-byte.)
+  const bool rows_vec = strides_vec && d->k % 4 == 0 && aligned16(lhs) && aligned16(rhs);
+  if (d->batch_rank <= 1 && (rows_vec || (d->k >= 64 && d->m * d->n * batches <= kMaxLaunchWorkItems / 256 * 4))) {
     const std::int64_t lbs = d->batch_rank == 1 ? d->lhs_batch_strides[0] : 0;
     const std::int64_t rbs = d->batch_rank == 1 ? d->rhs_batch_strides[0] : 0;
     if (trans_b && d->m == 1)

@@ -137,3 +137,26 @@ def test_unaligned_operands(capi, trans, shift):
     """Sizes of 16-byte rows at addresses between them."""
     for m, n, k in ((700, 704, 128), (64, 64, 256), (16, 512, 1024), (1, 300, 512), (1100, 1100, 260)):
         check(capi, m, n, k, trans, shift=shift, leak=False)
+
+
+@pytest.mark.parametrize("trans", [False, True])
+def test_more_rows_than_a_launch_holds(capi, trans):
+    """2^26 + 70 rows of 65 k by one column: a wave each would be more
+    work-items than HIP counts."""
+    rows, k, tail = (1 << 26) + 70, 65, 200
+    rng = np.random.default_rng(5)
+    a, b, out = capi.DeviceBuffer(4 * rows * k), capi.DeviceArray.from_numpy(rng.standard_normal(k).astype(np.float32)), \
+        capi.DeviceBuffer(4 * rows)
+    capi.check(capi.lib().tcx_hip_fill(0, a.ptr, rows * k, 1.0, capi.stream()), "fill")
+    capi.check(capi.lib().tcx_hip_fill(0, out.ptr, rows, -7.0, capi.stream()), "fill")
+    last = rng.standard_normal((tail, k)).astype(np.float32)
+    capi.check(capi.lib().tcx_hip_memcpy_h2d(a.address + 4 * (rows - tail) * k, last.ctypes.data, last.nbytes, capi.stream()), "h2d")
+    m, n = (1, rows) if trans else (rows, 1)
+    lhs, rhs = (b.ptr, a.ptr) if trans else (a.ptr, b.ptr)
+    capi.gemm(lhs, rhs, out.ptr, capi.gemm_desc(m, n, k, rhs_transposed=trans))
+    got = np.empty(tail, np.float32)
+    column = b.numpy().astype(np.float64)
+    for first, expected in ((rows - tail, last @ column), (0, np.full(tail, column.sum())),
+                            ((1 << 25) + 7, np.full(tail, column.sum()))):
+        capi.check(capi.lib().tcx_hip_memcpy_d2h(got.ctypes.data, out.address + 4 * first, got.nbytes, capi.stream()), "d2h")
+        assert np.abs(got - expected).max() <= 1e-4 * np.sqrt(k)
