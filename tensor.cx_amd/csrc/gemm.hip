@@ -312,10 +312,10 @@ extern "C" int tcx_hip_gemm_f32_ws(const float* lhs, const float* rhs, float* ou
     const std::int64_t rbs = d->batch_rank == 1 ? d->rhs_batch_strides[0] : 0;
     if (trans_b && d->m == 1)
       return gemm::launch_gemv(rhs, lhs, out, d->bias, d->n, d->k, batches, rbs, lbs, d->n, 1, true,
-                               d->activation, s);
+                               d->activation, rows_vec, s);
     if (d->n == 1)
       return gemm::launch_gemv(lhs, rhs, out, d->bias, d->m, d->k, batches, lbs, rbs, d->m, 1, false,
-                               d->activation, s);
+                               d->activation, rows_vec, s);
   }
   // One row of A against a row-major B per batch item (rows of 512+
   // columns), with enough items x 1024-column chunks to give every CU a

@@ -1667,7 +1667,10 @@ __device__ __forceinline__ float4_t stream_load4(const float* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const float4_u*>(p));
 }
 
-template <int KW>
+// kRagged: K no multiple of 4 or rows off a 16-byte boundary. Apart, as what
+// rows of any address need cost rows of 4 k a fifth of their time (705 x 1852 of
+// them 268 us, 316).
+template <int KW, bool kRagged>
 __global__ __launch_bounds__(256) void gemv_f32_kernel(const float* __restrict__ R, const float* __restrict__ v,
                                                        float* __restrict__ y, const float* __restrict__ bias,
                                                        std::int64_t rows, std::int64_t K, std::int64_t batches,
@@ -1685,9 +1688,16 @@ __global__ __launch_bounds__(256) void gemv_f32_kernel(const float* __restrict__
     const float* __restrict__ rp = R + batch * r_batch + i * K;
     const float* __restrict__ vp = v + batch * v_batch;
     // This wave's run of K: whole 1024-element strides first, 4-element
-    // groups after, from rows at any 4-byte address; the last K % 4 elements
-    // are single words of the last wave.
-    const std::int64_t K4 = K & ~std::int64_t{3};
+    // groups after; the last K % 4 elements are single words of the last wave.
+    auto load = [](const float* p) -> float4_t {
+      if constexpr (kRagged) return *reinterpret_cast<const float4_u*>(p);
+      else return *reinterpret_cast<const float4_t*>(p);
+    };
+    auto load_once = [](const float* p) -> float4_t {
+      if constexpr (kRagged) return stream_load4(p);
+      else return stream_load(reinterpret_cast<const float4_t*>(p));
+    };
+    const std::int64_t K4 = kRagged ? K & ~std::int64_t{3} : K;
     const std::int64_t run = (K / 4 + KW - 1) / KW * 4;
     const std::int64_t k_begin = part * run, k_end = min(K4, k_begin + run);
     float s[8] = {};
@@ -1695,18 +1705,18 @@ __global__ __launch_bounds__(256) void gemv_f32_kernel(const float* __restrict__
     for (; k + 7 * 256 < k_end; k += 8 * 256) {
       float4_t w[8], x[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) w[u] = stream_load4(rp + k + 256 * u);
+      for (int u = 0; u < 8; ++u) w[u] = load_once(rp + k + 256 * u);
 #pragma unroll
-      for (int u = 0; u < 8; ++u) x[u] = *reinterpret_cast<const float4_u*>(vp + k + 256 * u);
+      for (int u = 0; u < 8; ++u) x[u] = load(vp + k + 256 * u);
 #pragma unroll
       for (int u = 0; u < 8; ++u) s[u] += (w[u].x * x[u].x + w[u].y * x[u].y) + (w[u].z * x[u].z + w[u].w * x[u].w);
     }
     for (; k < k_end; k += 256) {
-      const float4_t w = stream_load4(rp + k);
-      const float4_t x = *reinterpret_cast<const float4_u*>(vp + k);
+      const float4_t w = load_once(rp + k);
+      const float4_t x = load(vp + k);
       s[0] += (w.x * x.x + w.y * x.y) + (w.z * x.z + w.w * x.w);
     }
-    if (part == KW - 1 && K4 + lane < K) s[1] += rp[K4 + lane] * vp[K4 + lane];
+    if (kRagged && part == KW - 1 && K4 + lane < K) s[1] += rp[K4 + lane] * vp[K4 + lane];
     sum = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
   }
   sum = wave_sum(sum);
@@ -2166,22 +2176,21 @@ inline int launch_tiny(GemmArgs& args, bool trans_b, hipStream_t stream) {
 // 16-byte aligned): KW waves per row, more when rows are few.
 inline int launch_gemv(const float* R, const float* v, float* y, const float* bias, std::int64_t rows,
                        std::int64_t K, std::int64_t batches, std::int64_t r_batch, std::int64_t v_batch,
-                       std::int64_t y_batch, std::int64_t y_stride, bool bias_per_row, int act, hipStream_t stream) {
+                       std::int64_t y_batch, std::int64_t y_stride, bool bias_per_row, int act, bool vec,
+                       hipStream_t stream) {
   const std::int64_t total = rows * batches;
   const int kw = total >= 4096 ? 1 : total >= 2048 ? 2 : 4;
   const std::int64_t blocks = (total * kw + 3) / 4;
   if (blocks > 0x7fffffff) return fail(TCX_INVALID_ARGUMENT, "gemm grid is too large");
   const dim3 grid(static_cast<unsigned>(blocks));
   const int bpr = bias_per_row ? 1 : 0;
-  if (kw == 1)
-    hipLaunchKernelGGL(gemv_f32_kernel<1>, grid, dim3(256), 0, stream, R, v, y, bias, rows, K, batches, r_batch,
-                       v_batch, y_batch, y_stride, bpr, act);
-  else if (kw == 2)
-    hipLaunchKernelGGL(gemv_f32_kernel<2>, grid, dim3(256), 0, stream, R, v, y, bias, rows, K, batches, r_batch,
-                       v_batch, y_batch, y_stride, bpr, act);
-  else
-    hipLaunchKernelGGL(gemv_f32_kernel<4>, grid, dim3(256), 0, stream, R, v, y, bias, rows, K, batches, r_batch,
-                       v_batch, y_batch, y_stride, bpr, act);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, R, v, y, bias, rows, K, batches, r_batch, v_batch, y_batch,
+                       y_stride, bpr, act);
+  };
+  if (kw == 1) go(vec ? gemv_f32_kernel<1, false> : gemv_f32_kernel<1, true>);
+  else if (kw == 2) go(vec ? gemv_f32_kernel<2, false> : gemv_f32_kernel<2, true>);
+  else go(vec ? gemv_f32_kernel<4, false> : gemv_f32_kernel<4, true>);
   return check(hipGetLastError(), "gemv launch");
 }
 
