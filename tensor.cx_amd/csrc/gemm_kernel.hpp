@@ -2269,7 +2269,16 @@ int launch_stream(GemmArgs& args, bool vec, hipStream_t stream) {
   }
   const std::int64_t chunks = (args.k + 15) / 16;
   int ks = 1;
-  while (ks < 16 && ks * 2 <= chunks && blocks * ks < 4096) ks *= 2;
+  if (kXCols && !vec) {
+    // Rows of any address against a [k, n] B: fewer waves, which in eight or
+    // sixteen a block cost more to join than they read (8000x4x440 scalar tiles
+    // 12.3 us, 16 waves a block 17.2, four 7.0; 30000x2x64 11.3, four 15.9, one
+    // 6.7), up to 12 a CU where each keeps seven chunks (20000x32x2050 with one
+    // 63, two 50).
+    while (ks < 16 && ks * 2 <= chunks && blocks * ks * 2 <= (chunks >= 14 * ks ? 3072 : 2048)) ks *= 2;
+  } else {
+    while (ks < 16 && ks * 2 <= chunks && blocks * ks < 4096) ks *= 2;
+  }
   if (J <= 16)
     launch_stream_ks<kXCols, kOutJI, 1>(args, vec, blocks, ks, stream);
   else

@@ -139,6 +139,12 @@ def test_unaligned_operands(capi, trans, shift):
         check(capi, m, n, k, trans, shift=shift, leak=False)
 
 
+@pytest.mark.parametrize("m,n,k", [(2708, 4, 440), (5000, 7, 260), (8000, 32, 129), (20000, 17, 1001), (30000, 2, 64)])
+def test_tall_and_narrow(capi, m, n, k):
+    """At most 32 columns of a [k, n] B, with one to eight waves a block."""
+    check(capi, m, n, k, False, shift=1, leak=False)
+
+
 @pytest.mark.parametrize("trans", [False, True])
 def test_more_rows_than_a_launch_holds(capi, trans):
     """2^26 + 70 rows of 65 k by one column: a wave each would be more
