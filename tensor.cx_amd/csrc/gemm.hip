@@ -125,8 +125,10 @@ bool full_rounds_128(std::int64_t m, std::int64_t n, std::int64_t batches) {
 // against 1253 us, 8191 x 2047 x 300 135 / 154, 4096 x 4096 x 525 200 / 225; but
 // without full rounds 2048 x 2049 x 2048 242 / 204, 3000 x 3001 x 1000 237 / 205,
 // 3441 x 4096 x 525 transposed 240 / 183: those leave the workspace that the
-// query offers unused. Around 10^9 multiply-adds the copies
-// and three extra launches cost more than they bring.
+// query offers unused. With less than 128 k, where scalar-load tiles would take
+// them instead, they run padded all the same (5760 x 5888 x 127, 90 % of nine
+// rounds short of two tiles: 153 us, scalar 195, ragged 199). Around 10^9
+// multiply-adds the copies and three extra launches cost more than they bring.
 constexpr std::int64_t kPadMinWork = std::int64_t{1} << 32;
 constexpr std::int64_t kPadAlign = 64;  // floats: 256-byte aligned regions
 
@@ -227,7 +229,7 @@ extern "C" int tcx_hip_gemm_f32_ws(const float* lhs, const float* rhs, float* ou
   for (int i = 0; i < d->batch_rank; ++i) batches *= d->batch_shape[i];
   if (batches != d->batch_count) return fail(TCX_INVALID_ARGUMENT, "gemm batch_count mismatch");
   if (d->m == 0 || d->n == 0 || batches == 0) return TCX_OK;
-  if (const PadPlan pad = pad_plan(d); pad.pad && full_rounds_128(d->m, d->n, 1) && d->k > 0 &&
+  if (const PadPlan pad = pad_plan(d); pad.pad && (d->k < 128 || full_rounds_128(d->m, d->n, 1)) && d->k > 0 &&
       lhs != nullptr && rhs != nullptr && out != nullptr &&
       workspace != nullptr && aligned16(workspace) &&
       workspace_bytes >= static_cast<size_t>(pad.a_floats + pad.b_floats + pad.c_floats) * sizeof(float)) {

@@ -8,6 +8,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
+import oracle
 from conftest import require_gpu
 
 pytestmark = pytest.mark.gpu
@@ -103,7 +104,7 @@ def test_direct_columns(capi, trans, n, k):
 def test_direct_many_tiles(capi, trans):
     check(capi, 2050, 2049, 70, trans)
     check(capi, 2050, 2048, 71, trans, leak=False)
-    check(capi, 1030, 1027, 4099, trans, workspace=True, leak=False)  # padded copies in the workspace
+    check(capi, 1030, 1027, 4099, trans, workspace=True, leak=False)  # 81 tiles of 128x128: the workspace is left alone
 
 
 @pytest.mark.parametrize("trans", [False, True])
@@ -137,6 +138,36 @@ def test_unaligned_operands(capi, trans, shift):
     """Sizes of 16-byte rows at addresses between them."""
     for m, n, k in ((700, 704, 128), (64, 64, 256), (16, 512, 1024), (1, 300, 512), (1100, 1100, 260)):
         check(capi, m, n, k, trans, shift=shift, leak=False)
+
+
+# Zero-padded copies in the workspace: 16 x 16 tiles of 128 x 128 (one full
+# round), and less than 128 k whatever the last round; without them 17 x 16 and
+# 24 x 24 tiles, whose last round is a small part of one.
+@pytest.mark.parametrize("trans", [False, True])
+@pytest.mark.parametrize("m,n,k,padded", [(2048, 2047, 1027, True), (5760, 5888, 127, True), (2048, 2049, 1026, False),
+                                          (3000, 3001, 1000, False)])
+def test_padded_copies(capi, m, n, k, padded, trans):
+    rng = np.random.default_rng(m + n + k)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((n, k) if trans else (k, n)).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float32)
+    da, db, dbias, out = (capi.DeviceArray.from_numpy(t) for t in (a, b, bias, np.empty((m, n), np.float32)))
+    linear = None
+    for act in ("none", "silu", "gelu"):
+        desc = capi.gemm_desc(m, n, k, rhs_transposed=trans, bias=dbias.ptr, activation=act)
+        workspace = capi.gemm_workspace(desc)
+        words = workspace.nbytes // 4
+        capi.check(capi.lib().tcx_hip_fill(0, workspace.ptr, words, 99.0, capi.stream()), "fill")
+        capi.gemm(da.ptr, db.ptr, out.ptr, desc, workspace=workspace)
+        used = np.empty(words, np.float32)
+        capi.check(capi.lib().tcx_hip_memcpy_d2h(used.ctypes.data, workspace.ptr, 4 * words, capi.stream()), "copy")
+        assert (used != 99).any() == padded
+        got = out.numpy()
+        if linear is None:
+            linear = got
+            error = np.abs(got - reference(a, b, trans, bias)).max()
+            assert error <= 1e-4 * np.sqrt(k), error
+        else:  # the same product, so the activation meets the same bits
+            np.testing.assert_allclose(got, getattr(oracle, act)(linear), rtol=1e-6, atol=1e-6)
 
 
 @pytest.mark.parametrize("m,n,k", [(2708, 4, 440), (5000, 7, 260), (8000, 32, 129), (20000, 17, 1001), (30000, 2, 64)])

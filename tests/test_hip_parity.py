@@ -1487,10 +1487,9 @@ def test_matmul_tall_short_k_narrow_n(cx, m, n, k, trans):
                                          (1000, 1001, 999, True)])
 def test_matmul_padded_odd_shapes(cx, m, n, k, trans):
     # Unbatched products whose K or N is not a multiple of 4 and of at least
-    # 2^32 multiply-adds run zero-padded copies through the 16-byte kernels
-    # when a workspace is brought (the backend brings it); the output is
-    # stripped with the bias and activation applied as the kernels' epilogue
-    # applies them. Smaller odd shapes keep the scalar-load kernels.
+    # 2^32 multiply-adds are offered a workspace for zero-padded copies (the
+    # backend brings it); with 272 and 289 tiles of 128x128 these leave it
+    # alone, and run the ragged 64x64 tiles as the smaller ones do.
     rng = np.random.default_rng(m + n + k)
     a = rng.standard_normal((m, k)).astype(np.float32)
     b = rng.standard_normal((n, k) if trans else (k, n)).astype(np.float32)
