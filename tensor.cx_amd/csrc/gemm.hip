@@ -413,7 +413,13 @@ extern "C" int tcx_hip_gemm_f32_ws(const float* lhs, const float* rhs, float* ou
   // Without 16-byte rows the direct kernel's ragged form stays ahead past three
   // rounds too, from K = 128 on (10 x 2472x385xK, scalar loads against ragged:
   // K = 33 52 / 62 us, 129 89 / 87, 257 123 / 109; 3000x3001x1000 253 / 205).
-  const bool direct64 = gemm::direct64_fits(d->m, d->n, d->k) && (vec || trans_b || d->n >= 4);
+  // One k-tile against a [k, n] B stays with the scalar loads where more than one
+  // round of 64x64 tiles leaves a last one too full for 32x64 (1932x1467, 713
+  // tiles, K = 4 to 63: 16.4 / 18.0 us; transposed 16.9 / 16.4).
+  const std::int64_t last = tiles_64 % 256;
+  const bool half = tiles_64 > 256 && tiles_64 <= 768 && last > 0 && last <= 128;
+  const bool direct64 = gemm::direct64_fits(d->m, d->n, d->k) && (vec || trans_b || d->n >= 4) &&
+                        (vec || trans_b || d->k > 64 || tiles_64 <= 256 || half);
   if (direct64 && (tiles_64 <= 768 || (!vec && d->k >= 128))) {
     // Skinny shapes whose 64x64 tiles are mostly padding run the small
     // kernel's 32x32 tiles when those waste at most two thirds as much
@@ -421,8 +427,7 @@ extern "C" int tcx_hip_gemm_f32_ws(const float* lhs, const float* rhs, float* ou
     // stays on 64x64 tiles, 24.2 against 33.8 us).
     const std::int64_t tiles_32 = ((d->m + 31) / 32) * ((d->n + 31) / 32) * batches;
     if (8 * tiles_64 > 3 * tiles_32 && gemm::small_fits(d->m, d->n, d->k)) return gemm::launch_small(args, trans_b, vec, s);
-    const std::int64_t last = tiles_64 % 256;
-    return gemm::launch_direct64(args, trans_b, tiles_64 > 256 && tiles_64 <= 768 && last > 0 && last <= 128, vec, s);
+    return gemm::launch_direct64(args, trans_b, half, vec, s);
   }
   return launch_config<64, 64, 16, 32, 32, 4, false, 4>(args, trans_b, vec, s);
 }
