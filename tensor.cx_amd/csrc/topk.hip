@@ -544,7 +544,7 @@ __global__ __launch_bounds__(1024) void topk_join_kernel(TopkArgs a) {
 // Short rows and few of them asked for: one wave a row, the row in registers
 // (kEach keys a lane), k rounds of the wave's first remaining element. Lane j
 // keeps the j-th, so the stores of a row are one instruction.
-constexpr std::int64_t kWaveRow = 1024, kWaveK = 8;
+constexpr std::int64_t kWaveRow = 1024, kWaveK = 8, kWaveWideK = 3;
 
 template <int kEach, bool kFp>
 __global__ __launch_bounds__(256) void topk_wave_kernel(TopkArgs a) {
@@ -601,7 +601,10 @@ template <int kThreads, bool kFp>
 void launch_topk(const TopkArgs& a, hipStream_t s) {
   const std::int64_t cap = kMaxLaunchWorkItems / kThreads;
   const dim3 grid(static_cast<unsigned>(a.rows < cap ? a.rows : cap));
-  if (a.k <= kFewK) hipLaunchKernelGGL((topk_kernel<kThreads, kFp, false, true>), grid, dim3(kThreads), 0, s, a);
+  // Four more where many rows of a few thousand elements share the CUs: ordered,
+  // 2424 x 4097 int32 with k = 13 180 us in k passes, 224 by the radix selection.
+  const bool few = a.k <= kFewK || (a.k <= kFewK + 4 && a.rows >= 512 && a.reduce > 2048 && a.reduce <= 8192);
+  if (few) hipLaunchKernelGGL((topk_kernel<kThreads, kFp, false, true>), grid, dim3(kThreads), 0, s, a);
   else hipLaunchKernelGGL((topk_kernel<kThreads, kFp, false, false>), grid, dim3(kThreads), 0, s, a);
 }
 
@@ -625,7 +628,10 @@ void launch_topk_parts(const TopkArgs& a, hipStream_t s) {
 
 // A wave a row up to kWaveRow elements and k = kWaveK: with k = 1, 14.7 us for
 // 65536 rows of 32 and 5.4 us for 4096 rows of 1000, against 144 and 22.7 us
-// with a block a row. Else 256 threads, of which a CU holds four or five blocks
+// with a block a row; with many rows up to twice k (60000 x 300 int32 with k = 13
+// 262 -> 152 us, equal values 1069 -> 153) and, for kWaveWideK elements, twice the
+// length (10000 x 1086 int32 with k = 1 30 -> 17 us, with k = 3 46 -> 27, equal
+// values 84 -> 27). Else 256 threads, of which a CU holds four or five blocks
 // (1024 rows of 50257 with k = 3 64 us, with 1024 threads 98; 8192 rows of 8193
 // 90 and 322; 1024 rows of 8193 16 and 42), and 1024 where one row has a CU to
 // itself and is long enough to keep them reading (one row of 50257 17 us,
@@ -633,10 +639,12 @@ void launch_topk_parts(const TopkArgs& a, hipStream_t s) {
 // where 256 would send k to the radix selection.
 template <bool kFp>
 void launch_topk_rows(const TopkArgs& a, hipStream_t s) {
-  if (a.reduce <= kWaveRow && a.k <= kWaveK) {
+  const bool short_row = a.reduce <= kWaveRow && (a.k <= kWaveK || (a.k <= 2 * kWaveK && a.rows >= (a.reduce > 256 ? 2048 : 4096)));
+  if (short_row || (a.reduce <= 2 * kWaveRow && a.k <= kWaveWideK && a.rows >= 256)) {
     if (a.reduce <= 64) launch_topk_wave<1, kFp>(a, s);
     else if (a.reduce <= 256) launch_topk_wave<4, kFp>(a, s);
-    else launch_topk_wave<16, kFp>(a, s);
+    else if (a.reduce <= kWaveRow) launch_topk_wave<16, kFp>(a, s);
+    else launch_topk_wave<32, kFp>(a, s);
   } else if ((a.reduce > 20000 && a.rows < 256) || (a.reduce > 256 && a.k > 64)) {
     launch_topk<1024, kFp>(a, s);
   } else {

@@ -139,3 +139,17 @@ def test_ordered_rows_take_little_longer(k):
             best = min(best, start.elapsed_ms(end))
         took.append(best)
     assert took[1] < 5 * took[0], took
+
+
+# A wave a row up to 2048 elements (k = 3) and, with 2048 or 4096 rows and more,
+# up to 16 elements of 1024; more of either, and fewer rows, take a block a row.
+@pytest.mark.parametrize("kind", ["special", "equal", "ordered", "int32"])
+@pytest.mark.parametrize("rows,n,ks", [(300, 1025, (1, 3, 4)), (256, 2048, (1, 2, 3)), (255, 2048, (3,)), (257, 2049, (3,)),
+                                       (2048, 300, (9, 13, 16, 17)), (2050, 1024, (16,)), (2047, 65, (9, 16)), (4096, 65, (9, 16)),
+                                       (600, 2500, (13, 16, 17))])
+def test_waves_and_blocks(cx, rows, n, ks, kind):
+    rng = np.random.default_rng(rows + n)
+    x = np.sort(values_of("special", (rows, n), rng), axis=-1) if kind == "ordered" else values_of(kind, (rows, n), rng)
+    for k in ks:
+        check(cx, x, -1, k, True, True)
+        check(cx, x, -1, k, False, False)
