@@ -58,14 +58,12 @@ def test_split_as_far_as_the_workspace_goes(batch, rows, cols, features, causal)
 
 
 def test_form_without_a_workspace():
-    """8 x 128 queries and 640 keys of 128 features are split over four-wave
-    blocks; whole, as many matrices as fill the CUs take the eight-wave form,
-    with a workspace at hand (which it has no use for) and without."""
+    """Calls that no split helps take the same form with a workspace at hand and
+    without; calls that are split are planned anew without one."""
     assert plan(40, 500, 500, 128).waves == plan(40, 500, 500, 128, limit=0).waves == 8
     assert plan(8, 128, 4096, 128).splits > 1
     whole, few = plan(8, 128, 4096, 128, limit=0), plan(8, 128, 128, 128, limit=0)
     assert (whole.waves, whole.keys) == (few.waves, few.keys) == (4, 32)
-    # 2 x 64 x 2048 x 64: eight parts of 32-key tiles, or one of 64-key tiles.
     assert plan(2, 64, 2048, 64).splits > 1 and plan(2, 64, 2048, 64, limit=0).keys == 64
 
 
